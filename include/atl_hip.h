@@ -459,6 +459,25 @@ int atl_anchored_score_mean_bwd(const float* g, const float* q, const float* D, 
 int64_t atl_knn_ws_bytes(int64_t P, int64_t n);
 int atl_knn_indices(const float* queries, int64_t Q, const float* points, int64_t P, int64_t n, int64_t k,
                     int64_t* idx, void* ws, int64_t ws_bytes, hipStream_t stream);
+/* The whole table of atl/objectives/mpcm.py:56-78 from the trajectories: tr (B, 1 + T, n, 2) holds the n positions at
+ * the reference time (row 0) and at T bin times; table (B, T, ny, nx, 2) written: per query (x0 + i step, y0 + j step)
+ * and bin the mean over the k nearest positions of the bin (atl_knn_indices' order) of their displacement, row 0 minus
+ * the bin's row.  NaN where fewer than k distances are finite.  The backward takes the same sizes and the forward's
+ * workspace and writes gtr (B, 1 + T, n, 2).  ws: atl_lut_table_ws_bytes bytes (-1: sizes out of range). */
+int64_t atl_lut_table_ws_bytes(int64_t B, int64_t T, int64_t n, int64_t nx, int64_t ny);
+int atl_lut_table_fwd(const float* tr, int64_t B, int64_t T, int64_t n, double x0, double y0, double step, int64_t nx,
+                      int64_t ny, int64_t k, float* table, void* ws, int64_t ws_bytes, hipStream_t stream);
+int atl_lut_table_bwd(const float* gtable, int64_t B, int64_t T, int64_t n, double x0, double y0, double step,
+                      int64_t nx, int64_t ny, int64_t k, const void* ws, int64_t ws_bytes, float* gtr,
+                      hipStream_t stream);
+/* Positions (B, nt, Hq * Wq, 2) of every tile trajectory at nt times (atl/motion/trajectories.py:88-97): coef
+ * (B, 2K, Hq, Wq) with element strides sb, sc, sy, sx; tile centres tile * i + offset; basis as
+ * atl_traj_displacement's.  nt K <= 4096.  The backward writes gcoef (B, 2K, Hq, Wq) contiguous. */
+int atl_tile_trajectories(const float* coef, int64_t sb, int64_t sc, int64_t sy, int64_t sx, int64_t B, int64_t K,
+                          int64_t Hq, int64_t Wq, double offset, int64_t tile, const float* times, int64_t nt,
+                          int64_t basis, float* out, hipStream_t stream);
+int atl_tile_trajectories_bwd(const float* gout, int64_t B, int64_t K, int64_t Hq, int64_t Wq, const float* times,
+                              int64_t nt, int64_t basis, float* gcoef, hipStream_t stream);
 
 #ifdef __cplusplus
 }

@@ -646,6 +646,81 @@ __global__ void __launch_bounds__(kBlock) k_traj_displacement(const float4* __re
   if (live && q == 0) out[n] = make_float2(sx, sy);
 }
 
+// Positions of every tile trajectory at nt times (PixelTrajectories.tile_trajectories): out (B, nt, n, 2) = tile
+// centre + sum_k c_k g_k(t), the coefficients read through the strides of the tile-centre view (B, 2K, Hq, Wq).
+// One thread per trajectory and group of kTileTimes times (blockIdx.y), so that 19200 trajectories still give 300
+// workgroups; a thread's coefficients stay in registers.  The basis, the positions and their gradient were about
+// 120 launches of torch's element-wise operations and two matrix products, bound by the launches; one launch each
+// way takes 7.1 and 4.8 us for 16 times of 19200 trajectories, K = 10.
+constexpr int kTileTimes = 4, kTileMaxTable = 4096;
+
+template <int K>
+__global__ void __launch_bounds__(kBlock) k_tile_traj(const float* __restrict__ coef, int64_t sb, int64_t sc, int64_t sy,
+                                                      int64_t sx, int Wq, int n, float offset, float tile,
+                                                      const float* __restrict__ times, int nt, int basis,
+                                                      float2* __restrict__ out) {
+  __shared__ float gs[kTileTimes][K];
+  const int s0 = blockIdx.y * kTileTimes, ns = min(kTileTimes, nt - s0);
+  if ((int)threadIdx.x < ns) {
+    float g[K];
+    traj_basis<K>(times[s0 + threadIdx.x], basis, g);
+#pragma unroll
+    for (int k = 0; k < K; ++k) gs[threadIdx.x][k] = g[k];
+  }
+  __syncthreads();
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const int row = i / Wq, col = i - row * Wq;
+  const float* c = coef + blockIdx.z * sb + row * sy + col * sx;
+  float cy[K], cx[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    cy[k] = c[k * sc];
+    cx[k] = c[(K + k) * sc];
+  }
+  const float px = (float)col * tile + offset, py = (float)row * tile + offset;
+  for (int s = 0; s < ns; ++s) {
+    float dx = 0.f, dy = 0.f;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      dx = fmaf(gs[s][k], cx[k], dx);
+      dy = fmaf(gs[s][k], cy[k], dy);
+    }
+    out[((int64_t)blockIdx.z * nt + s0 + s) * n + i] = make_float2(px + dx, py + dy);
+  }
+}
+
+// Its adjoint: gcoef (B, 2K, n) = sum over the times, in order, of g_k(t) times the position gradient's component
+// (blockIdx.y: 0 the y coefficients, 1 the x coefficients).
+template <int K>
+__global__ void __launch_bounds__(kBlock) k_tile_traj_bwd(const float2* __restrict__ gout, int n,
+                                                          const float* __restrict__ times, int nt, int basis,
+                                                          float* __restrict__ gcoef) {
+  extern __shared__ float gtab[];                // nt x K
+  for (int s = threadIdx.x; s < nt; s += kBlock) {
+    float g[K];
+    traj_basis<K>(times[s], basis, g);
+#pragma unroll
+    for (int k = 0; k < K; ++k) gtab[s * K + k] = g[k];
+  }
+  __syncthreads();
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const bool xs = blockIdx.y == 1;
+  float acc[K] = {};
+  const float2* go = gout + (int64_t)blockIdx.z * nt * n + i;
+#pragma unroll 4
+  for (int s = 0; s < nt; ++s) {
+    const float2 g2 = go[(int64_t)s * n];
+    const float g = xs ? g2.x : g2.y;
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] = fmaf(gtab[s * K + k], g, acc[k]);
+  }
+  float* o = gcoef + ((int64_t)blockIdx.z * 2 + blockIdx.y) * K * n + i;
+#pragma unroll
+  for (int k = 0; k < K; ++k) o[(int64_t)k * n] = acc[k];
+}
+
 // The exposure correction of atl/objectives/ats.py:31-50 for PixelTrajectories in one pass: anchor i's trajectory
 // start p (n_fp Picard steps p <- xa - d(p, t_a) from p = xa, as PixelTrajectories.origin), its coefficients
 // looked up once at p, the trajectory evaluated at the n_check bin centres, y = p + d(p, c_k), and k_visible's
@@ -1288,6 +1363,56 @@ int atl_traj_displacement(const float* field_cl, int64_t B, int64_t C, int64_t K
 #undef ATL_TRAJ_CASE
   }
   return check_launch("traj_displacement");
+}
+
+static int tile_traj_bad(const char* what, int64_t B, int64_t K, int64_t Hq, int64_t Wq, int64_t nt, int64_t basis) {
+  if (B < 0 || B > 65535 || K < 1 || K > kTrajMaxK || Hq < 0 || Wq < 0 || (Wq > 0 && Hq > ((int64_t)1 << 30) / Wq) ||
+      nt < 0 || nt * K > kTileMaxTable || basis < 0 || basis > 2) {
+    set_error("%s: bad sizes (1 <= K <= %d, K times at most %d, basis 0, 1 or 2)", what, kTrajMaxK, kTileMaxTable);
+    return 1;
+  }
+  return 0;
+}
+
+#define ATL_TILE_CASES                                                                                            \
+  ATL_TILE_CASE(1) ATL_TILE_CASE(2) ATL_TILE_CASE(3) ATL_TILE_CASE(4) ATL_TILE_CASE(5) ATL_TILE_CASE(6)           \
+  ATL_TILE_CASE(7) ATL_TILE_CASE(8) ATL_TILE_CASE(9) ATL_TILE_CASE(10) ATL_TILE_CASE(11) ATL_TILE_CASE(12)        \
+  ATL_TILE_CASE(13) ATL_TILE_CASE(14) ATL_TILE_CASE(15) ATL_TILE_CASE(16)
+
+int atl_tile_trajectories(const float* coef, int64_t sb, int64_t sc, int64_t sy, int64_t sx, int64_t B, int64_t K,
+                          int64_t Hq, int64_t Wq, double offset, int64_t tile, const float* times, int64_t nt,
+                          int64_t basis, float* out, hipStream_t stream) {
+  if (tile_traj_bad("tile_trajectories", B, K, Hq, Wq, nt, basis)) return 1;
+  const int n = (int)(Hq * Wq);
+  if (n == 0 || B == 0 || nt == 0) return 0;
+  if (!coef || !times || !out) { set_error("tile_trajectories: null argument"); return 1; }
+  const dim3 grid(grid_for(n), (unsigned)((nt + kTileTimes - 1) / kTileTimes), (unsigned)B);
+  switch (K) {
+#define ATL_TILE_CASE(k)                                                                                          \
+    case k: hipLaunchKernelGGL(k_tile_traj<k>, grid, dim3(kBlock), 0, stream, coef, sb, sc, sy, sx, (int)Wq, n,   \
+                               (float)offset, (float)tile, times, (int)nt, (int)basis, (float2*)out); break;
+    ATL_TILE_CASES
+#undef ATL_TILE_CASE
+  }
+  return check_launch("tile_trajectories");
+}
+
+int atl_tile_trajectories_bwd(const float* gout, int64_t B, int64_t K, int64_t Hq, int64_t Wq, const float* times,
+                              int64_t nt, int64_t basis, float* gcoef, hipStream_t stream) {
+  if (tile_traj_bad("tile_trajectories_bwd", B, K, Hq, Wq, nt, basis)) return 1;
+  const int n = (int)(Hq * Wq);
+  if (n == 0 || B == 0) return 0;
+  if ((nt > 0 && (!gout || !times)) || !gcoef) { set_error("tile_trajectories_bwd: null argument"); return 1; }
+  const dim3 grid(grid_for(n), 2, (unsigned)B);
+  const size_t lds = (size_t)(nt * K) * sizeof(float);
+  switch (K) {
+#define ATL_TILE_CASE(k)                                                                                          \
+    case k: hipLaunchKernelGGL(k_tile_traj_bwd<k>, grid, dim3(kBlock), lds, stream, (const float2*)gout, n, times, \
+                               (int)nt, (int)basis, gcoef); break;
+    ATL_TILE_CASES
+#undef ATL_TILE_CASE
+  }
+  return check_launch("tile_trajectories_bwd");
 }
 
 int atl_traj_origin(const float* field_cl, int64_t B, int64_t C, int64_t K, int64_t Hg, int64_t Wg, const float* xy,

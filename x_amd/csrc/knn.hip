@@ -206,9 +206,419 @@ __global__ void __launch_bounds__(kBlock) k_knn_query(const float2* __restrict__
     if (s < k) o[s] = D[s] < INFINITY ? (int64_t)J[s] : (int64_t)-1;
 }
 
+// ------------------------------------------------------------------------------ the displacement table, fused
+// table (P, ny * nx, 2): per lattice query and plane, the mean displacement of the plane's k nearest points, and its
+// adjoint, without the indices (k_knn_query's order and ties, so the same set).  The mean needs the set and not its
+// order: a query first brackets its k-th distance, counting its candidates under seven thresholds at a time (14
+// instructions a candidate, nothing kept), then adds up the points under the bracket and picks the few inside it by
+// (distance, index).  The sorted insertion of k_knn_query costs 350 instructions a candidate, and took 560 us for 15
+// planes of 19200 points, k = 32; with the bracketing the whole forward takes 164 us on an even point set and 237 us
+// where trajectories of up to 25 px leave parts of the sensor empty (picking the bracket's points one pass each
+// instead of kPick a pass: 190 and 267 us).  One thread per query, a wave on an 8 x 8 patch,
+// so that its lanes read the same cells.
+//
+// The adjoint gathers: a point takes the gradient of every query whose k-th (distance, index) it does not exceed, the
+// same fp32 distance giving the same decision.  Queries stand in blocks of 4 x 4 with the largest k-th distance of
+// each block, so that a point tests about ten blocks (61 us; 88 us with a gradient loaded per taken query; torch's
+// scatter of 9.2M rows through atomics took 180 us, and the gather and mean forward another 130).
+constexpr int kQB = 4;                           // queries per block side
+constexpr int kPick = 4;                         // points picked from the bracket in one pass
+constexpr int kPatch = 16;                       // queries per workgroup side: 4 waves of 8 x 8
+
+struct LutLayout {
+  int64_t cnt, pmax, start, part, xy, dv, id, kth, kid, bmax, bytes;   // cnt and pmax are cleared together
+};
+
+LutLayout lut_layout(int64_t P, int64_t n, int64_t nx, int64_t ny) {
+  const int64_t ncell = P * (n + 1), nb = ((nx + kQB - 1) / kQB) * ((ny + kQB - 1) / kQB);
+  LutLayout L;
+  int64_t off = 0;
+  L.cnt = off;   off += ncell * 4;
+  L.pmax = off;  off = align256(off + P * 4);
+  L.start = off; off += align256((ncell + 1) * 4);
+  L.part = off;  off += align256((scan_tiles(ncell) + 1) * 4);
+  L.xy = off;    off += align256(P * n * 8);
+  L.dv = off;    off += align256(P * n * 8);
+  L.id = off;    off += align256(P * n * 4);
+  L.kth = off;   off += align256(P * nb * kQB * kQB * 4);
+  L.kid = off;   off += align256(P * nb * kQB * kQB * 4);
+  L.bmax = off;  off += align256(P * nb * 4);
+  L.bytes = off;
+  return L;
+}
+
+// k_knn_geom's grid for queries x0 + i * step, y0 + j * step: known on the host.
+KnnGeom lattice_geom(float x0, float y0, float step, int64_t nx, int64_t ny, int64_t n) {
+  const float w = fmaxf((float)(nx - 1) * step, 1.f), h = fmaxf((float)(ny - 1) * step, 1.f);
+  const double ncap = (double)n + 1.0, cs = sqrt((double)w * (double)h / (double)n);
+  KnnGeom g;
+  g.GX = (int)fmin(fmax(ceil((double)w / cs), 1.0), ncap);
+  g.GY = (int)fmin(fmax(ceil((double)h / cs), 1.0), floor(ncap / g.GX));
+  g.GY = g.GY < 1 ? 1 : g.GY;
+  g.ox = x0; g.oy = y0;
+  g.csx = w / (float)g.GX; g.csy = h / (float)g.GY;
+  g.icx = (float)g.GX / w; g.icy = (float)g.GY / h;
+  return g;
+}
+
+// k_knn_bin for the points tr (planes / T, 1 + T, n, 2): plane p = (b, s) holds the positions at time s, row 0 of its
+// batch those at the reference time, and a point's displacement is their difference.
+template <bool SCATTER>
+__global__ void __launch_bounds__(kBlock) k_lut_bin(const float2* __restrict__ tr, int T, int n, KnnGeom g,
+                                                    int* __restrict__ cnt, const int* __restrict__ start,
+                                                    float2* __restrict__ xy, float2* __restrict__ dv,
+                                                    int* __restrict__ id) {
+  const int j = blockIdx.x * kBlock + threadIdx.x;
+  if (j >= n) return;
+  const int plane = blockIdx.y, batch = plane / T;
+  const float2 p = tr[((int64_t)plane + batch + 1) * n + j];
+  const int64_t c = (int64_t)plane * (n + 1) + (int64_t)cell_of(p.y, g.oy, g.icy, g.GY) * g.GX + cell_of(p.x, g.ox, g.icx, g.GX);
+  if (!SCATTER) {
+    atomicAdd(cnt + c, 1);
+  } else {
+    const float2 r = tr[(int64_t)batch * (T + 1) * n + j];
+    const int slot = start[c] + atomicSub(cnt + c, 1) - 1;
+    xy[slot] = p;
+    dv[slot] = make_float2(r.x - p.x, r.y - p.y);
+    id[slot] = j;
+  }
+}
+
+__device__ __forceinline__ uint64_t dist_key(float d, int j) {   // orders (d, j), d >= 0
+  return ((uint64_t)__float_as_uint(d) << 32) | (uint32_t)j;
+}
+
+__global__ void __launch_bounds__(kBlock) k_lut_query(float x0, float y0, float step, int nx, int ny, int n, int k,
+                                                      KnnGeom g, const int* __restrict__ start,
+                                                      const float2* __restrict__ xy, const float2* __restrict__ dv,
+                                                      const int* __restrict__ id, float2* __restrict__ table,
+                                                      float* __restrict__ kth, int* __restrict__ kid,
+                                                      float* __restrict__ bmax, unsigned* __restrict__ pmax) {
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int npx = (nx + kPatch - 1) / kPatch;
+  const int blk = lane >> 4, l = lane & 15;      // a 16-lane row of the wave is one block of 4 x 4 queries
+  const int ix = (int)(blockIdx.x % npx) * kPatch + (wave & 1) * 8 + (blk & 1) * kQB + (l & 3);
+  const int iy = (int)(blockIdx.x / npx) * kPatch + (wave >> 1) * 8 + (blk >> 1) * kQB + (l >> 2);
+  const int plane = blockIdx.y;
+  const bool live = ix < nx && iy < ny;
+  const int* __restrict__ cs = start + (int64_t)plane * (n + 1);
+  const float qx = (float)ix * step + x0, qy = (float)iy * step + y0;
+  float dk = 0.f;                                // the k-th distance, its index, and whether others may share it
+  int jk = 0;
+  bool tie = false;
+  if (live) {
+    const int qcx = cell_of(qx, g.ox, g.icx, g.GX), qcy = cell_of(qy, g.oy, g.icy, g.GY);
+    const float slack = 1e-4f * (g.csx + g.csy) + 1e-5f * (fabsf(g.ox) + fabsf(g.oy) + fabsf(qx) + fabsf(qy));
+    // f(d, slot) over the points of a row range of cells, two loads in flight
+    auto row = [&](int b, int e, auto&& f) {
+      for (int t = b; t < e; t += 2) {
+        const int t2 = min(t + 1, e - 1);
+        const float2 p = xy[(uint32_t)t], p2 = xy[(uint32_t)t2];
+        const float dx = qx - p.x, dy = qy - p.y, dx2 = qx - p2.x, dy2 = qy - p2.y;
+        f(dx * dx + dy * dy, t);
+        if (t2 != t) f(dx2 * dx2 + dy2 * dy2, t2);
+      }
+    };
+    // over every cell that can hold a point closer than sqrt(hi): a point can be binned one rounding away
+    auto disc = [&](float hi, auto&& f) {
+      const float rad = __builtin_amdgcn_sqrtf(hi) + slack;   // ~1 ulp: far inside the slack
+      const int ya = cell_of(qy - rad, g.oy, g.icy, g.GY), yb = cell_of(qy + rad, g.oy, g.icy, g.GY);
+      for (int y = ya; y <= yb; ++y) {
+        const float lo = g.oy + (float)y * g.csy;
+        const float off = fmaxf(fmaxf(lo - qy, qy - (lo + g.csy)) - slack, 0.f);
+        const float hw = __builtin_amdgcn_sqrtf(fmaxf(rad * rad - off * off, 0.f)) + slack;
+        const int xa = cell_of(qx - hw, g.ox, g.icx, g.GX), xb = cell_of(qx + hw, g.ox, g.icx, g.GX);
+        row(cs[y * g.GX + xa], cs[y * g.GX + xb + 1], f);
+      }
+    };
+    float th[7];
+    int c[7];
+    auto count = [&](float d, int) {
+#pragma unroll
+      for (int i = 0; i < 7; ++i) c[i] += d < th[i] ? 1 : 0;
+    };
+    // an upper bound of the k-th distance from the smallest block of cells around the query that shows one: the
+    // thresholds lie around the distance at which the block's density gives k points, and out to the block's corner
+    float hi = INFINITY, lo = 0.f;
+    int chi = 0, clo = 0;                        // points under hi and under lo (chi: 0 until counted)
+    int r = 0;
+    while ((2 * r + 1) * (2 * r + 1) < k) ++r;
+    for (;;) {
+      const int xa = max(qcx - r, 0), xb = min(qcx + r, g.GX - 1), ya = max(qcy - r, 0), yb = min(qcy + r, g.GY - 1);
+      int m = 0;
+      for (int y = ya; y <= yb; ++y) m += cs[y * g.GX + xb + 1] - cs[y * g.GX + xa];
+      if (m >= k) {
+        const float area = (float)((xb - xa + 1) * (yb - ya + 1)) * g.csx * g.csy;
+        const float e = area * (float)k / (3.14159265f * (float)m);
+        const float ddx = fmaxf(qx - (g.ox + (float)xa * g.csx), g.ox + (float)(xb + 1) * g.csx - qx);
+        const float ddy = fmaxf(qy - (g.oy + (float)ya * g.csy), g.oy + (float)(yb + 1) * g.csy - qy);
+        const float far = fmaxf(ddx * ddx + ddy * ddy, 1.2f * e);   // the block's corner: all but points beyond the grid
+        const float q = cbrtf(far / (1.15f * e));
+        th[0] = 0.55f * e; th[1] = 0.8f * e; th[2] = 0.95f * e; th[3] = 1.15f * e; th[4] = th[3] * q; th[5] = th[4] * q;
+        th[6] = far;
+#pragma unroll
+        for (int i = 0; i < 7; ++i) c[i] = 0;
+        for (int y = ya; y <= yb; ++y) row(cs[y * g.GX + xa], cs[y * g.GX + xb + 1], count);
+#pragma unroll
+        for (int i = 6; i >= 0; --i)
+          if (c[i] >= k) hi = th[i];
+        if (hi < INFINITY) break;
+      }
+      if (xa == 0 && ya == 0 && xb == g.GX - 1 && yb == g.GY - 1) break;   // every cell seen
+      r += 1 + r / 2;
+    }
+    // narrow (lo, hi] until at most three points of it are taken; the first cuts lie where the bound above usually
+    // leaves the distance, so that one round is enough for most waves
+    for (int it = 0; it < 8; ++it) {
+      const float w = hi - lo;
+      if (it == 0 && hi < INFINITY) {
+        th[0] = 0.55f * hi; th[1] = 0.68f * hi; th[2] = 0.76f * hi; th[3] = 0.82f * hi; th[4] = 0.88f * hi;
+        th[5] = 0.93f * hi; th[6] = 0.97f * hi;
+      } else if (hi < INFINITY) {
+#pragma unroll
+        for (int i = 0; i < 7; ++i) th[i] = lo + w * (0.125f * (float)(i + 1));
+      } else {                                   // no bound: far or few points, cut over their powers of two
+        const float e = fmaxf(lo, g.csx * g.csy);
+#pragma unroll
+        for (int i = 0; i < 7; ++i) th[i] = e * (float)(1 << (2 * i + 2));
+      }
+#pragma unroll
+      for (int i = 0; i < 7; ++i) c[i] = 0;
+      int all = 0;
+      disc(hi, [&](float d, int s) {
+        all += d < hi ? 1 : 0;
+        count(d, s);
+      });
+      chi = all;
+      float nlo = lo, nhi = hi;
+      int ncl = clo, nch = all;
+#pragma unroll
+      for (int i = 0; i < 7; ++i)
+        if (th[i] > lo && c[i] < k) { nlo = th[i]; ncl = c[i]; }
+#pragma unroll
+      for (int i = 6; i >= 0; --i)
+        if (th[i] < hi && c[i] >= k) { nhi = th[i]; nch = c[i]; }
+      const bool same = nlo == lo && nhi == hi;
+      lo = nlo; hi = nhi; clo = ncl; chi = nch;
+      if (chi < k || k - clo < kPick || same) break;
+    }
+    // the points under lo, and the k - clo first of those in [lo, hi) by (distance, index), kPick at a time
+    float sx = 0.f, sy = 0.f;
+    uint64_t last = 0, key[kPick];
+    int ks[kPick];
+    for (int m = clo; m < k; m += kPick) {
+#pragma unroll
+      for (int i = 0; i < kPick; ++i) { key[i] = ~(uint64_t)0; ks[i] = -1; }
+      const bool first = m == clo;
+      disc(hi, [&](float d, int s) {
+        if (d < lo) {
+          if (first) {
+            const float2 v = dv[(uint32_t)s];
+            sx += v.x;
+            sy += v.y;
+          }
+        } else if (d < hi) {
+          uint64_t ck = dist_key(d, id[(uint32_t)s]);
+          if ((first || ck > last) && ck < key[kPick - 1]) {
+            int cs_ = s;
+#pragma unroll
+            for (int i = 0; i < kPick; ++i) {
+              const bool lt = ck < key[i];
+              const uint64_t tk = key[i];
+              const int ts = ks[i];
+              key[i] = lt ? ck : tk;
+              ks[i] = lt ? cs_ : ts;
+              ck = lt ? tk : ck;
+              cs_ = lt ? ts : cs_;
+            }
+          }
+        }
+      });
+#pragma unroll
+      for (int i = 0; i < kPick; ++i)
+        if (m + i < k) {
+          if (ks[i] < 0) {                       // fewer than k finite distances
+            sx = sy = NAN;
+          } else {
+            const float2 v = dv[(uint32_t)ks[i]];
+            sx += v.x;
+            sy += v.y;
+          }
+          last = key[i];
+          // a point at the same distance may be left out unless the next key is known to lie further
+          tie = i + 1 >= kPick || (uint32_t)(key[i + 1 < kPick ? i + 1 : i] >> 32) == (uint32_t)(last >> 32);
+        }
+      if (ks[kPick - 1] < 0) {
+        if (k - m > kPick) { sx = sy = NAN; last = ~(uint64_t)0; }
+        break;
+      }
+    }
+    const bool short_ = last == ~(uint64_t)0;    // too few: every finite distance counts
+    dk = short_ ? INFINITY : __uint_as_float((uint32_t)(last >> 32));
+    jk = (int)(uint32_t)last;
+    tie = tie && !short_;
+    const float inv = (float)k;
+    table[(int64_t)plane * nx * ny + (int64_t)iy * nx + ix] = make_float2(sx / inv, sy / inv);
+  }
+  const int nbx = (nx + kQB - 1) / kQB, nby = (ny + kQB - 1) / kQB;
+  const int bx = ix / kQB, by = iy / kQB;
+  const bool block_live = bx < nbx && by < nby;
+  const int64_t bi = ((int64_t)plane * nby + by) * nbx + bx;
+  if (block_live) {                              // NaN: no query here; negative: ties are decided by the index
+    kth[bi * (kQB * kQB) + l] = live ? __uint_as_float(__float_as_uint(dk) | (tie ? 0x80000000u : 0u)) : NAN;
+    kid[bi * (kQB * kQB) + l] = jk;
+  }
+  float m = dk;
+#pragma unroll
+  for (int d = 8; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, kWave));
+  if (block_live && l == 0) bmax[bi] = m;
+  m = fmaxf(m, __shfl_xor(m, 16, kWave));
+  m = fmaxf(m, __shfl_xor(m, 32, kWave));
+  if (lane == 0) atomicMax(pmax + plane, __float_as_uint(m));   // distances are not negative: bits order them
+}
+
+// gtr rows 1..T of every batch: minus the point's gradient (its displacement is reference minus position).
+__global__ void __launch_bounds__(kBlock) k_lut_adjoint(float x0, float y0, float step, int nx, int ny, int n, int T,
+                                                        int k, const float2* __restrict__ xy,
+                                                        const int* __restrict__ id, const float4* __restrict__ kth,
+                                                        const int* __restrict__ kid, const float* __restrict__ bmax,
+                                                        const unsigned* __restrict__ pmax,
+                                                        const float2* __restrict__ gtable, float2* __restrict__ gtr) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const int plane = blockIdx.y;
+  const int64_t slot = (int64_t)plane * n + i;
+  const float2 p = xy[slot];
+  const int j = id[slot];
+  const int nbx = (nx + kQB - 1) / kQB, nby = (ny + kQB - 1) / kQB;
+  // blocks within the plane's largest k-th distance; the hundredth of a step covers the roundings
+  const float R = sqrtf(__uint_as_float(pmax[plane])) + 0.01f * step;
+  const float ib = 1.f / ((float)kQB * step), eps = 0.01f * step;
+  auto block_of = [&](float v, float o, int nb) { return (int)fminf(fmaxf(floorf((v - o) * ib), 0.f), (float)(nb - 1)); };
+  const int xa = block_of(p.x - R, x0, nbx), xb = block_of(p.x + R, x0, nbx);
+  const int ya = block_of(p.y - R, y0, nby), yb = block_of(p.y + R, y0, nby);
+  const float2* __restrict__ gt = gtable + (int64_t)plane * nx * ny;
+  float gx = 0.f, gy = 0.f;
+  for (int by = ya; by <= yb; ++by)
+    for (int bx = xa; bx <= xb; ++bx) {
+      const float lx = (float)(bx * kQB) * step + x0, ly = (float)(by * kQB) * step + y0;
+      const float ex = fmaxf(fmaxf(lx - p.x, p.x - (lx + 3.f * step)) - eps, 0.f);
+      const float ey = fmaxf(fmaxf(ly - p.y, p.y - (ly + 3.f * step)) - eps, 0.f);
+      const int64_t bi = ((int64_t)plane * nby + by) * nbx + bx;
+      if (!(ex * ex + ey * ey <= bmax[bi])) continue;
+      // a row of four queries at a time; their gradients are loaded whether or not they are taken (a load under a
+      // condition of its own was a wait per query)
+#pragma unroll
+      for (int ly = 0; ly < kQB; ++ly) {
+        const int iy = by * kQB + ly;
+        const float4 kq = kth[bi * kQB + ly];
+        const float dks[kQB] = {kq.x, kq.y, kq.z, kq.w};
+        const float dy = ((float)iy * step + y0) - p.y;
+        const float2* gr = gt + (uint32_t)(min(iy, ny - 1) * nx);
+        float2 gv[kQB];
+#pragma unroll
+        for (int lx = 0; lx < kQB; ++lx) gv[lx] = gr[(uint32_t)min(bx * kQB + lx, nx - 1)];
+#pragma unroll
+        for (int lx = 0; lx < kQB; ++lx) {
+          const float dx = ((float)(bx * kQB + lx) * step + x0) - p.x;
+          const float d = dx * dx + dy * dy, dk = fabsf(dks[lx]);
+          bool take = d <= dk;                   // false for NaN
+          if (d == dk && __float_as_uint(dks[lx]) >> 31) take = j <= kid[bi * (kQB * kQB) + ly * kQB + lx];
+          gx += take ? gv[lx].x : 0.f;
+          gy += take ? gv[lx].y : 0.f;
+        }
+      }
+    }
+  const float inv = (float)k;
+  gtr[((int64_t)plane + plane / T + 1) * n + j] = make_float2(-gx / inv, -gy / inv);
+}
+
+// gtr row 0 of every batch: minus the sum of the other rows (every displacement starts at the reference position).
+__global__ void __launch_bounds__(kBlock) k_lut_ref_grad(int n, int T, float2* __restrict__ gtr) {
+  const int j = blockIdx.x * kBlock + threadIdx.x;
+  if (j >= n) return;
+  float2* g = gtr + (int64_t)blockIdx.y * (T + 1) * n + j;
+  float x = 0.f, y = 0.f;
+#pragma unroll 4
+  for (int s = 1; s <= T; ++s) {
+    const float2 v = g[(int64_t)s * n];
+    x -= v.x;
+    y -= v.y;
+  }
+  g[0] = make_float2(x, y);
+}
+
+int lut_bad(const char* what, int64_t B, int64_t T, int64_t n, double step, int64_t nx, int64_t ny, int64_t k) {
+  const int64_t lim = (int64_t)1 << 31;
+  if (B < 0 || T < 1 || n < 1 || nx < 0 || ny < 0 || !(step > 0) || B > 65535 || T > 65535 || B * T > 65535 ||
+      n >= lim || nx >= lim || ny >= lim || nx * ny > ((int64_t)1 << 30) || (B * T + B) * (n + 1) >= lim || k < 1 ||
+      k > kKnnMaxK || k > n) {
+    set_error("%s: bad sizes B=%lld T=%lld n=%lld nx=%lld ny=%lld k=%lld (1 <= k <= min(n, %d))", what, (long long)B,
+              (long long)T, (long long)n, (long long)nx, (long long)ny, (long long)k, kKnnMaxK);
+    return 1;
+  }
+  return 0;
+}
+
 }  // namespace
 
 extern "C" {
+
+int64_t atl_lut_table_ws_bytes(int64_t B, int64_t T, int64_t n, int64_t nx, int64_t ny) {
+  if (lut_bad("lut_table", B, T, n, 1.0, nx, ny, 1)) return -1;
+  return lut_layout(B * T, n, nx, ny).bytes;
+}
+
+int atl_lut_table_fwd(const float* tr, int64_t B, int64_t T, int64_t n, double x0, double y0, double step, int64_t nx,
+                      int64_t ny, int64_t k, float* table, void* ws, int64_t ws_bytes, hipStream_t stream) {
+  if (lut_bad("lut_table_fwd", B, T, n, step, nx, ny, k)) return 1;
+  if (B == 0 || nx * ny == 0) return 0;
+  const int64_t P = B * T, ncell = P * (n + 1);
+  const LutLayout L = lut_layout(P, n, nx, ny);
+  if (!tr || !table || !ws || ws_bytes < L.bytes) {
+    set_error("lut_table_fwd: null argument or a workspace of %lld bytes, need %lld", (long long)ws_bytes, (long long)L.bytes);
+    return 1;
+  }
+  char* w = (char*)ws;
+  int *cnt = (int*)(w + L.cnt), *start = (int*)(w + L.start), *id = (int*)(w + L.id);
+  float2 *xy = (float2*)(w + L.xy), *dv = (float2*)(w + L.dv);
+  const KnnGeom g = lattice_geom((float)x0, (float)y0, (float)step, nx, ny, n);
+  const int64_t clear = ncell + P;               // the counts and the planes' largest distances behind them
+  hipLaunchKernelGGL(k_knn_zero, dim3(grid_for(clear)), dim3(kBlock), 0, stream, cnt, clear);
+  const dim3 pgrid(grid_for(n), (unsigned)P);
+  hipLaunchKernelGGL((k_lut_bin<false>), pgrid, dim3(kBlock), 0, stream, (const float2*)tr, (int)T, (int)n, g, cnt,
+                     (const int*)nullptr, (float2*)nullptr, (float2*)nullptr, (int*)nullptr);
+  scan32(cnt, ncell, (int*)(w + L.part), start, stream);
+  hipLaunchKernelGGL((k_lut_bin<true>), pgrid, dim3(kBlock), 0, stream, (const float2*)tr, (int)T, (int)n, g, cnt,
+                     (const int*)start, xy, dv, id);
+  const dim3 qgrid((unsigned)(((nx + kPatch - 1) / kPatch) * ((ny + kPatch - 1) / kPatch)), (unsigned)P);
+  hipLaunchKernelGGL(k_lut_query, qgrid, dim3(kBlock), 0, stream, (float)x0, (float)y0, (float)step, (int)nx, (int)ny,
+                     (int)n, (int)k, g, (const int*)start, (const float2*)xy, (const float2*)dv, (const int*)id,
+                     (float2*)table, (float*)(w + L.kth), (int*)(w + L.kid), (float*)(w + L.bmax), (unsigned*)(w + L.pmax));
+  return check_launch("lut_table_fwd");
+}
+
+int atl_lut_table_bwd(const float* gtable, int64_t B, int64_t T, int64_t n, double x0, double y0, double step,
+                      int64_t nx, int64_t ny, int64_t k, const void* ws, int64_t ws_bytes, float* gtr,
+                      hipStream_t stream) {
+  if (lut_bad("lut_table_bwd", B, T, n, step, nx, ny, k)) return 1;
+  if (B == 0) return 0;
+  const int64_t P = B * T;
+  const LutLayout L = lut_layout(P, n, nx, ny);
+  if (nx * ny == 0 || !gtable || !gtr || !ws || ws_bytes < L.bytes) {
+    set_error("lut_table_bwd: no query, null argument or a workspace of %lld bytes, need %lld", (long long)ws_bytes, (long long)L.bytes);
+    return 1;
+  }
+  const char* w = (const char*)ws;
+  const dim3 pgrid(grid_for(n), (unsigned)P);
+  hipLaunchKernelGGL(k_lut_adjoint, pgrid, dim3(kBlock), 0, stream, (float)x0, (float)y0, (float)step, (int)nx,
+                     (int)ny, (int)n, (int)T, (int)k, (const float2*)(w + L.xy), (const int*)(w + L.id),
+                     (const float4*)(w + L.kth), (const int*)(w + L.kid), (const float*)(w + L.bmax), (const unsigned*)(w + L.pmax),
+                     (const float2*)gtable, (float2*)gtr);
+  hipLaunchKernelGGL(k_lut_ref_grad, dim3(grid_for(n), (unsigned)B), dim3(kBlock), 0, stream, (int)n, (int)T,
+                     (float2*)gtr);
+  return check_launch("lut_table_bwd");
+}
 
 int64_t atl_knn_ws_bytes(int64_t P, int64_t n) {
   if (P < 0 || n < 0 || P * (n + 1) >= (int64_t)1 << 31) return -1;

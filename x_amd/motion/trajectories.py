@@ -25,7 +25,7 @@ import math
 import numpy as np
 import torch
 
-from ..ops.functional import TRAJ_BASES, TRAJ_MAX_K, _tile_plan_ok, traj_displacement, traj_origin
+from ..ops.functional import TRAJ_BASES, TRAJ_MAX_K, _tile_plan_ok, tile_trajectories, traj_displacement, traj_origin
 from .base import Motion, as_time
 from .parametric import sample_grid
 
@@ -221,6 +221,9 @@ class PixelTrajectories(Motion):
         """Positions (B, n_t, Hq*Wq, 2) in (x, y) of every tile trajectory at ``times`` (the look-up table of
         MotionPriorCMax)."""
         dev, K = self.tile_c.device, self.K
+        pos = tile_trajectories(self.tile_c, times.to(torch.float32), K, self.basis_kind, self.offset, self.tile)
+        if pos is not None:                                             # on the device one kernel each way
+            return pos
         cy = torch.arange(self.Hq, device=dev, dtype=torch.float32) * self.tile + self.offset
         cx = torch.arange(self.Wq, device=dev, dtype=torch.float32) * self.tile + self.offset
         start = torch.cartesian_prod(cy, cx).flip(-1)                   # (Hq*Wq, 2) in (x, y), row-major

@@ -4,8 +4,8 @@ displaced by a look-up table, plus a Charbonnier smoothness of that table.
 The table (``lut_flow``, mpcm.py:56-78) holds, for every cell of a ``lut`` x ``lut`` pixel grid and every time bin,
 the mean displacement to t_ref of the K trajectories nearest to the cell centre at the bin's mid time.  The
 nearest-neighbour search is the loss's dominant cost in the reference (a dense distance matrix and a top-k per
-plane); here it is one HIP pass over grid-binned points (``x_amd.ops.knn_indices``), and the table's gather and mean
-stay torch ops so that the gradient reaches the trajectory coefficients as in the reference.
+plane); here a HIP pass over grid-binned points finds the neighbours and their mean together (``lut_table``), and the
+gradient reaches the trajectory coefficients as in the reference.
 """
 from __future__ import annotations
 
@@ -13,6 +13,7 @@ import torch
 
 from ..core.events import EventPacket
 from ..ops import knn_indices
+from ..ops.functional import lut_table, lut_table_torch
 from .base import IWEConfig, Objective, make_iwe, sobel
 
 __all__ = ["MotionPriorCMaxLoss", "knn_indices", "charbonnier_tv"]
@@ -55,16 +56,15 @@ class MotionPriorCMaxLoss(Objective):
         edges = torch.linspace(0, 1, self.num_bins + 1, device=dev)
         mids = (edges[:-1] + edges[1:]) * 0.5
         tr = motion.tile_trajectories(torch.cat([t_ref.reshape(1).to(mids), mids]))   # (B, 1 + bins, n, 2)
-        at_ref, at_mid = tr[:, :1], tr[:, 1:]
-        centres = self.cell_centres(H, W, dev)
-        k = min(self.num_knn, at_mid.shape[2])
-        idx = knn_indices(centres, at_mid.detach(), k)                                 # (B, bins, Q, k)
-        disp = at_ref - at_mid                                                         # (B, bins, n, 2)
-        B, nb, n, _ = disp.shape
-        picked = torch.gather(disp.reshape(B * nb, n, 2), 1,
-                              idx.reshape(B * nb, -1, 1).expand(-1, -1, 2))            # (B * bins, Q * k, 2)
-        table = picked.view(B, nb, -1, k, 2).mean(3)
         Hl, Wl = -(-H // self.lut), -(-W // self.lut)
+        k = min(self.num_knn, tr.shape[2])
+        B, nb = tr.shape[0], tr.shape[1] - 1
+        half = self.lut / 2.0 - 0.5
+        table = None
+        if type(self).cell_centres is MotionPriorCMaxLoss.cell_centres and self.lut > 0:
+            table = lut_table(tr, half, half, float(self.lut), Wl, Hl, k)
+        if table is None:
+            table = lut_table_torch(tr, self.cell_centres(H, W, dev), k)
         return table.view(B, nb, Hl, Wl, 2), edges
 
     def __call__(self, ev: EventPacket, motion):

@@ -1336,3 +1336,121 @@ def knn_indices(queries: torch.Tensor, points: torch.Tensor, k: int, chunk: int 
     with torch.cuda.device(pts.device):
         call("atl_knn_indices", ptr(q), Q, ptr(pts), B * T, n, k, ptr(out), ptr(ws), nbytes, stream_of(pts))
     return out
+
+
+# ------------------------------------------------------------------ tile trajectories and the displacement table
+TILE_TABLE_MAX = 4096
+
+
+def _plain_device(*ts) -> bool:
+    """Whether a fused op that replaces a chain of torch operations may take these tensors: plain fp32 device tensors,
+    and no transform or mode at work that has to see the operations themselves (tracing, torch.func, forward-mode
+    derivatives, autocast's casts, dispatch modes)."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == F32 for t in ts)
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
+            and not torch.is_autocast_enabled("cuda") and torch._C._len_torch_dispatch_stack() == 0)
+
+
+class _TileTrajectories(torch.autograd.Function):
+    """PixelTrajectories.tile_trajectories (atl/motion/trajectories.py:88-97) in one kernel each way.  A backward that
+    is itself differentiated runs as the torch expression of the adjoint."""
+
+    @staticmethod
+    def forward(ctx, coef, times, K, kind, offset, tile):
+        B, _, Hq, Wq = coef.shape
+        nt = times.shape[0]
+        ctx.save_for_backward(times)
+        ctx.shape, ctx.kind = (B, K, Hq, Wq), kind
+        out = torch.empty(B, nt, Hq * Wq, 2, device=coef.device, dtype=F32)
+        with torch.cuda.device(coef.device):
+            call("atl_tile_trajectories", ptr(coef), *coef.stride(), B, K, Hq, Wq, offset, tile, ptr(times), nt,
+                 TRAJ_BASES[kind], ptr(out), stream_of(coef))
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        times, = ctx.saved_tensors
+        B, K, Hq, Wq = ctx.shape
+        if torch.is_grad_enabled():
+            from ..motion.trajectories import basis
+            gc = torch.einsum("tk,btnc->bckn", basis(times, K, ctx.kind), g).flip(1)
+            return gc.reshape(B, 2 * K, Hq, Wq), None, None, None, None, None
+        g = g.contiguous()
+        gc = torch.empty(B, 2 * K, Hq, Wq, device=g.device, dtype=F32)
+        with torch.cuda.device(g.device):
+            call("atl_tile_trajectories_bwd", ptr(g), B, K, Hq, Wq, ptr(times), times.shape[0], TRAJ_BASES[ctx.kind],
+                 ptr(gc), stream_of(g))
+        return gc, None, None, None, None, None
+
+
+def tile_trajectories(coef: torch.Tensor, times: torch.Tensor, K: int, kind: str, offset: float, tile: int):
+    """Positions (B, n_t, Hq * Wq, 2) of the tile trajectories of ``coef`` (B, 2K, Hq, Wq; any strides) at ``times``
+    (n_t), or None where the device path does not apply: more coefficients or times than its tables hold, times that
+    carry a gradient, or tensors and modes that need the torch operations."""
+    if (coef.dim() != 4 or times.dim() != 1 or coef.shape[1] != 2 * K or not 1 <= K <= TRAJ_MAX_K
+            or K * times.shape[0] > TILE_TABLE_MAX or times.requires_grad or coef.device != times.device
+            or coef.shape[0] > 65535 or not _plain_device(coef, times)):
+        return None
+    return _TileTrajectories.apply(coef, times.contiguous(), int(K), kind, float(offset), int(tile))
+
+
+def lut_table_torch(tr: torch.Tensor, centres: torch.Tensor, k: int) -> torch.Tensor:
+    """(B, T, Q, 2) mean displacement (row 0 of ``tr`` (B, 1 + T, n, 2) minus row 1 + s) of the k points of bin s
+    nearest to each centre (Q, 2), as torch operations on knn_indices' choice (atl/objectives/mpcm.py:67-77)."""
+    at_ref, at_mid = tr[:, :1], tr[:, 1:]
+    idx = knn_indices(centres, at_mid.detach(), k)                                     # (B, T, Q, k)
+    disp = at_ref - at_mid                                                             # (B, T, n, 2)
+    B, T, n, _ = disp.shape
+    picked = torch.gather(disp.reshape(B * T, n, 2), 1, idx.reshape(B * T, -1, 1).expand(-1, -1, 2))
+    return picked.view(B, T, -1, k, 2).mean(3)
+
+
+class _LutTable(torch.autograd.Function):
+    """lut_table_torch over a lattice of centres in HIP kernels, without the indices: the forward keeps each query's
+    k-th (distance, index) and the binned points, and the backward gathers each point's gradient from the queries that
+    took it.  A backward that is itself differentiated runs as torch operations."""
+
+    @staticmethod
+    def forward(ctx, tr, x0, y0, step, nx, ny, k):
+        B, T, n, _ = tr.shape
+        T -= 1
+        nbytes = load_library().atl_lut_table_ws_bytes(B, T, n, nx, ny)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=tr.device)
+        out = torch.empty(B, T, ny * nx, 2, device=tr.device, dtype=F32)
+        with torch.cuda.device(tr.device):
+            call("atl_lut_table_fwd", ptr(tr), B, T, n, x0, y0, step, nx, ny, k, ptr(out), ptr(ws), nbytes,
+                 stream_of(tr))
+        ctx.save_for_backward(tr, ws)
+        ctx.lattice = x0, y0, step, nx, ny, k
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        tr, ws = ctx.saved_tensors
+        x0, y0, step, nx, ny, k = ctx.lattice
+        B, T, n, _ = tr.shape
+        T -= 1
+        if torch.is_grad_enabled():
+            cy = torch.arange(ny, device=g.device, dtype=F32) * step + y0
+            cx = torch.arange(nx, device=g.device, dtype=F32) * step + x0
+            idx = knn_indices(torch.cartesian_prod(cy, cx).flip(-1), tr.detach()[:, 1:], k).view(B, T, -1, 1)
+            rows = (g / k)[:, :, :, None].expand(-1, -1, -1, k, -1).reshape(B, T, -1, 2)
+            gd = torch.zeros(B, T, n, 2, device=g.device, dtype=F32).scatter_add(2, idx.expand(-1, -1, -1, 2), rows)
+            return torch.cat([gd.sum(1, keepdim=True), -gd], 1), None, None, None, None, None, None
+        g = g.contiguous()
+        gtr = torch.empty_like(tr)
+        with torch.cuda.device(g.device):
+            call("atl_lut_table_bwd", ptr(g), B, T, n, x0, y0, step, nx, ny, k, ptr(ws), ws.numel(), ptr(gtr),
+                 stream_of(g))
+        return gtr, None, None, None, None, None, None
+
+
+def lut_table(tr: torch.Tensor, x0: float, y0: float, step: float, nx: int, ny: int, k: int):
+    """lut_table_torch for the ny x nx centres (x0 + i step, y0 + j step), row-major, or None where the device path does
+    not apply (more neighbours than its limit, sizes past 32-bit cells, no centre or bin, other tensors or modes)."""
+    if (tr.dim() != 4 or tr.shape[-1] != 2 or not 1 <= k <= min(tr.shape[2], KNN_MAX_K) or tr.shape[1] < 2
+            or tr.shape[0] < 1 or nx < 1 or ny < 1 or not step > 0 or not _plain_device(tr)
+            or load_library().atl_lut_table_ws_bytes(tr.shape[0], tr.shape[1] - 1, tr.shape[2], nx, ny) < 0):
+        return None
+    return _LutTable.apply(tr.contiguous(), float(x0), float(y0), float(step), int(nx), int(ny), int(k))
