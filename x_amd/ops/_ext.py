@@ -14,6 +14,7 @@ The library is built in-tree by ``python x_amd/csrc/build.py`` (or ``__graft_ent
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from pathlib import Path
@@ -237,8 +238,23 @@ def ptr(t: torch.Tensor | None):
     return ctypes.c_void_p(0) if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+def raw_stream(dev: torch.device) -> int:
+    """Handle of the device's current stream (torch.cuda.current_stream(dev).cuda_stream without the stream object:
+    0.2 us instead of 4.6, at each entry point)."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
 def stream_of(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return ctypes.c_void_p(raw_stream(t.device))
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device(dev: torch.device):
+    """torch.cuda.device(dev) where the thread's current device is another one; nothing to do where it is ``dev``
+    already (0.2 us instead of 3)."""
+    return _HERE if torch._C._cuda_getDevice() == dev.index else torch.cuda.device(dev)
 
 
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype, dev: torch.device, shape=None):
@@ -271,7 +287,7 @@ class HipOps:
         _need(pos, "pos", F32, dev, (N, 2)); _need(w, "w", F32, dev, (N,)); _need(b, "b", I64, dev, (N,))
         img = torch.zeros(int(B), int(H), int(W), device=dev, dtype=F32)
         nbytes = load_library().atl_tile_ws_bytes(N, int(B), int(H), int(W)) if N > 0 and int(B) > 0 else -1
-        with torch.cuda.device(dev):
+        with on_device(dev):
             if nbytes >= 0:          # tile-binned LDS accumulation
                 ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
                 call("atl_splat_bilinear_fwd_ws", ptr(pos), ptr(w), ptr(b), N, int(B), int(H), int(W), ptr(img),
@@ -288,7 +304,7 @@ class HipOps:
         _need(b, "b", I64, dev, (N,))
         B, H, W = gimg.shape
         gpos = torch.empty_like(pos); gw = torch.empty_like(w)
-        with torch.cuda.device(dev):
+        with on_device(dev):
             call("atl_splat_bilinear_bwd", ptr(gimg), ptr(pos), ptr(w), ptr(b), N, B, H, W, ptr(gpos), ptr(gw),
                  stream_of(pos))
         return [gpos, gw]
@@ -300,7 +316,7 @@ class HipOps:
         img = torch.zeros(int(B), int(H), int(W), device=dev, dtype=F32)
         nbytes = (load_library().atl_splat_gauss_ws_bytes(N, int(B), int(H), int(W), int(radius))
                   if N > 0 and int(B) > 0 else -1)
-        with torch.cuda.device(dev):
+        with on_device(dev):
             if nbytes >= 0:          # tile-binned LDS accumulation
                 ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
                 call("atl_splat_gauss_fwd_ws", ptr(pos), ptr(w), ptr(b), N, int(B), int(H), int(W), float(sigma),
@@ -317,7 +333,7 @@ class HipOps:
         _need(b, "b", I64, dev, (N,))
         B, H, W = gimg.shape
         gpos = torch.empty_like(pos); gw = torch.empty_like(w)
-        with torch.cuda.device(dev):
+        with on_device(dev):
             call("atl_splat_gauss_bwd", ptr(gimg), ptr(pos), ptr(w), ptr(b), N, B, H, W, float(sigma), int(radius),
                  ptr(gpos), ptr(gw), stream_of(pos))
         return [gpos, gw]
@@ -328,7 +344,7 @@ class HipOps:
         _need(img, "img", F32, dev); _need(pos, "pos", F32, dev, (N, 2)); _need(b, "b", I64, dev, (N,))
         B, H, W = img.shape
         out = torch.empty(N, device=dev, dtype=F32)
-        with torch.cuda.device(dev):
+        with on_device(dev):
             call("atl_gather_bilinear_fwd", ptr(img), ptr(pos), ptr(b), N, B, H, W, ptr(out), stream_of(pos))
         return out
 
@@ -340,7 +356,7 @@ class HipOps:
         B, H, W = img.shape
         gimg = torch.zeros_like(img); gpos = torch.empty_like(pos)
         nbytes = load_library().atl_tile_ws_bytes(N, B, H, W) if N > 0 and B > 0 else -1
-        with torch.cuda.device(dev):
+        with on_device(dev):
             if nbytes >= 0:          # tile-binned LDS accumulation of gimg
                 ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
                 call("atl_gather_bilinear_bwd_ws", ptr(gval), ptr(img), ptr(pos), ptr(b), N, B, H, W, ptr(gimg),
@@ -357,7 +373,7 @@ class HipOps:
         _need(b, "b", I64, dev, (N,))
         vox = torch.zeros(int(B), int(C), int(H), int(W), device=dev, dtype=F32)
         nbytes = load_library().atl_voxel_ws_bytes(N, int(B), int(C), int(H), int(W)) if N > 0 and int(B) > 0 else -1
-        with torch.cuda.device(dev):
+        with on_device(dev):
             if nbytes >= 0:          # tile-binned LDS accumulation, the time bins as channels
                 ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
                 call("atl_voxel_grid_ws", ptr(pos), ptr(t), ptr(p), ptr(b), N, int(B), int(C), int(H), int(W),
@@ -401,7 +417,7 @@ class HipOps:
         out = torch.empty(M, device=ax.device, dtype=F32)
         args = (ptr(sy), ptr(sv), ptr(st), ptr(sid), ptr(cs), E, ncell, ptr(ax), ptr(at), ptr(ac), ptr(aid), M,
                 ptr(sc), int(S), int(GH), int(GW), float(h), float(tau), float(cut), ptr(out), ptr(count))
-        with torch.cuda.device(ax.device):
+        with on_device(ax.device):
             if plan_order:
                 call("atl_ats_pair_fwd", *args, stream_of(ax))
             else:
@@ -421,7 +437,7 @@ class HipOps:
         gv = torch.zeros(int(N), 2, device=ax.device, dtype=F32)
         args = (ptr(g), ptr(sy), ptr(sv), ptr(st), ptr(sid), ptr(cs), E, ncell, ptr(ax), ptr(at), ptr(ac), ptr(aid),
                 M, ptr(sc), int(S), int(GH), int(GW), float(h), float(tau), float(cut), int(N), ptr(gv))
-        with torch.cuda.device(ax.device):
+        with on_device(ax.device):
             if per_pair_atomics:
                 call("atl_ats_pair_bwd", *args, stream_of(ax))
             elif ws is not None:

@@ -24,7 +24,7 @@ import numpy as np
 import torch
 
 from . import reference as ref
-from ._ext import F32, I64, FastGeometry, HipLibraryError, call, ext_supports, get_ext, load_library, ptr, stream_of
+from ._ext import F32, I64, FastGeometry, HipLibraryError, call, ext_supports, get_ext, load_library, on_device, ptr, raw_stream, stream_of
 
 
 def _f32(t):
@@ -170,7 +170,7 @@ def _cached_copy(fld: torch.Tensor, layout: str, make) -> torch.Tensor:
     copies = _SCOPE.copies
     if copies is None:
         return make()
-    ver, st = fld._version, torch.cuda.current_stream(fld.device).cuda_stream
+    ver, st = fld._version, raw_stream(fld.device)
     for src, v, lay, s, cp in copies:
         if (lay == layout and v == ver and s == st and src.data_ptr() == fld.data_ptr() and src.shape == fld.shape
                 and src.stride() == fld.stride() and src.dtype == fld.dtype and src._version == ver):
@@ -185,7 +185,7 @@ def _channels_last(fld: torch.Tensor) -> torch.Tensor:
     def make():
         B, C, Hg, Wg = fld.shape
         fcl = torch.empty(B, Hg, Wg, 4 * ((C + 3) // 4), device=fld.device, dtype=F32)
-        with torch.cuda.device(fld.device):
+        with on_device(fld.device):
             call("atl_field_channels_last", ptr(fld), B, C, Hg, Wg, ptr(fcl), stream_of(fld))
         return fcl
     return _cached_copy(fld, "cl", make)
@@ -196,7 +196,7 @@ def _interleaved(fld: torch.Tensor) -> torch.Tensor:
     def make():
         B, _, Hg, Wg = fld.shape
         fil = torch.empty(B, Hg, Wg, 2, device=fld.device, dtype=F32)
-        with torch.cuda.device(fld.device):
+        with on_device(fld.device):
             call("atl_flow_interleave", ptr(fld), B, Hg, Wg, ptr(fil), stream_of(fld))
         return fil
     return _cached_copy(fld, "il", make)
@@ -225,7 +225,7 @@ class _SampleGrid(torch.autograd.Function):
         ctx.plan = None
         Q = (C + 3) // 4
         cl = _SampleGrid.CL_MIN_CHANNELS <= C <= 256 and N * Q < 2 ** 31 - 1024
-        with torch.cuda.device(pos.device):
+        with on_device(pos.device):
             st = stream_of(pos)
             if cl:
                 fcl = _channels_last(fld_in)
@@ -258,7 +258,7 @@ class _SampleGrid(torch.autograd.Function):
         B, C, Hg, Wg = ctx.shape
         g = g.contiguous().float()
         gf = gp = None
-        with torch.cuda.device(pos.device):
+        with on_device(pos.device):
             if ctx.needs_input_grad[0]:
                 gf = torch.zeros(B, C, Hg, Wg, device=pos.device, dtype=F32)
                 if ctx.rows:
@@ -304,7 +304,7 @@ class _WarpSplatGather(torch.autograd.Function):
         img = torch.empty(B, H, W, device=xy.device, dtype=F32)          # written by the launch
         vals = torch.empty(N, device=xy.device, dtype=F32)
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=xy.device)
-        with torch.cuda.device(xy.device):
+        with on_device(xy.device):
             call("atl_warp_splat_gather_fwd", ptr(grid), B, Hg, Wg, ptr(xy), ptr(t), ptr(b), N, H, W, float(t_ref),
                  int(bool(mask_border)), ptr(img), ptr(vals), ptr(ws), nbytes, stream_of(xy))
         ctx.save_for_backward(img, xy, t, b, ws)
@@ -321,7 +321,7 @@ class _WarpSplatGather(torch.autograd.Function):
         ggrid = torch.empty(B, 2, Hg, Wg, device=xy.device, dtype=F32)   # written by the launch
         gimg = None if gimg is None else gimg.contiguous().float()
         gvals = None if gvals is None else gvals.contiguous().float()
-        with torch.cuda.device(xy.device):
+        with on_device(xy.device):
             call("atl_warp_splat_gather_bwd", ptr(img), ptr(gvals), ptr(gimg), ptr(xy), ptr(t), ptr(b), xy.shape[0],
                  B, H, W, Hg, Wg, ctx.t_ref, ptr(ggrid), ptr(ws), ws.numel(), stream_of(xy))
         return ggrid, None, None, None, None, None, None, None
@@ -358,7 +358,7 @@ class _ImageVariance(torch.autograd.Function):
         if nbytes < 0:
             raise ValueError(f"image_variance: unsupported sizes {tuple(x.shape)}")
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
-        with torch.cuda.device(x.device):
+        with on_device(x.device):
             call("atl_image_variance", ptr(x), B, n, ptr(mean), ptr(var), ptr(ws), nbytes, stream_of(x))
         ctx.save_for_backward(x, mean)
         ctx.shape = (B, n)
@@ -370,7 +370,7 @@ class _ImageVariance(torch.autograd.Function):
         B, n = ctx.shape
         g = gvar.contiguous().float().view(B)
         gimg = torch.empty_like(x)
-        with torch.cuda.device(x.device):
+        with on_device(x.device):
             call("atl_image_variance_bwd", ptr(x), ptr(mean), ptr(g), B, n, ptr(gimg), stream_of(x))
         return gimg
 
@@ -399,7 +399,7 @@ class _TrajDisplacement(torch.autograd.Function):
         N = gpos.shape[0]
         out = torch.empty(N, 2, device=gpos.device, dtype=F32)
         ctx.plan = None
-        with torch.cuda.device(gpos.device):
+        with on_device(gpos.device):
             st = stream_of(gpos)
             fcl = _channels_last(fld)
             call("atl_traj_displacement", ptr(fcl), B, C, K, Hg, Wg, ptr(gpos), ptr(b), ptr(t), N, basis, ptr(out),
@@ -423,7 +423,7 @@ class _TrajDisplacement(torch.autograd.Function):
         N = gpos.shape[0]
         gd = gd.contiguous().float()
         gf = gp = None
-        with torch.cuda.device(gpos.device):
+        with on_device(gpos.device):
             st = stream_of(gpos)
             if ctx.bspline:
                 # the gradient rows are formed from gd and t inside both kernels (no (N, 2K) rows in memory)
@@ -527,7 +527,7 @@ class _TrajOrigin(torch.autograd.Function):
         fin = t_dst is not None
         P = torch.empty(n + int(fin), N, 2, device=xy.device, dtype=F32)   # grid coordinates of every look-up
         p = torch.empty(N, 2, device=xy.device, dtype=F32)
-        with torch.cuda.device(xy.device):
+        with on_device(xy.device):
             st = stream_of(xy)
             fcl = _channels_last(fld)
             call("atl_traj_origin", ptr(fcl), B, C, K, Hg, Wg, ptr(xy), ptr(t), ptr(b), N, n, float(offset), int(tile),
@@ -552,7 +552,7 @@ class _TrajOrigin(torch.autograd.Function):
         gD = torch.empty(n + int(fin), N, 2, device=gy.device, dtype=F32)   # gradient of every look-up
         gxy = torch.empty_like(gy) if ctx.needs_input_grad[1] else None
         gf = None
-        with torch.cuda.device(gy.device):
+        with on_device(gy.device):
             st = stream_of(gy)
             g = gy
             if fin:                                                  # y = p + d(p, t_dst)
@@ -637,7 +637,7 @@ def plan_stats(v: torch.Tensor, xa: torch.Tensor):
     """(vmax, min x, min y, max x, max y) of the plan geometry from one device reduction (one host sync)."""
     dev = v.device
     stats = torch.empty(5, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         call("atl_plan_stats", ptr(v), v.shape[0], ptr(xa), xa.shape[0], ptr(stats), stream_of(v))
     f = decode_ordered(stats.cpu().numpy())
     return float(f[0]), float(f[1]), float(f[2]), -float(f[3]), -float(f[4])
@@ -674,7 +674,7 @@ def _build_pair_plan_hip(x, t, v, b, B, H, W, anchors, h, tau, cut, n_slices, an
     b, anchors = b.contiguous().long(), anchors.contiguous().long()
     N, M = t.shape[0], anchors.shape[0]
     xa_all = _f32(x[anchors] if anchor_xy is None else anchor_xy.detach())
-    with torch.cuda.device(dev):
+    with on_device(dev):
         vmax, *bbox = plan_stats(vd, xa_all)
         geo = plan_geometry(vmax if N else 0.0, bbox, M, h, tau, cut, S, W, H)
         GW, GH, cell, ox, oy = geo["GW"], geo["GH"], geo["cell"], geo["ox"], geo["oy"]
@@ -860,7 +860,7 @@ class FastPairPlan:
                                       ctypes.byref(self.geo)) != 0:
             raise HipLibraryError("atl_fast_geometry_init: " + lib.atl_last_error().decode(errors="replace"))
         self.ws = torch.empty(int(self.geo.ws_bytes), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with on_device(dev):
             if self.traj:
                 call("atl_fast_plan_traj", ctypes.byref(self.geo), ptr(self.x), ptr(self.coef), self.K,
                      ptr(self.table), ptr(self.t), ptr(self.b), ptr(self.anchors), ptr(self.anchor_xy), ptr(self.ws),
@@ -871,7 +871,7 @@ class FastPairPlan:
 
     def forward(self, count: Optional[torch.Tensor] = None) -> torch.Tensor:
         out = torch.zeros(self.M, dtype=F32, device=self.device)
-        with torch.cuda.device(self.device):
+        with on_device(self.device):
             call("atl_fast_pair_fwd", ctypes.byref(self.geo), ptr(self.ws), ptr(out), ptr(count), stream_of(out))
         return out
 
@@ -887,7 +887,7 @@ class FastPairPlan:
             raise ValueError("a trajectory plan has backward_traj")
         gS = self._check_gs(gS)
         gv = torch.empty(self.N, 2, dtype=F32, device=self.device)
-        with torch.cuda.device(self.device):
+        with on_device(self.device):
             call("atl_fast_pair_bwd", ctypes.byref(self.geo), ptr(self.ws), ptr(gS), ptr(gv), stream_of(gv))
         return gv
 
@@ -899,7 +899,7 @@ class FastPairPlan:
             raise ValueError("a trajectory plan has backward_traj")
         gS = self._check_gs(gS)
         gg = torch.empty(int(B), 2, int(Hg), int(Wg), dtype=F32, device=self.device)   # written by the adjoint
-        with torch.cuda.device(self.device):
+        with on_device(self.device):
             st = stream_of(gg)
             call("atl_fast_pair_bwd_src", ctypes.byref(self.geo), ptr(self.ws), ptr(gS), st)
             call("atl_fast_flow_adjoint", ctypes.byref(self.geo), ptr(self.ws), int(Hg), int(Wg), int(img_h),
@@ -913,7 +913,7 @@ class FastPairPlan:
         gS = self._check_gs(gS)
         gp = torch.empty(self.N, 2, dtype=F32, device=self.device)
         gc = torch.empty(self.N, 2 * self.K, dtype=F32, device=self.device)
-        with torch.cuda.device(self.device):
+        with on_device(self.device):
             call("atl_fast_pair_bwd_traj", ctypes.byref(self.geo), ptr(self.ws), ptr(gS), ptr(self.coef), self.K,
                  ptr(self.table), ptr(gp), ptr(gc), stream_of(gp))
         return gp, gc
@@ -1060,7 +1060,7 @@ def events_sorted(t: torch.Tensor, b: torch.Tensor) -> bool:
     """True if the keys b*4 + t ascend in event order (device check, one host sync)."""
     t, b = _f32(t), b.contiguous().long()
     flag = torch.empty(1, dtype=torch.int32, device=t.device)
-    with torch.cuda.device(t.device):
+    with on_device(t.device):
         call("atl_check_sorted", ptr(t), ptr(b), t.shape[0], ptr(flag), stream_of(t))
     return int(flag.item()) == 0
 
@@ -1095,7 +1095,7 @@ def window_counts(t: torch.Tensor, b: torch.Tensor, idx: torch.Tensor, tau: floa
         t, b, idx = t[order].contiguous(), b[order].contiguous(), inv[idx].contiguous()
     M = t.shape[0] if idx is None else idx.shape[0]
     out = torch.empty(M, dtype=F32, device=t.device)
-    with torch.cuda.device(t.device):
+    with on_device(t.device):
         call("atl_window_counts", ptr(t), ptr(b), t.shape[0], ptr(idx), M, float(tau), ptr(out), stream_of(t))
     return out
 
@@ -1127,7 +1127,7 @@ def event_noise(xy: torch.Tensor, seed: int, offset: int, h: float, dequantize: 
         raise ValueError("xy must be (N, 2)")
     xs = torch.empty_like(xy)
     xa = torch.empty_like(xy) if smooth else None
-    with torch.cuda.device(xy.device):
+    with on_device(xy.device):
         call("atl_event_noise", ptr(xy), xy.shape[0], int(seed) & (2 ** 64 - 1), int(offset) & (2 ** 64 - 1),
              float(h), int(bool(dequantize)), ptr(xs), ptr(xa), stream_of(xy))
     return xs, xa
@@ -1139,7 +1139,7 @@ def bin_counts(t_all, b_all, B, n_check=16, assume_sorted: bool = False) -> torc
     atomics."""
     t_all, b_all = _f32(t_all), b_all.contiguous().long()
     dev = t_all.device
-    with torch.cuda.device(dev):
+    with on_device(dev):
         if assume_sorted:
             counts = torch.empty(B, n_check, dtype=F32, device=dev)
             call("atl_bin_counts_sorted", ptr(t_all), ptr(b_all), t_all.shape[0], B, n_check, ptr(counts),
@@ -1159,7 +1159,7 @@ def visible_fraction_linear(xa, va, ta, ba, t_all, b_all, B, H, W, tau, n_check=
     counts = bin_counts(t_all, b_all, B, n_check, assume_sorted)
     out = torch.empty(ta.shape[0], dtype=F32, device=dev)
     centres = bin_centres(n_check, dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         st = stream_of(xa)
         call("atl_visible_fraction", ptr(xa), ptr(va), ptr(ta), ptr(ba), ta.shape[0], ptr(counts), ptr(centres), B,
              n_check, float(tau), int(H), int(W), ptr(out), st)
@@ -1182,7 +1182,7 @@ def traj_visible_fraction(fld, K: int, basis: str, n_fp: int, offset: float, til
     edges = torch.linspace(0, 1, n_check + 1, device=dev)
     centres = (0.5 * (edges[:-1] + edges[1:])).contiguous()
     out = torch.empty(ta.shape[0], dtype=F32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         call("atl_traj_visible", ptr(_channels_last(fld)), B_, C, int(K), Hg, Wg, ptr(xa), ptr(ta), ptr(ba),
              ta.shape[0], int(n_fp), float(offset), int(tile), TRAJ_BASES[basis], ptr(counts), ptr(centres), n_check,
              float(tau), int(H), int(W), ptr(out), stream_of(xa))
@@ -1198,7 +1198,7 @@ class _AnchoredEpilogue(torch.autograd.Function):
         vis = None if vis is None else _f32(vis)
         M = S.shape[0]
         ls, q, D = (torch.empty(M, dtype=F32, device=S.device) for _ in range(3))
-        with torch.cuda.device(S.device):
+        with on_device(S.device):
             call("atl_anchored_epilogue_fwd", ptr(S), ptr(wc), ptr(vis), M, float(h), float(eps), ptr(ls), ptr(q),
                  ptr(D), stream_of(S))
         ctx.save_for_backward(q, D)
@@ -1209,7 +1209,7 @@ class _AnchoredEpilogue(torch.autograd.Function):
         q, D = ctx.saved_tensors
         gS = torch.empty_like(q)
         g = g.contiguous().float()
-        with torch.cuda.device(q.device):
+        with on_device(q.device):
             call("atl_anchored_epilogue_bwd", ptr(g), ptr(q), ptr(D), q.shape[0], ptr(gS), stream_of(q))
         return gS, None, None, None, None
 
@@ -1237,7 +1237,7 @@ class _AnchoredScoreMean(torch.autograd.Function):
         q, D = (torch.empty(M, dtype=F32, device=S.device) for _ in range(2))
         out = torch.empty(2, dtype=F32, device=S.device)
         st = stream_of(S)
-        with torch.cuda.device(S.device):
+        with on_device(S.device):
             call("atl_anchored_score_mean_fwd", ptr(S), ptr(wc), ptr(vis), M, float(h), float(eps), ptr(q), ptr(D),
                  ptr(_mean_scratch(S.device)), ptr(out), st)
         ctx.save_for_backward(q, D)
@@ -1253,7 +1253,7 @@ class _AnchoredScoreMean(torch.autograd.Function):
         q, D = ctx.saved_tensors
         gS = torch.empty_like(q)
         g = g.contiguous().float()
-        with torch.cuda.device(q.device):
+        with on_device(q.device):
             call("atl_anchored_score_mean_bwd", ptr(g), ptr(q), ptr(D), q.shape[0], ptr(gS), stream_of(q))
         return gS, None, None, None, None
 
@@ -1333,7 +1333,7 @@ def knn_indices(queries: torch.Tensor, points: torch.Tensor, k: int, chunk: int 
     if nbytes < 0:
         raise ValueError(f"knn_indices: {B * T} planes of {n} points are too many for 32-bit cell indices")
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=pts.device)
-    with torch.cuda.device(pts.device):
+    with on_device(pts.device):
         call("atl_knn_indices", ptr(q), Q, ptr(pts), B * T, n, k, ptr(out), ptr(ws), nbytes, stream_of(pts))
     return out
 
@@ -1363,7 +1363,7 @@ class _TileTrajectories(torch.autograd.Function):
         ctx.save_for_backward(times)
         ctx.shape, ctx.kind = (B, K, Hq, Wq), kind
         out = torch.empty(B, nt, Hq * Wq, 2, device=coef.device, dtype=F32)
-        with torch.cuda.device(coef.device):
+        with on_device(coef.device):
             call("atl_tile_trajectories", ptr(coef), *coef.stride(), B, K, Hq, Wq, offset, tile, ptr(times), nt,
                  TRAJ_BASES[kind], ptr(out), stream_of(coef))
         return out
@@ -1378,7 +1378,7 @@ class _TileTrajectories(torch.autograd.Function):
             return gc.reshape(B, 2 * K, Hq, Wq), None, None, None, None, None
         g = g.contiguous()
         gc = torch.empty(B, 2 * K, Hq, Wq, device=g.device, dtype=F32)
-        with torch.cuda.device(g.device):
+        with on_device(g.device):
             call("atl_tile_trajectories_bwd", ptr(g), B, K, Hq, Wq, ptr(times), times.shape[0], TRAJ_BASES[ctx.kind],
                  ptr(gc), stream_of(g))
         return gc, None, None, None, None, None
@@ -1418,7 +1418,7 @@ class _LutTable(torch.autograd.Function):
         nbytes = load_library().atl_lut_table_ws_bytes(B, T, n, nx, ny)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=tr.device)
         out = torch.empty(B, T, ny * nx, 2, device=tr.device, dtype=F32)
-        with torch.cuda.device(tr.device):
+        with on_device(tr.device):
             call("atl_lut_table_fwd", ptr(tr), B, T, n, x0, y0, step, nx, ny, k, ptr(out), ptr(ws), nbytes,
                  stream_of(tr))
         ctx.save_for_backward(tr, ws)
@@ -1440,7 +1440,7 @@ class _LutTable(torch.autograd.Function):
             return torch.cat([gd.sum(1, keepdim=True), -gd], 1), None, None, None, None, None, None
         g = g.contiguous()
         gtr = torch.empty_like(tr)
-        with torch.cuda.device(g.device):
+        with on_device(g.device):
             call("atl_lut_table_bwd", ptr(g), B, T, n, x0, y0, step, nx, ny, k, ptr(ws), ws.numel(), ptr(gtr),
                  stream_of(g))
         return gtr, None, None, None, None, None, None
