@@ -777,3 +777,58 @@ def test_image_variance_matches_fp64(shape):
     (v * T(g)).sum().backward()
     (v64 * torch.as_tensor(g.astype(np.float64))).sum().backward()
     close_rel(N(x.grad), x64.grad.numpy(), 1e-5)
+
+
+@pytest.mark.parametrize("H,W,sigma,R", [(9, 7, 0.4, 0), (20, 24, 0.6, 1), (33, 47, 1.0, 3), (33, 47, 1.6, 5), (12, 70, 3.0, 9),
+                                         (40, 30, 3.3, 10)])
+def test_splat_gauss_backward_columns_and_radii(H, W, sigma, R):
+    # every column count of the four-lane backward, centres up to R outside the image, and the wider fallback (R = 10)
+    print(f"gauss backward {H}x{W} sigma={sigma} R={R}", flush=True)
+    rng = np.random.default_rng(R)
+    n = 515
+    pos = (rng.random((n, 2)) * [W + 2 * R + 2, H + 2 * R + 2] - R - 1).astype(np.float32)
+    w, b = rng.normal(size=n).astype(np.float32), rng.integers(0, 2, n)
+    g = rng.normal(size=(2, H, W)).astype(np.float32)
+    gp, gw = F.get_ext().splat_gauss_bwd(T(g), T(pos), T(w), T(b), sigma, R)
+    wp, ww = O.splat_gauss_bwd(g, pos, w, b, sigma, R)
+    # (2 R + 1)^2 terms of either sign: fp32 sums to a few ulp of the largest result
+    assert np.abs(N(gw) - ww).max() <= 1e-5 * np.abs(ww).max()
+    assert np.abs(N(gp) - wp).max() <= 1e-5 * np.abs(wp).max()
+
+
+@pytest.mark.parametrize("C", [1, 2, 24, 25])
+def test_voxel_chains_crowded_pixels(C):
+    # 24 bins are the most that the chained accumulation's LDS holds; crowded base voxels over several rounds
+    print(f"voxel chains C={C}", flush=True)
+    rng = np.random.default_rng(C)
+    n, H, W = 6000, 40, 50
+    pos = (rng.random((n, 2)) * [W, H]).astype(np.float32)
+    pos[:2500] = [17.25, 9.5]
+    pos[2500:2520] = [-0.5, H - 0.75]
+    t = rng.random(n).astype(np.float32)
+    t[:1200] = 0.5
+    p, b = rng.normal(size=n).astype(np.float32), rng.integers(0, 2, n)
+    got = N(F.voxel_grid(T(pos), T(t), T(p), T(b), 2, C, H, W, normalize=None))
+    mag = float(O.voxel_grid(pos, t, np.abs(p), b, 2, C, H, W).max())
+    _voxel_cases_close(got, O.voxel_grid(pos, t, p, b, 2, C, H, W), mag)
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (3, 7), (2, 4096), (2, 4097), (1, 5 * 4096 + 3), (2, 1025 * 4096 + 4)])
+def test_standardise_nonzero_rows(shape):
+    print(f"standardise {shape}", flush=True)
+    g = torch.Generator().manual_seed(shape[1])
+    x = torch.randn(*shape, generator=g) * 3 + 1
+    x[torch.rand(*shape, generator=g) < 0.6] = 0
+    x[0, -1] = 2.5
+    d = x.to(DEV)
+    F._standardise_nonzero(d)
+    want = x.double()
+    for row in want:
+        nz = row != 0
+        if nz.sum() > 1:
+            row[nz] = (row[nz] - row[nz].mean()) / row[nz].std()
+        else:
+            row[nz] = 0.0
+    # the mean and the deviation are rounded to fp32 once each, then two operations
+    assert (d.cpu().double() - want).abs().max() <= 8 * 2.0 ** -24 * max(float(want.abs().max()), 1.0)
+    assert torch.equal(d.cpu() == 0, want.float() == 0) or shape[1] == 1

@@ -168,6 +168,71 @@ __global__ void __launch_bounds__(kBlock) k_splat_gauss_bwd(const float* __restr
   gpos[n] = make_float2(wn * sx, wn * sy);
 }
 
+// The same backward with four lanes per event for R <= kGaussQuadR: a lane takes every fourth column (NC of them),
+// so that the four read a row's pixels side by side, and the weight is the product of a column and a row factor,
+// NC + 2 R + 1 exponentials per lane instead of (2 R + 1)^2 per event.  100k events of R = 3: 21.8 -> 8.2 us (one
+// lane per event left 1.5 waves per SIMD, each waiting on 49 loads).
+constexpr int kGaussQuadR = 9;
+template <int NC>
+__global__ void __launch_bounds__(kBlock) k_splat_gauss_bwd_quad(const float* __restrict__ gimg,
+                                                                 const float2* __restrict__ pos,
+                                                                 const float* __restrict__ w,
+                                                                 const int64_t* __restrict__ bidx, int64_t N,
+                                                                 int64_t B, int H, int W, float inv2s2, float norm,
+                                                                 float s2, int R, float2* __restrict__ gpos,
+                                                                 float* __restrict__ gw) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int64_t n = i >> 2;
+  const int l = (int)i & 3;
+  float sw = 0.f, sx = 0.f, sy = 0.f;
+  if (n < N) {
+    const int64_t b = bidx[n];
+    const float2 p = pos[n];
+    const float rx = roundf(p.x), ry = roundf(p.y);
+    if (batch_ok(b, B) &&
+        rx >= (float)(-R) && rx <= (float)(W - 1 + R) && ry >= (float)(-R) && ry <= (float)(H - 1 + R)) {
+      const int cx = (int)rx, cy = (int)ry;
+      const float* base = gimg + b * (int64_t)H * W;
+      float ex[NC], dx[NC];
+      int col[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int xx = cx - R + l + 4 * c;
+        dx[c] = (float)xx - p.x;
+        const bool in = xx >= 0 && xx < W && xx <= cx + R;
+        ex[c] = in ? expf(-(dx[c] * dx[c]) * inv2s2) : 0.f;
+        col[c] = in ? xx : -1;
+      }
+      const int ylo = max(cy - R, 0), yhi = min(cy + R, H - 1);
+      for (int yy = ylo; yy <= yhi; ++yy) {
+        const float dy = (float)yy - p.y;
+        const float ey = expf(-(dy * dy) * inv2s2);
+        float r0 = 0.f, r1 = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const float v = col[c] >= 0 ? base[yy * W + col[c]] : 0.f;
+          const float e = ex[c] * v;
+          r0 += e;
+          r1 += e * dx[c];
+        }
+        sw += ey * r0;
+        sx += ey * r1;
+        sy += ey * (dy * r0);
+      }
+    }
+  }
+#pragma unroll
+  for (int d = 1; d <= 2; d <<= 1) {
+    sw += __shfl_xor(sw, d, kWave);
+    sx += __shfl_xor(sx, d, kWave);
+    sy += __shfl_xor(sy, d, kWave);
+  }
+  if (n >= N || l != 0) return;
+  gw[n] = sw * norm;
+  const float k = w[n] * norm;
+  gpos[n] = make_float2(k * sx / s2, k * sy / s2);
+}
+
 // Trilinear polarity voting, csrc/atl_cpu.cpp:256-286.
 __global__ void __launch_bounds__(kBlock) k_voxel_grid(const float2* __restrict__ pos, const float* __restrict__ t,
                                                        const float* __restrict__ pol,
@@ -1196,8 +1261,18 @@ int atl_splat_gauss_bwd(const float* gimg, const float* pos, const float* w, con
   if (N == 0) return 0;
   const float s2 = (float)(sigma * sigma);
   const float inv2s2 = 1.f / (2.f * s2), norm = 1.f / (2.f * (float)M_PI * s2);
-  hipLaunchKernelGGL(k_splat_gauss_bwd, dim3(grid_for(N)), dim3(kBlock), 0, stream, gimg, (const float2*)pos, w, b,
+  const int nc = R <= kGaussQuadR ? (int)(2 * R + 4) / 4 : 0;   // columns per lane
+  const dim3 qgrid(grid_for(4 * N));
+  switch (nc) {
+#define ATL_GAUSS_CASE(k) \
+    case k: hipLaunchKernelGGL(k_splat_gauss_bwd_quad<k>, qgrid, dim3(kBlock), 0, stream, gimg, (const float2*)pos, w, b, N, B, \
+                                (int)H, (int)W, inv2s2, norm, s2, (int)R, (float2*)gpos, gw); break;
+    ATL_GAUSS_CASE(1) ATL_GAUSS_CASE(2) ATL_GAUSS_CASE(3) ATL_GAUSS_CASE(4) ATL_GAUSS_CASE(5)
+#undef ATL_GAUSS_CASE
+    default:
+      hipLaunchKernelGGL(k_splat_gauss_bwd, dim3(grid_for(N)), dim3(kBlock), 0, stream, gimg, (const float2*)pos, w, b,
                      N, B, (int)H, (int)W, inv2s2, norm, s2, (int)R, (float2*)gpos, gw);
+  }
   return check_launch("splat_gauss_bwd");
 }
 

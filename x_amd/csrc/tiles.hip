@@ -590,6 +590,189 @@ __global__ void __launch_bounds__(kAccBlock) k_tile_accum_bins(const int4* __res
   }
 }
 
+// Voxel grid without LDS float atomics (16 x 16 tiles): eight of them per record bound the scatter form (60 us for
+// 1M events in 15 bins of 640 x 480; see k_tile_accum_bins for their rate).  The records of a round are chained by
+// base voxel (time bin and base corner) with one LDS integer exchange each; the thread whose record opened a chain
+// adds up the chain's eight corner sums in registers (most chains hold one to three records: the time bins spread
+// the crowded pixels of an edge), and the sums are then added into the window in eight phases, one per corner.  In
+// one phase all base voxels write different voxels, so the additions are plain LDS reads and writes.  35 us on the same input.
+constexpr int kVoxChainLds = 65536;               // bytes of LDS for the window, the chain heads and the records
+inline size_t vox_chain_lds(int C) {
+  return (size_t)C * (kBinT + 1) * (kBinT + 1) * 4 + (size_t)(C + 1) * kBins * 4 + (size_t)kAccChunk * 20;
+}
+
+__global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restrict__ info,
+                                                           const int* __restrict__ nchunk,
+                                                           const float4* __restrict__ rec, TileGeo g,
+                                                           float* __restrict__ out) {
+  constexpr int T = kBinT, L = T + 1;
+  extern __shared__ float4 vlds[];
+  float4* srec = vlds;                            // kAccChunk records
+  int* snext = (int*)(srec + kAccChunk);          // the next record of the chain, -1 at its end
+  int* head = snext + kAccChunk;                  // (C + 1) x kBins chain heads, -1: empty
+  float* acc = (float*)(head + (g.C + 1) * kBins);   // C x L x L window
+  if ((int)blockIdx.x >= *nchunk) return;
+  const int4 ci = info[blockIdx.x];
+  const int key = ci.x, s0 = ci.y, s1 = ci.z;
+  const int tid = threadIdx.x;
+  for (int i = tid; i < (g.C + 1) * kBins; i += kAccBlock) head[i] = -1;
+  for (int i = tid; i < g.C * L * L; i += kAccBlock) acc[i] = 0.f;
+  const int64_t pl = (int64_t)g.H * g.W;
+  const int plane = g.TY * g.TX;
+  const int b = key / plane, r = key - b * plane;
+  const int ty = r / g.TX, tx = r - ty * g.TX;
+  const int ox = tx * T - 1, oy = ty * T - 1;
+  __syncthreads();
+  for (int base = s0; base < s1; base += kAccChunk) {
+    int vox[kAccItems];                           // the chain this thread's record opened, -1: none
+    int prev[kAccItems];
+#pragma unroll
+    for (int u = 0; u < kAccItems; ++u) {
+      const int i = u * kAccBlock + tid, k = base + i;
+      vox[u] = -1;
+      prev[u] = 0;
+      if (k < s1) {
+        const float4 q = rec[k];
+        int x0, y0;
+        const int t1 = (int)floorf(q.w) + 1;      // base time bin + 1
+        if (image_base(q.x, q.y, g.H, g.W, x0, y0) && (unsigned)t1 <= (unsigned)g.C) {   // as the binning tested
+          srec[i] = make_float4(q.x - (float)x0, q.y - (float)y0, q.z, q.w - (float)(t1 - 1));
+          vox[u] = (t1 * T + (y0 - oy)) * T + (x0 - ox);
+          prev[u] = atomicExch(head + vox[u], i);
+          snext[i] = prev[u];
+        }
+      }
+    }
+    __syncthreads();
+    float s[kAccItems][8];
+#pragma unroll
+    for (int u = 0; u < kAccItems; ++u) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s[u][k] = 0.f;
+      if (vox[u] < 0) continue;
+      if (prev[u] != -1) {                        // not the chain's first record: another thread adds it up
+        vox[u] = -1;
+        continue;
+      }
+      // the corner weights 1 - |corner - position| are a fraction or one minus it, from exact differences
+      for (int i = head[vox[u]]; i >= 0; i = snext[i]) {
+        const float4 q = srec[i];
+        const float wx[2] = {1.f - q.x, 1.f - (1.f - q.x)}, wy[2] = {1.f - q.y, 1.f - (1.f - q.y)},
+                    wt[2] = {1.f - q.w, 1.f - (1.f - q.w)};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s[u][k] += q.z * wt[k >> 2] * wy[(k >> 1) & 1] * wx[k & 1];
+      }
+      head[vox[u]] = -1;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+#pragma unroll
+      for (int u = 0; u < kAccItems; ++u) {
+        if (vox[u] < 0) continue;
+        const int tt = vox[u] / (T * T) - 1 + (k >> 2);
+        const int ly = (vox[u] / T) % T + ((k >> 1) & 1), lx = vox[u] % T + (k & 1);
+        if ((unsigned)tt < (unsigned)g.C) acc[(tt * L + ly) * L + lx] += s[u][k];
+      }
+      __syncthreads();
+    }
+  }
+  for (int a = tid; a < L * L; a += kAccBlock) {
+    const int py = oy + a / L, px = ox + a % L;
+    if (py < 0 || py >= g.H || px < 0 || px >= g.W) continue;
+    for (int ch = 0; ch < g.C; ++ch) {
+      const float v = acc[ch * L * L + a];
+      if (v != 0.f) atomicAdd(out + ((int64_t)b * g.C + ch) * pl + (int64_t)py * g.W + px, v);
+    }
+  }
+}
+
+// Truncated-Gaussian splat in gather form (16 x 16 tiles): the scatter form's (2 R + 1)^2 LDS float atomics per
+// record took 47 us for 100k events of radius 3 on 320 x 240.  A round's records are put in the row-major order of
+// their centres (one LDS integer atomic each); the centres that reach a window pixel from one row then stand side by
+// side, and the pixel's thread adds up its 2 R + 1 runs, the same fp32 products, in registers: 23.5 us.
+constexpr int kGaussPix = 4;                      // window pixels per thread: (16 + 2 R)^2 <= 1024 for R <= 8
+static_assert((kBinT + 2 * kMaxGaussRadius) * (kBinT + 2 * kMaxGaussRadius) <= kGaussPix * kAccBlock, "window");
+
+__global__ void __launch_bounds__(kAccBlock) k_gauss_accum(const int4* __restrict__ info,
+                                                           const int* __restrict__ nchunk,
+                                                           const float4* __restrict__ rec, TileGeo g,
+                                                           float* __restrict__ out) {
+  constexpr int T = kBinT;
+  __shared__ int bcnt[kBins];
+  __shared__ int bstart[kBins + 1];
+  __shared__ int wsum[kAccBlock / kWave + 1];
+  __shared__ float sx[kAccChunk], sy[kAccChunk], sw[kAccChunk];
+  if ((int)blockIdx.x >= *nchunk) return;
+  const int4 ci = info[blockIdx.x];
+  const int key = ci.x, s0 = ci.y, s1 = ci.z;
+  const int tid = threadIdx.x, R = g.R, L = T + 2 * R;
+  const int plane = g.TY * g.TX;
+  const int b = key / plane, r = key - b * plane;
+  const int ty = r / g.TX, tx = r - ty * g.TX;
+  const int ox = tx * T - 2 * R, oy = ty * T - 2 * R;   // window column, row 0; centre columns start R later
+  float s[kGaussPix] = {};
+  for (int base = s0; base < s1; base += kAccChunk) {
+    float4 q[kAccItems];
+    int bin[kAccItems], rank[kAccItems];
+    bcnt[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kAccItems; ++u) {
+      const int k = base + u * kAccBlock + tid;
+      bin[u] = -1;
+      rank[u] = 0;
+      int cx, cy;
+      if (k < s1) {
+        q[u] = rec[k];
+        if (gauss_centre(q[u].x, q[u].y, g, cx, cy)) {   // always: the binning applied this test
+          bin[u] = (cy - oy - R) * T + (cx - ox - R);
+          rank[u] = atomicAdd(bcnt + bin[u], 1);
+        }
+      }
+    }
+    __syncthreads();
+    int total;
+    const int first = block_exclusive_scan<kAccBlock>(bcnt[tid], wsum, total);
+    bstart[tid] = first;
+    if (tid == 0) bstart[kBins] = total;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kAccItems; ++u) {
+      if (bin[u] < 0) continue;
+      const int p = bstart[bin[u]] + rank[u];
+      sx[p] = q[u].x;
+      sy[p] = q[u].y;
+      sw[p] = q[u].z * g.norm;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kGaussPix; ++u) {
+      const int a = u * kAccBlock + tid;
+      if (a >= L * L) break;
+      const int ly = a / L, lx = a - ly * L;
+      const float fx = (float)(ox + lx), fy = (float)(oy + ly);
+      // centres within R: columns lx - 2 R .. lx and rows ly - 2 R .. ly of the tile's 16 x 16
+      const int c0 = max(lx - 2 * R, 0), c1 = min(lx, T - 1);
+      for (int row = max(ly - 2 * R, 0); row <= min(ly, T - 1); ++row) {
+        const int e = bstart[row * T + c1 + 1];
+        for (int p = bstart[row * T + c0]; p < e; ++p) {
+          const float dx = fx - sx[p], dy = fy - sy[p];
+          s[u] += sw[p] * expf(-(dx * dx + dy * dy) * g.inv2s2);
+        }
+      }
+    }
+    __syncthreads();                              // the next round reuses the counts and the sorted records
+  }
+#pragma unroll
+  for (int u = 0; u < kGaussPix; ++u) {
+    const int a = u * kAccBlock + tid;
+    if (a >= L * L) break;
+    const int py = oy + a / L, px = ox + a % L;
+    if (py < 0 || py >= g.H || px < 0 || px >= g.W || s[u] == 0.f) continue;
+    atomicAdd(out + ((int64_t)b * g.H + py) * g.W + px, s[u]);
+  }
+}
+
 // Many-channel grid adjoint (kGrid, C > 4 channels, 16 x 16 tiles) in the gather form of k_tile_accum_bins: each
 // round of up to 512 records is ranked by base node with one LDS integer atomic each and its fractions are stored
 // in base-node order; then, four channels at a time, every thread loads those channels of its own records (16
@@ -1322,6 +1505,83 @@ __global__ void k_tile_zero1(int* p) { p[0] = 0; }
 // ATL_TILE_SCATTER=1 in the environment selects the scatter form of the accumulation for every mode (read at
 // every call, so that a test can compare both forms in one process).  A backward that reuses its forward's chunk
 // list may therefore run the other form on it: the scatter form takes chunks of any length, in rounds.
+// Standardisation of a row's non-zero entries (x - mean) / sd in place (sd of n - 1; 1 where it is not positive, as
+// for a single entry): chunk sums of count, x and x^2 in fp64, then every workgroup adds up its row's chunk sums in a
+// fixed order and rewrites its own chunk.  Two launches that read the row twice and write it once; the twenty torch
+// operations they replace (masks, where, sums, products) took 125 us on a 15 x 480 x 640 grid, these 15 us.
+constexpr int kStdChunk = 4096, kStdMaxChunks = 1024;
+struct NzPart {
+  double n, s, q;
+};
+inline int64_t std_chunks(int64_t n) {
+  const int64_t c = (n + kStdChunk - 1) / kStdChunk;
+  return c < 1 ? 1 : c > kStdMaxChunks ? kStdMaxChunks : c;
+}
+
+__device__ __forceinline__ NzPart nz_block_sum(NzPart v, double (&lds)[3][kBlock / kWave]) {
+  v.n = wave_sum(v.n); v.s = wave_sum(v.s); v.q = wave_sum(v.q);
+  const int w = threadIdx.x / kWave;
+  if ((threadIdx.x & (kWave - 1)) == 0) { lds[0][w] = v.n; lds[1][w] = v.s; lds[2][w] = v.q; }
+  __syncthreads();
+  NzPart t{0., 0., 0.};
+#pragma unroll
+  for (int k = 0; k < kBlock / kWave; ++k) { t.n += lds[0][k]; t.s += lds[1][k]; t.q += lds[2][k]; }
+  return t;
+}
+
+__global__ void __launch_bounds__(kBlock) k_nz_part(const float* __restrict__ x, int64_t n, int64_t per, int vec,
+                                                    NzPart* __restrict__ part) {
+  __shared__ double lds[3][kBlock / kWave];
+  const float* row = x + blockIdx.y * n;
+  const int64_t i0 = blockIdx.x * per, i1 = min(i0 + per, n);
+  int c = 0;
+  double s = 0., q = 0.;
+  auto add = [&](float v) {
+    c += v != 0.f ? 1 : 0;
+    const double d = (double)v;
+    s += d;
+    q += d * d;
+  };
+  if (vec) {
+    for (int64_t i = i0 + 4 * threadIdx.x; i < i1; i += 4 * kBlock) {
+      const float4 v = *(const float4*)(row + i);
+      add(v.x); add(v.y); add(v.z); add(v.w);
+    }
+  } else {
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += kBlock) add(row[i]);
+  }
+  const NzPart t = nz_block_sum(NzPart{(double)c, s, q}, lds);
+  if (threadIdx.x == 0) part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = t;
+}
+
+__global__ void __launch_bounds__(kBlock) k_nz_apply(float* __restrict__ x, int64_t n, int64_t per, int vec,
+                                                     const NzPart* __restrict__ part) {
+  __shared__ double lds[3][kBlock / kWave];
+  NzPart v{0., 0., 0.};
+  for (int k = threadIdx.x; k < (int)gridDim.x; k += kBlock) {
+    const NzPart p = part[(int64_t)blockIdx.y * gridDim.x + k];
+    v.n += p.n; v.s += p.s; v.q += p.q;
+  }
+  const NzPart t = nz_block_sum(v, lds);
+  const double mu = t.s / fmax(t.n, 1.);
+  const double var = fmax(t.q - t.s * mu, 0.) / (t.n - 1.);     // 0 / 0 for a single entry: not positive below
+  const bool nan = !(t.q - t.s * mu >= 0.) && !(t.q - t.s * mu < 0.);   // fmax drops a NaN
+  const float mean = (float)mu, sd = nan ? 1.f : (float)sqrt(var);
+  const float div = sd > 0.f ? sd : 1.f;
+  float* row = x + blockIdx.y * n;
+  const int64_t i0 = blockIdx.x * per, i1 = min(i0 + per, n);
+  auto one = [&](float a) { return a != 0.f ? (a - mean) / div : a; };
+  if (vec) {
+    for (int64_t i = i0 + 4 * threadIdx.x; i < i1; i += 4 * kBlock) {
+      float4 a = *(const float4*)(row + i);
+      a.x = one(a.x); a.y = one(a.y); a.z = one(a.z); a.w = one(a.w);
+      *(float4*)(row + i) = a;
+    }
+  } else {
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += kBlock) row[i] = one(row[i]);
+  }
+}
+
 bool tile_scatter_form() {
   const char* e = std::getenv("ATL_TILE_SCATTER");
   return e && e[0] == '1';
@@ -1332,9 +1592,9 @@ bool tile_scatter_form() {
 // form.
 template <int MODE, int C>
 bool tile_gather(const TileGeo& g) {
-  constexpr bool kGatherForm =
-      MODE == kImage || MODE == kImageG || MODE == kGridVal || (MODE == kGrid && C >= 1 && C <= 4);
-  return kGatherForm && g.T == kBinT && !tile_scatter_form();
+  constexpr bool kGatherForm = MODE == kImage || MODE == kImageG || MODE == kGridVal || MODE == kGauss ||
+                               MODE == kVoxel || (MODE == kGrid && C >= 1 && C <= 4);
+  return kGatherForm && g.T == kBinT && (MODE != kVoxel || vox_chain_lds(g.C) <= kVoxChainLds) && !tile_scatter_form();
 }
 
 template <int MODE, int C>
@@ -1384,8 +1644,14 @@ void tile_accum(const TileGeo& g, const TileLayout& L, const void* ws, const flo
   const int nc = C > 0 ? C : g.C;
   const size_t edge = MODE == kGauss ? (size_t)(g.T + 2 * g.R) : (size_t)(g.T + 1);
   const size_t lds = (size_t)nc * edge * edge * sizeof(float);
-  if (gather)
-    hipLaunchKernelGGL((k_tile_accum_bins<MODE, kGatherForm ? (C > 0 ? C : 1) : 1>), dim3(grid), dim3(kAccBlock), 0,
+  if (gather && MODE == kVoxel)
+    hipLaunchKernelGGL(k_voxel_accum, dim3(grid), dim3(kAccBlock), vox_chain_lds(g.C), stream, (const int4*)info,
+                       (const int*)nchunk, (const float4*)(w + L.rec), g, out);
+  else if (gather && MODE == kGauss)
+    hipLaunchKernelGGL(k_gauss_accum, dim3(grid), dim3(kAccBlock), 0, stream, (const int4*)info, (const int*)nchunk,
+                       (const float4*)(w + L.rec), g, out);
+  else if (gather)
+    hipLaunchKernelGGL((k_tile_accum_bins<kGatherForm ? MODE : kImage, kGatherForm ? (C > 0 ? C : 1) : 1>), dim3(grid), dim3(kAccBlock), 0,
                        stream, (const int4*)info, (const int*)nchunk, (const float4*)(w + L.rec), gout, g, out);
   else if (g.T == 16)
     hipLaunchKernelGGL((k_tile_accum<MODE, C, 16>), dim3(grid), dim3(kAccBlock), lds, stream, (const int4*)info,
@@ -1951,6 +2217,25 @@ int atl_voxel_grid_ws(const float* pos, const float* t, const float* p, const in
   if (!pos || !t || !p || !b || !vox) { set_error("voxel_grid_ws: null argument"); return 1; }
   tile_bin_accum<kVoxel, 0>(g, L, ws, pos, b, p, vox, stream, t);
   return check_launch("voxel_grid_ws");
+}
+
+int64_t atl_standardise_nonzero_ws_bytes(int64_t rows, int64_t n) {
+  if (rows < 0 || n < 0 || rows > 65535) return -1;
+  return rows * std_chunks(n) * (int64_t)sizeof(NzPart);
+}
+
+int atl_standardise_nonzero(float* x, int64_t rows, int64_t n, void* ws, int64_t ws_bytes, hipStream_t stream) {
+  const int64_t need = atl_standardise_nonzero_ws_bytes(rows, n);
+  if (need < 0) { set_error("standardise_nonzero: bad sizes rows=%lld n=%lld (at most 65535 rows)", (long long)rows, (long long)n); return 1; }
+  if (rows == 0 || n == 0) return 0;
+  if (!x || !ws || ws_bytes < need) { set_error("standardise_nonzero: null argument or a workspace of %lld bytes, need %lld", (long long)ws_bytes, (long long)need); return 1; }
+  const int nch = (int)std_chunks(n);
+  const int64_t per = ((n + nch - 1) / nch + 3) & ~(int64_t)3;   // multiples of 4: chunks start on 16 bytes
+  const int vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  const dim3 grid((unsigned)nch, (unsigned)rows);
+  hipLaunchKernelGGL(k_nz_part, grid, dim3(kBlock), 0, stream, (const float*)x, n, per, vec, (NzPart*)ws);
+  hipLaunchKernelGGL(k_nz_apply, grid, dim3(kBlock), 0, stream, x, n, per, vec, (const NzPart*)ws);
+  return check_launch("standardise_nonzero");
 }
 
 int atl_gather_bilinear_bwd_ws(const float* gval, const float* img, const float* pos, const int64_t* b, int64_t N,

@@ -107,6 +107,8 @@ _SIGS = {
     "atl_fast_pair_bwd": [_P, _P, _P, _P, _P],
     "atl_fast_plan_traj": [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _P],
     "atl_fast_pair_bwd_traj": [_P, _P, _P, _P, _I, _P, _P, _P, _P],
+    "atl_standardise_nonzero_ws_bytes": [_I, _I],
+    "atl_standardise_nonzero": [_P, _I, _I, _P, _I, _P],
     "atl_knn_ws_bytes": [_I, _I],
     "atl_lut_table_ws_bytes": [_I, _I, _I, _I, _I],
     "atl_lut_table_fwd": [_P, _I, _I, _I, _D, _D, _D, _I, _I, _I, _P, _P, _I, _P],
@@ -125,7 +127,7 @@ _SIGS = {
 }
 _RESTYPE = {"atl_scan_work_size": ctypes.c_int64, "atl_grid_plan_bytes": ctypes.c_int64,
             "atl_tile_ws_bytes": ctypes.c_int64, "atl_splat_gauss_ws_bytes": ctypes.c_int64,
-            "atl_anchored_score_mean_scratch_bytes": ctypes.c_int64, "atl_knn_ws_bytes": ctypes.c_int64, "atl_lut_table_ws_bytes": ctypes.c_int64,
+            "atl_anchored_score_mean_scratch_bytes": ctypes.c_int64, "atl_knn_ws_bytes": ctypes.c_int64, "atl_standardise_nonzero_ws_bytes": ctypes.c_int64, "atl_lut_table_ws_bytes": ctypes.c_int64,
             "atl_voxel_ws_bytes": ctypes.c_int64, "atl_warp_splat_gather_ws_bytes": ctypes.c_int64,
             "atl_ats_pair_ws_bytes": ctypes.c_int64, "atl_ats_pair_bwd_ws_bytes": ctypes.c_int64, "atl_traj_field_bwd_bytes": ctypes.c_int64,
             "atl_sample_grid_bwd_rows_bytes": ctypes.c_int64, "atl_plan_sort_bytes": ctypes.c_int64,

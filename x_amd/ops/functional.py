@@ -1269,6 +1269,14 @@ def anchored_score_mean(S, wc, vis, h, eps):
 def _standardise_nonzero(rows: torch.Tensor) -> None:
     """In place, per row: the non-zero entries minus their mean, divided by their sample standard deviation
     (n - 1 in the denominator) when it is positive; zero entries stay zero."""
+    if rows.is_cuda:
+        nbytes = load_library().atl_standardise_nonzero_ws_bytes(*rows.shape)
+        if nbytes >= 0:
+            ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=rows.device)
+            with on_device(rows.device):
+                call("atl_standardise_nonzero", ptr(rows), rows.shape[0], rows.shape[1], ptr(ws), nbytes,
+                     stream_of(rows))
+            return
     nz = rows != 0
     n = nz.sum(1, keepdim=True)
     mean = torch.where(nz, rows, 0.0).sum(1, keepdim=True) / n.clamp(min=1)
