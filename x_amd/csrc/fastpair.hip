@@ -49,8 +49,12 @@ constexpr int kMaxBuckets = 16384;
 static_assert(kMaxBuckets <= kScanSmallMax, "bucket totals are scanned by one workgroup");
 constexpr int kSortBlock = 512;                    // pass-2 workgroup
 constexpr int kP1Block = 1024;                     // pass-1 workgroup
-constexpr int kSrcPerBlock = 4096;                 // pass-1 sources per block (4 per thread)
-constexpr int kAncPerBlock = 8192;                 // pass-1 anchors per block (8 per thread)
+constexpr int kSrcPerBlock = 4096;                 // pass-1 sources per block, at most (4 per thread)
+// Sources per pass-1 block by event count, so that some 250 to 500 blocks are in flight: each pass costs a block 14 to
+// 25 us whatever the count, as its threads take their sources one after another (100k sources of 17 slices: 28 blocks
+// of 4096 ran 24 + 14 us and the entry passes 48 us, 108 blocks of 1024 run 11 + 6 us and the entry passes 21 us).  Anchors: twice as many per
+// block; entry passes: half as many.
+__host__ inline int src_per_block(int64_t N) { return N > 786432 ? kSrcPerBlock : N > 393216 ? kSrcPerBlock / 2 : kSrcPerBlock / 4; }
 constexpr int kUnroll = 8;                         // record arrays padded by the longest walk step
 constexpr int kStep = 4;                           // candidates per walk step
 constexpr int kStepLong = 8;                       // the step of a wave whose walks are long (dense neighbourhoods)
@@ -71,6 +75,8 @@ struct FGeo {
   int ncell_pad;               // ncell rounded up to whole buckets: anchor keys start here, source keys at 2x
   int MS;                      // max slices per source
   int nblk_e, nblk_a;          // pass-1 blocks over sources, over anchors
+  int spb;                     // sources per pass-1 block (2 spb anchors; spb / 2 source records per entry block)
+  int apw;                     // anchors per forward wave
   int nbuckets;                // 3 * ncell_pad >> bshift
   int bshift;                  // log2 of the keys per bucket
   float tau, half_delta, delta;
@@ -312,8 +318,8 @@ __global__ void __launch_bounds__(kP1Block) k_sort_pass1(const float2* __restric
   if (src_blk && K > 0) {
     // trajectory sources, one at a time: the 2K coefficients stay in registers across the source's slices
     constexpr int KK = K > 0 ? K : 1;
-    const int64_t j0 = (int64_t)(blk - G.nblk_a) * kSrcPerBlock;
-    for (int u = 0; u < kSrcPerBlock / kP1Block; ++u) {
+    const int64_t j0 = (int64_t)(blk - G.nblk_a) * G.spb;
+    for (int u = 0; u < G.spb / kP1Block; ++u) {
       const int64_t j = j0 + u * kP1Block + threadIdx.x;
       if (j >= N) break;
       if (!SCATTER) {
@@ -363,13 +369,14 @@ __global__ void __launch_bounds__(kP1Block) k_sort_pass1(const float2* __restric
     // the source record only: keyed by the cell of the own-slice entry, in the entries' fp32 operations.  All
     // loads first (indices clamped to the last source), so that they are in flight together.
     constexpr int per = kSrcPerBlock / kP1Block;
-    const int64_t j0 = (int64_t)(blk - G.nblk_a) * kSrcPerBlock + threadIdx.x;
+    const int64_t j0 = (int64_t)(blk - G.nblk_a) * G.spb + threadIdx.x;
+    const int64_t j1 = min((int64_t)(blk - G.nblk_a + 1) * G.spb, N);
     int64_t bs[per];
     float ts[per];
     float2 xs[per], vs[per];
 #pragma unroll
     for (int u = 0; u < per; ++u) {
-      const int64_t j = min(j0 + u * kP1Block, N - 1);
+      const int64_t j = min(j0 + u * kP1Block, j1 - 1);
       bs[u] = b[j];
       ts[u] = t[j];
       xs[u] = x[j];
@@ -379,7 +386,7 @@ __global__ void __launch_bounds__(kP1Block) k_sort_pass1(const float2* __restric
     for (int u = 0; u < per; ++u) {
       const int64_t j = j0 + u * kP1Block;
       const int64_t bj = bs[u];
-      if (j >= N || bj < 0 || bj >= G.B) continue;
+      if (j >= j1 || bj < 0 || bj >= G.B) continue;
       const float tj = ts[u];
       const float2 xj = xs[u], vj = vs[u];
       int lo, hi;
@@ -395,15 +402,16 @@ __global__ void __launch_bounds__(kP1Block) k_sort_pass1(const float2* __restric
     }
   } else if (src_blk) {
     constexpr int per = kSrcPerBlock / kP1Block;
-    const int64_t j0 = (int64_t)(blk - G.nblk_a) * kSrcPerBlock;
+    const int64_t j0 = (int64_t)(blk - G.nblk_a) * G.spb;
+    const int64_t j1 = min(j0 + G.spb, N);
     float2 xj[per], vj[per];
     float tj[per];
     int64_t bj[per];
 #pragma unroll
     for (int u = 0; u < per; ++u) {              // all loads of the thread's sources first
       const int64_t j = j0 + u * kP1Block + threadIdx.x;
-      bj[u] = j < N ? b[j] : -1;
-      if (j < N) {
+      bj[u] = j < j1 ? b[j] : -1;
+      if (j < j1) {
         tj[u] = t[j];
         xj[u] = x[j];
         vj[u] = v[j];
@@ -458,8 +466,8 @@ __global__ void __launch_bounds__(kP1Block) k_sort_pass1(const float2* __restric
       }
     }
   } else {
-    const int64_t m0 = (int64_t)blk * kAncPerBlock;
-    const int64_t m1 = m0 + kAncPerBlock < M ? m0 + kAncPerBlock : M;
+    const int64_t m0 = (int64_t)blk * (2 * G.spb);
+    const int64_t m1 = min(m0 + 2 * G.spb, M);
     constexpr int kAB = 4;                       // anchors per batch: loads, slot atomics and stores grouped
     for (int64_t mb = m0 + threadIdx.x; mb < m1; mb += kAB * blockDim.x) {
       int key[kAB], slot[kAB];
@@ -650,7 +658,7 @@ __global__ void __launch_bounds__(kSortBlock) k_sort_pass2(const int* __restrict
 // the slice-centre position is computed again from the source record by k_entry_write, in the same fp32
 // operations, after k_entry_rank has put the items in cell order.
 constexpr int kEntBlock = 512;                     // entry passes: workgroup
-constexpr int kEntSrcPerBlock = 2048;              // entry passes: source records per block (4 per thread)
+constexpr int kEntSrcPerBlock = 2048;              // entry passes: source records per block, at most (4 per thread)
 template <bool SCATTER>
 __global__ void __launch_bounds__(kEntBlock) k_entry_pass(const Rec* __restrict__ srec, const int* __restrict__ start,
                                                        FGeo G, int* __restrict__ cnt, int* __restrict__ bpos,
@@ -659,7 +667,7 @@ __global__ void __launch_bounds__(kEntBlock) k_entry_pass(const Rec* __restrict_
   const int nb0 = G.ncell_pad >> G.bshift;       // the entries' buckets
   const int EA = start[2 * G.ncell_pad];
   const int Nv = start[3 * G.ncell_pad] - EA;
-  const int q0 = blockIdx.x * kEntSrcPerBlock;
+  const int q0 = blockIdx.x * (G.spb / 2), q1 = min(q0 + G.spb / 2, Nv);
   if (q0 >= Nv) return;                          // the same blocks return in both passes
   int* __restrict__ mycnt = cnt + (int64_t)blockIdx.x * nb0;
   for (int i = threadIdx.x; i < nb0; i += blockDim.x) {
@@ -675,11 +683,11 @@ __global__ void __launch_bounds__(kEntBlock) k_entry_pass(const Rec* __restrict_
   constexpr int per = kEntSrcPerBlock / kEntBlock;
   Rec r[per];
 #pragma unroll
-  for (int u = 0; u < per; ++u) r[u] = srec[min(q0 + u * kEntBlock + (int)threadIdx.x, Nv - 1)];   // all in flight
+  for (int u = 0; u < per; ++u) r[u] = srec[min(q0 + u * kEntBlock + (int)threadIdx.x, q1 - 1)];   // all in flight
 #pragma unroll
   for (int u = 0; u < per; ++u) {
     const int q = q0 + u * kEntBlock + threadIdx.x;
-    if (q >= Nv) continue;
+    if (q >= q1) continue;
     const float tj = __int_as_float(r[u].i.x);
     const float2 xj = make_float2(r[u].f.x, r[u].f.y), vj = make_float2(r[u].f.z, r[u].f.w);
     const int bj = r[u].i.z / scells;
@@ -720,14 +728,14 @@ __global__ void __launch_bounds__(kEntBlock) k_entry_scatter(const Rec* __restri
   const int nb0 = G.ncell_pad >> G.bshift;
   const int EA = start[2 * G.ncell_pad];
   const int Nv = start[3 * G.ncell_pad] - EA;
-  const int q0 = blockIdx.x * kEntSrcPerBlock;
+  const int q0 = blockIdx.x * (G.spb / 2), q1 = min(q0 + G.spb / 2, Nv);
   if (q0 >= Nv) return;
   for (int i = threadIdx.x; i < nb0; i += blockDim.x) hist[i] = 0;
   const int scells = G.S * G.GH * G.GW;
   constexpr int per = kEntSrcPerBlock / kEntBlock;
   Rec r[per];
 #pragma unroll
-  for (int u = 0; u < per; ++u) r[u] = srec[min(q0 + u * kEntBlock + (int)threadIdx.x, Nv - 1)];
+  for (int u = 0; u < per; ++u) r[u] = srec[min(q0 + u * kEntBlock + (int)threadIdx.x, q1 - 1)];
   __syncthreads();                               // the histogram is cleared
   int key[per][MAXE], rank[per][MAXE];
 #pragma unroll
@@ -738,7 +746,7 @@ __global__ void __launch_bounds__(kEntBlock) k_entry_scatter(const Rec* __restri
     const int bj = r[u].i.z / scells;
     int lo, hi;
     slice_range(tj, G, lo, hi);
-    if (q >= Nv) hi = lo - 1;                    // no entries
+    if (q >= q1) hi = lo - 1;                    // no entries
 #pragma unroll
     for (int k = 0; k < MAXE; ++k) {
       key[u][k] = -1;
@@ -914,7 +922,7 @@ __device__ __forceinline__ bool pair_test(int id_a, int id_s, float ta, float ts
 }
 
 // ------------------------------------------------------------------------------------------ walks
-// Queries come in cell order, kAnchorsPerWave (forward) or 64 (backward) to a wave.  Forward: the anchors of up
+// Queries come in cell order, G.apw (forward) or 64 (backward) to a wave.  Forward: the anchors of up
 // to G.gcells consecutive cells of one row (about kGroupWidth px) form a group; the group's anchors are
 // wave-uniform and the lanes take 64 candidates of the group's common neighbourhood at a time (coalesced loads, each candidate read once
 // for the whole group); every anchor's sum is reduced across the wave after its last chunk.  A walk with one lane per anchor reads a different cache line in every
@@ -923,7 +931,11 @@ __device__ __forceinline__ bool pair_test(int id_a, int id_s, float ta, float ts
 
 constexpr int kPairBlock = 64;                     // workgroup of the pair walks
 constexpr int kBwdParts = 2;                       // backward lanes per source (each walks part of its slices)
-static_assert(kBwdParts == 1 || kBwdParts == 2 || kBwdParts == 4, "a source's parts are combined by a butterfly");
+// Lanes per source of the linear backward where the sources alone would leave SIMDs without waves: each lane takes
+// fewer slices.  100k sources ran 43 us with 2 lanes and 38 us with 8, 3000 sources
+// 22 and 9 us; 250k sources and more run the same or slower with 4.
+constexpr int kBwdPartsSmall = 8;
+constexpr int64_t kBwdSmall = 131072;              // sources
 constexpr int kGroup = 8;                          // queries evaluated per pass over a group's candidates
 constexpr double kGroupWidth = 9.0;                // a forward group spans cells of one row over about this many px
 
@@ -1274,8 +1286,11 @@ __device__ __forceinline__ void fwd_pass(const FPlan& p, const FGeo& G, int plan
 // every lane takes candidates in the walks).  The wave's time follows the density around its anchors, and
 // smaller units let the hardware's wave queue even out dense and sparse regions: 16 anchors per wave run the
 // C3 forward in 365 us against 410 us with 64 (32: 379 us; 8 or 12: as 16; 4: 390 us).
+// Fewer anchors leave SIMDs without a wave, and a wave then lasts as long as its 16 anchors' passes one after another:
+// 20k anchors ran 30 us with 16 and 15.6 us with 4, 3000 anchors 17 and 8 us.
 constexpr int kAnchorsPerWave = 16;
-constexpr int kAnchorsPerBlock = kPairBlock / kWave * kAnchorsPerWave;
+__host__ inline int anchors_per_wave(int64_t M) { return M > 131072 ? kAnchorsPerWave : M > 65536 ? 8 : 4; }
+static_assert(kPairBlock == kWave, "one wave per workgroup of the pair walks");
 
 // Register budgets (amdgpu_waves_per_eu: the compiler keeps the kernel within the registers of that many waves
 // per SIMD): the forward fits 8 waves without spills (53 VGPRs, 69 unconstrained), the backward 6 (80 VGPRs, three
@@ -1286,14 +1301,14 @@ constexpr int kAnchorsPerBlock = kPairBlock / kWave * kAnchorsPerWave;
 template <bool COUNT>
 __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(8))) k_fast_fwd(FPlan p, FGeo G, int M, float* __restrict__ out,
                                                      int* __restrict__ count) {
-  const int lb = xcd_block((M + kAnchorsPerBlock - 1) / kAnchorsPerBlock);
+  const int lb = xcd_block((M + G.apw - 1) / G.apw);
   if (lb < 0) return;
   const int lane = threadIdx.x & (kWave - 1);
-  const int wbase = (lb * (kPairBlock / kWave) + (int)(threadIdx.x / kWave)) * kAnchorsPerWave;
+  const int wbase = lb * G.apw;
   const int E = uni(p.start[G.ncell_pad]);
   const int Mv = uni(p.start[2 * G.ncell_pad]) - E;
   if (wbase >= Mv) return;
-  const int n = min(kAnchorsPerWave, Mv - wbase);
+  const int n = min(G.apw, Mv - wbase);
   float R, R2;
   search_radius(p.P, G, R, R2);
   R = unif(R);
@@ -1386,7 +1401,7 @@ __global__ void __launch_bounds__(kBlock) k_fast_gather_gs(FPlan p, FGeo G, int 
 // own anchor record (sp), and with an event repeated among the anchors (kLooId) the event ids are compared, as
 // the reference does.
 enum { kLooNone = 0, kLooPos = 1, kLooId = 2 };
-template <int LOO>
+template <int LOO, int PARTS>
 __device__ __forceinline__ float2 bwd_source(const FPlan& p, const FGeo& G, float R, float R2, float4 sr, int sid,
                                              float tj, int key, int sp, int part, int2* tab) {
   const int plane_cells = G.GH * G.GW;
@@ -1395,9 +1410,9 @@ __device__ __forceinline__ float2 bwd_source(const FPlan& p, const FGeo& G, floa
   const int* aid = (const int*)p.arec + 4;         // event id of record k: aid[8 * k]
   int lo_l, hi_l;
   slice_range(tj, G, lo_l, hi_l);
-  if (kBwdParts > 1) {                             // part p of kBwdParts: its share of the slices, in order
+  {                                                // part p of PARTS: its share of the slices, in order
     const int L = max(hi_l - lo_l + 1, 0);
-    const int a = lo_l + (part * L) / kBwdParts, b = lo_l + ((part + 1) * L) / kBwdParts - 1;
+    const int a = lo_l + (part * L) / PARTS, b = lo_l + ((part + 1) * L) / PARTS - 1;
     lo_l = a;
     hi_l = b;
   }
@@ -1455,11 +1470,12 @@ __device__ __forceinline__ float2 bwd_source(const FPlan& p, const FGeo& G, floa
 // Backward: every source (one lane each, own-slice tile order) sums, over the anchors of each slice of its
 // range within R of its slice-centre position, gS_i * k * dt / h^2 * r (csrc/atl_cpu.cpp:240-248);
 // gv[j] = the total (each source has one record: no atomics).
+template <int PARTS>
 __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(6))) k_fast_bwd(FPlan p, FGeo G, int N, float2* __restrict__ gv,
                                                       float2* __restrict__ gvr) {
   __shared__ int2 tab[kRowTab * kPairBlock];           // per-lane row spans of the current slice (column threadIdx.x)
-  constexpr int kSrcPerWave = kWave / kBwdParts;
-  const int lb = xcd_block((N + kPairBlock / kBwdParts - 1) / (kPairBlock / kBwdParts));
+  constexpr int kSrcPerWave = kWave / PARTS;
+  const int lb = xcd_block((N + kPairBlock / PARTS - 1) / (kPairBlock / PARTS));
   if (lb < 0) return;
   const int lane = threadIdx.x & (kWave - 1);
   const int part = lane / kSrcPerWave, ls = lane - part * kSrcPerWave;
@@ -1494,11 +1510,11 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
                                                                                                     : kLooNone;
   if (have) {
     if (loo == kLooId)
-      m = bwd_source<kLooId>(p, G, R, R2, SR.f, si.y, tj, si.z, sp, part, mytab);
+      m = bwd_source<kLooId, PARTS>(p, G, R, R2, SR.f, si.y, tj, si.z, sp, part, mytab);
     else if (loo == kLooPos)
-      m = bwd_source<kLooPos>(p, G, R, R2, SR.f, si.y, tj, si.z, sp, part, mytab);
+      m = bwd_source<kLooPos, PARTS>(p, G, R, R2, SR.f, si.y, tj, si.z, sp, part, mytab);
     else
-      m = bwd_source<kLooNone>(p, G, R, R2, SR.f, si.y, tj, si.z, sp, part, mytab);
+      m = bwd_source<kLooNone, PARTS>(p, G, R, R2, SR.f, si.y, tj, si.z, sp, part, mytab);
   }
 #pragma unroll
   for (int o = kSrcPerWave; o < kWave; o <<= 1) {  // the parts of a source sit kSrcPerWave lanes apart
@@ -1881,8 +1897,10 @@ bool make_geo(const atl_fast_geometry* geo, FGeo& G) {
   G.icf = 1.f / G.cf;
   G.GW = (int)geo->GW; G.GH = (int)geo->GH; G.S = (int)geo->S; G.B = geo->B;
   G.ncell = (int)geo->ncell; G.ncell_pad = (int)geo->ncell_pad; G.MS = (int)geo->max_span;
-  G.nblk_e = (int)((geo->N + kSrcPerBlock - 1) / kSrcPerBlock);
-  G.nblk_a = (int)((geo->M + kAncPerBlock - 1) / kAncPerBlock);
+  G.spb = src_per_block(geo->N);
+  G.nblk_e = (int)((geo->N + G.spb - 1) / G.spb);
+  G.nblk_a = (int)((geo->M + 2 * G.spb - 1) / (2 * G.spb));
+  G.apw = anchors_per_wave(geo->M);
   G.bshift = geo->bucket_shift;
   if (G.bshift < kMinBucketShift || G.bshift > kMaxBucketShift) return false;
   G.nbuckets = (int)((3 * geo->ncell_pad) >> G.bshift);
@@ -1924,6 +1942,16 @@ FPlan make_plan(void* ws, const atl_fast_geometry* geo) {
 unsigned xcd_grid(int64_t nblocks) {
   const int64_t g = kXcd * kXcdRun;
   return (unsigned)(((nblocks + g - 1) / g) * g);
+}
+
+void launch_bwd(const FPlan& p, const FGeo& G, int64_t N, float2* gv, float2* gvr, hipStream_t stream) {
+  const int parts = N > kBwdSmall ? kBwdParts : kBwdPartsSmall;
+  const int spw = kWave / parts;                   // sources per wave
+  const dim3 grid(xcd_grid((N + spw - 1) / spw));
+  if (parts == kBwdParts)
+    hipLaunchKernelGGL(k_fast_bwd<kBwdParts>, grid, dim3(kPairBlock), 0, stream, p, G, (int)N, gv, gvr);
+  else
+    hipLaunchKernelGGL(k_fast_bwd<kBwdPartsSmall>, grid, dim3(kPairBlock), 0, stream, p, G, (int)N, gv, gvr);
 }
 
 }  // namespace
@@ -1975,7 +2003,8 @@ int atl_fast_geometry_init(int64_t N, int64_t M, int64_t B, int64_t H, int64_t W
     nbuckets = 3 * ncell_pad / keys;
     if (nbuckets <= kMaxBuckets) break;
   }
-  const double nblk = std::ceil((double)N / kSrcPerBlock) + std::ceil((double)M / kAncPerBlock);
+  const int spb = src_per_block(N);
+  const double nblk = std::ceil((double)N / spb) + std::ceil((double)M / (2 * spb));
   // GW, GH < 32768: anchor records pack (cy, cx) into 16-bit halves
   if (3 * ncell_pad + 1 >= 2.0e9 || ecap + M + N >= 2.0e9 || nbuckets > kMaxBuckets || nbuckets * nblk + 1 >= 2.0e9 ||
       g.GW >= 32768 || g.GH >= 32768) {
@@ -2068,9 +2097,9 @@ int fast_plan_impl(const atl_fast_geometry* geo, const FGeo& G, const float* x, 
     const Rec* srec = at_off<Rec>(ws, geo->off_srec);
     const int* start = at_off<int>(ws, geo->off_start);
     const size_t elds = (size_t)bpk * sizeof(int);
-    // per-block counts: (N / kEntSrcPerBlock) * bpk <= nblk * nbuckets ints (kEntSrcPerBlock = kSrcPerBlock / 2)
-    static_assert(2 * kEntSrcPerBlock >= kSrcPerBlock, "the entry passes' counts fit the plan's count array");
-    const unsigned eblk = (unsigned)((N + kEntSrcPerBlock - 1) / kEntSrcPerBlock);
+    // per-block counts: ceil(2 N / spb) * bpk <= 2 nblk_e * bpk < nblk * nbuckets ints (nbuckets = 3 bpk)
+    static_assert(2 * kEntSrcPerBlock == kSrcPerBlock, "an entry block takes half a pass-1 block's sources");
+    const unsigned eblk = (unsigned)((2 * N + G.spb - 1) / G.spb);
     if (eblk > 0 && G.MS <= 12) {                // keys and ranks in registers
       auto scatter = G.MS <= 8 ? k_entry_scatter<8> : k_entry_scatter<12>;
       hipLaunchKernelGGL(scatter, dim3(eblk), dim3(kEntBlock), elds, stream, srec, start, G, bpos, item);
@@ -2135,7 +2164,7 @@ int atl_fast_pair_fwd(const atl_fast_geometry* geo, const void* ws, float* out, 
   if (!ws || (geo->M > 0 && !out)) { set_error("fast_pair_fwd: null argument"); return 1; }
   if (geo->M == 0) return 0;
   const FPlan p = make_plan((void*)ws, geo);
-  const unsigned grid = xcd_grid((geo->M + kAnchorsPerBlock - 1) / kAnchorsPerBlock);
+  const unsigned grid = xcd_grid((geo->M + G.apw - 1) / G.apw);
   if (count)
     hipLaunchKernelGGL(k_fast_fwd<true>, dim3(grid), dim3(kPairBlock), 0, stream, p, G, (int)geo->M, out, count);
   else
@@ -2152,8 +2181,7 @@ int atl_fast_pair_bwd(const atl_fast_geometry* geo, void* ws, const float* gS, f
   hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
                      (int)geo->M, gS, (int)geo->N, (float2*)gv);
   if (geo->M > 0)
-    hipLaunchKernelGGL(k_fast_bwd, dim3(xcd_grid((geo->N + kPairBlock / kBwdParts - 1) / (kPairBlock / kBwdParts))),
-                       dim3(kPairBlock), 0, stream, p, G, (int)geo->N, (float2*)gv, (float2*)nullptr);
+    launch_bwd(p, G, geo->N, (float2*)gv, nullptr, stream);
   return check_launch("fast_pair_bwd");
 }
 
@@ -2169,8 +2197,7 @@ int atl_fast_pair_bwd_src(const atl_fast_geometry* geo, void* ws, const float* g
   float2* gvr = at_off<float2>(ws, geo->off_trec);
   hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
                      (int)geo->M, gS, (int)geo->N, (float2*)nullptr);
-  hipLaunchKernelGGL(k_fast_bwd, dim3(xcd_grid((geo->N + kPairBlock / kBwdParts - 1) / (kPairBlock / kBwdParts))),
-                     dim3(kPairBlock), 0, stream, p, G, (int)geo->N, (float2*)nullptr, gvr);
+  launch_bwd(p, G, geo->N, nullptr, gvr, stream);
   return check_launch("fast_pair_bwd_src");
 }
 

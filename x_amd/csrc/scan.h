@@ -114,8 +114,44 @@ __global__ void __launch_bounds__(kBlock) k_scan32t_write(const int* __restrict_
   if (blockIdx.x == 0 && threadIdx.x == 0) out[0] = 0;
 }
 
+constexpr int kScanSmallBlock = 1024;
+constexpr int kScanSmallMax = 16384;
+
+// The transposed scan of up to kScanSmallMax counts (some tens of thousands of events) in one workgroup and one launch:
+// 5 us against 2.7 + 4.1 us and a launch more for the two passes (100k events, 300 tiles: 7500 counts).
+__global__ void __launch_bounds__(kScanSmallBlock) k_scan32t_small(const int* __restrict__ in, int nkeys, int nblk,
+                                                                   int* __restrict__ out) {
+  __shared__ int wsum[kScanSmallBlock / kWave + 1];
+  constexpr int kPer = kScanSmallMax / kScanSmallBlock;
+  const int n = nkeys * nblk, i0 = threadIdx.x * kPer;
+  int key = i0 / nblk, blk = i0 - key * nblk;
+  int v[kPer];
+  int s = 0;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    v[k] = i0 + k < n ? in[blk * nkeys + key] : 0;
+    s += v[k];
+    if (++blk == nblk) {
+      blk = 0;
+      ++key;
+    }
+  }
+  int total;
+  int run = block_exclusive_scan<kScanSmallBlock>(s, wsum, total);
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    if (i0 + k < n) out[i0 + k] = run;
+    run += v[k];
+  }
+  if (threadIdx.x == 0) out[n] = total;
+}
+
 inline void scan32t(const int* in, int nkeys, int nblk, int* part, int* out, hipStream_t stream) {
   const int64_t n = (int64_t)nkeys * nblk;
+  if (n <= kScanSmallMax) {
+    hipLaunchKernelGGL(k_scan32t_small, dim3(1), dim3(kScanSmallBlock), 0, stream, in, nkeys, nblk, out);
+    return;
+  }
   const int64_t tiles = scan_tiles(n);
   hipLaunchKernelGGL(k_scan32t_reduce, dim3((unsigned)tiles), dim3(kBlock), 0, stream, in, nkeys, nblk, n, part);
   hipLaunchKernelGGL(k_scan32t_write, dim3((unsigned)tiles), dim3(kBlock), 0, stream, in, nkeys, nblk, n,
@@ -124,8 +160,6 @@ inline void scan32t(const int* in, int nkeys, int nblk, int* part, int* out, hip
 
 // Exclusive scan of n <= kScanSmallMax counts (bucket or tile totals) into their start positions: one
 // workgroup, one launch.
-constexpr int kScanSmallBlock = 1024;
-constexpr int kScanSmallMax = 16384;
 
 __global__ void __launch_bounds__(kScanSmallBlock) k_scan_small(const int* __restrict__ tot, int n,
                                                                 int* __restrict__ pos) {
