@@ -68,8 +68,8 @@ HBM_PEAK = 8.0e12                      # bytes/s
 # compulsory HBM bytes per event of the anchored step: positions 8, dequantisation 8, smoothing 8, time 4,
 # batch 8 (the flow grid and its gradient are added per call); with the splat leg: + 20 forward + 32 backward
 STEP_BYTES_PER_EVENT, SPLAT_BYTES_PER_EVENT = 36, 52
-KERNEL_OF = {"atl_fast_pair_fwd": "k_fast_fwd<false>", "atl_fast_pair_bwd": "k_fast_bwd", "atl_fast_pair_bwd_src": "k_fast_bwd",
-             "atl_fast_pair_bwd_traj": "k_fast_bwd_traj<10>"}
+KERNEL_OF = {"atl_fast_pair_fwd": "k_fast_fwd<false>", "atl_fast_pair_bwd": "k_entry_bwd<false>", "atl_fast_pair_bwd_src": "k_entry_bwd<false>",
+             "atl_fast_pair_bwd_traj": "k_entry_bwd<true>"}
 COUNTERS = ROOT / "profiles" / "anchored_score_1M_640x480_counters.md"
 
 

@@ -1,7 +1,7 @@
 // Fused anchored pair sums on gfx950: the reference's (source, slice) entries and the anchors binned into
 // one fixed, clamped fine-cell grid per slice, then a gather-form forward (the anchors of one cell share a
-// wave, whose lanes take the candidate entries of their neighbourhood) and a source-centric backward (one
-// lane per source, walking the anchors around all of its slices), both over disc-pruned rows of fine cells.
+// wave, whose lanes take the candidate entries of their neighbourhood) and an entry-centric backward (one
+// lane per entry, over the anchors around it), both over disc-pruned rows of fine cells.
 //
 // What is kept identical to the reference (csrc/atl_cpu.cpp:176-253, atl/ops/functional.py:150-177):
 //   * the slice range of every source and its slice-centre position y = x + v (c_s - t), op for op in fp32;
@@ -24,9 +24,8 @@
 // records.  Entries and anchors
 // share one key space (anchor keys offset by the padded cell count), so both sorts run in the same
 // launches.  The same sort also orders the sources by the cell of their own-slice position (in tiles of
-// 8 x 8 cells, so that a wave's sources form a compact patch), and the
-// backward gives each source one lane that walks the anchors of all its slices: the gradient of a source
-// is complete in registers and written once, without atomics.
+// 8 x 8 cells, so that 64 of them form a compact patch).  The backward gives every entry a lane that sums over the
+// anchors of its own slice, and a source adds up its entries' sums in slice order: no atomics.
 #include <algorithm>
 #include <type_traits>
 
@@ -55,10 +54,8 @@ constexpr int kSrcPerBlock = 4096;                 // pass-1 sources per block, 
 // of 4096 ran 24 + 14 us and the entry passes 48 us, 108 blocks of 1024 run 11 + 6 us and the entry passes 21 us).  Anchors: twice as many per
 // block; entry passes: half as many.
 __host__ inline int src_per_block(int64_t N) { return N > 786432 ? kSrcPerBlock : N > 393216 ? kSrcPerBlock / 2 : kSrcPerBlock / 4; }
-constexpr int kUnroll = 8;                         // record arrays padded by the longest walk step
+constexpr int kUnroll = 8;                         // record arrays padded by at least a walk step
 constexpr int kStep = 4;                           // candidates per walk step
-constexpr int kStepLong = 8;                       // the step of a wave whose walks are long (dense neighbourhoods)
-constexpr int kLongWalk = 256;                     // a lane's slice candidates above which its wave steps long
 constexpr int kSliceBatch = 4;                     // pass 1: slices of one source keyed and placed together
 
 constexpr int kXcd = 8;                            // XCDs: consecutive workgroups go round-robin over them
@@ -95,11 +92,9 @@ constexpr int kMaxPlanes = 1024;
 struct FParams {
   int vmax;                    // max ||v|| over sources
   int atmax;                   // max |t_a - c_s| over anchors
-  int dup;                     // non-zero if an event occurs more than once among the anchors
-  int unique;                  // non-zero if the anchors are every event in order (no index array): no repeats
   int nonfinite;               // non-zero if a backward record (anchor position, time or gS) is not finite
   int planes;                  // non-zero if the per-plane maxima below were written (trajectory plans)
-  int pad[2];
+  int pad[4];
 };                             // followed by B * S ints (ordered): each plane's max ||v|| when `planes`
 
 __device__ __forceinline__ int* plane_vmax(const FParams* P) { return (int*)(P + 1) ; }
@@ -287,7 +282,7 @@ __global__ void __launch_bounds__(kP1Block) k_sort_pass1(const float2* __restric
                                                        const float2* __restrict__ anchor_xy, int64_t M, FGeo G,
                                                        int* __restrict__ cnt, int* __restrict__ bsum,
                                                        Rec* __restrict__ trec, FParams* __restrict__ P,
-                                                       int* __restrict__ self, int* __restrict__ eself,
+                                                       int* __restrict__ spos, int* __restrict__ eself,
                                                        const float* __restrict__ coef,
                                                        const float* __restrict__ tab) {
   extern __shared__ int hist[];
@@ -310,7 +305,6 @@ __global__ void __launch_bounds__(kP1Block) k_sort_pass1(const float2* __restric
     }
     hist[i] = h;
   }
-  if (!SCATTER && blk == 0 && threadIdx.x == 0 && !anchors) P->unique = 1;
   __syncthreads();
   // anchor blocks first: they are about a quarter of a source block's work, and dispatched last they would
   // queue on the few CUs left free by the source blocks
@@ -323,7 +317,7 @@ __global__ void __launch_bounds__(kP1Block) k_sort_pass1(const float2* __restric
       const int64_t j = j0 + u * kP1Block + threadIdx.x;
       if (j >= N) break;
       if (!SCATTER) {
-        self[j] = -1;
+        spos[j] = -1;
         eself[j] = -1;
       }
       const int64_t bj = b[j];
@@ -415,10 +409,7 @@ __global__ void __launch_bounds__(kP1Block) k_sort_pass1(const float2* __restric
         tj[u] = t[j];
         xj[u] = x[j];
         vj[u] = v[j];
-        if (!SCATTER) {                            // "no anchor record" / "no own-slice entry" until pass 2
-          self[j] = -1;
-          eself[j] = -1;
-        }
+        if (!SCATTER) eself[j] = -1;               // "no own-slice entry" until the entries are written
       }
     }
 #pragma unroll
@@ -521,11 +512,11 @@ constexpr int kSortItems = 8;
 struct SortOut {
   int* start;
   float4* epos;                // entries: (y.x, y.y, v.x, v.y)
-  float* etim;                 // entries: t
+  float2* etq;                 // entries: t, and the source record (linear model) or event id (trajectories) as bits
   int* eself;                  // per event: its entry in slice floor(t / delta), -1 if none
   Rec* arec;                   // anchors
   Rec* srec;                   // sources
-  int* self;                   // per event: its anchor record, -1 if none
+  int* spos;                   // trajectories, per event: its source record, -1 if none
 };
 
 __device__ __forceinline__ int anchor_slice(float t, const FGeo& G) {
@@ -622,11 +613,11 @@ __global__ void __launch_bounds__(kSortBlock) k_sort_pass2(const int* __restrict
     if (space == 0) {
       o.epos[pos] = r.f;
       const float tj = __int_as_float(r.i.x);
-      o.etim[pos] = tj;
+      o.etq[pos] = make_float2(tj, __int_as_float(r.i.y));   // one store: a scattered line costs what it holds
       if ((r.i.z / plane_cells) % G.S == anchor_slice(tj, G)) o.eself[r.i.y] = pos;
     } else {
       out[pos] = r;
-      if (space == 1) o.self[r.i.x] = pos;       // the anchor's event id -> its record
+      if (space == 2 && o.spos) o.spos[r.i.y] = pos;
     }
   };
   if (one) {
@@ -889,7 +880,7 @@ __global__ void __launch_bounds__(kBlock) k_entry_write(const int2* __restrict__
     const int sl = (it[u].y / plane_cells) % G.S;
     const float dt = slice_centre(sl, G.delta) - tj;
     o.epos[pos] = make_float4(r[u].f.x + r[u].f.z * dt, r[u].f.y + r[u].f.w * dt, r[u].f.z, r[u].f.w);
-    o.etim[pos] = tj;
+    o.etq[pos] = make_float2(tj, __int_as_float(it[u].x));
     if (sl == anchor_slice(tj, G)) o.eself[r[u].i.y] = pos;
   }
 }
@@ -897,12 +888,13 @@ __global__ void __launch_bounds__(kBlock) k_entry_write(const int2* __restrict__
 // ------------------------------------------------------------------------------------------ pair walks
 struct FPlan {
   const float4* epos;          // entries in cell order: (y.x, y.y, v.x, v.y)
-  const float* etim;           // entries in cell order: t
+  const float2* etq;           // entries in cell order: SortOut::etq
   const int* eself;            // per event: position of its own-slice entry, -1 if none
   const Rec* arec;             // anchors in cell order
   const Rec* srec;             // sources in own-slice cell order, tile by tile (source_key)
   float4* brec;                // anchors in cell order for the backward: (x, y, t, gS / h^2)
-  int* self;                   // per event: position of its own anchor record, -1 if it is no anchor
+  int* bes;                    // anchors in cell order: position of the event's own entry in the slice, -1 if none
+  const int* spos;             // trajectories: SortOut::spos
   const int* start;            // 3*ncell_pad + 1: entry cells, anchor cells (offset by E), source cells
   FParams* P;
 };
@@ -922,20 +914,13 @@ __device__ __forceinline__ bool pair_test(int id_a, int id_s, float ta, float ts
 }
 
 // ------------------------------------------------------------------------------------------ walks
-// Queries come in cell order, G.apw (forward) or 64 (backward) to a wave.  Forward: the anchors of up
-// to G.gcells consecutive cells of one row (about kGroupWidth px) form a group; the group's anchors are
-// wave-uniform and the lanes take 64 candidates of the group's common neighbourhood at a time (coalesced loads, each candidate read once
-// for the whole group); every anchor's sum is reduced across the wave after its last chunk.  A walk with one lane per anchor reads a different cache line in every
-// lane, and that is what bounds it.  Backward: one lane per source walks its own neighbourhoods (sources'
-// per-slice positions differ, so a group shares less there than it costs to set up).
+// Forward: anchors in cell order, G.apw to a wave.  The anchors of up to G.gcells consecutive cells of one row (about
+// kGroupWidth px) form a group; the group's anchors are wave-uniform and the lanes take 64 candidates of the group's
+// common neighbourhood at a time (coalesced loads, each candidate read once for the whole group); every anchor's sum
+// is reduced across the wave after its last chunk.  Anchors that stand close together are taken all at once
+// (fwd_common).  Backward: entries in cell order, 64 to a wave (entry_sum).
 
 constexpr int kPairBlock = 64;                     // workgroup of the pair walks
-constexpr int kBwdParts = 2;                       // backward lanes per source (each walks part of its slices)
-// Lanes per source of the linear backward where the sources alone would leave SIMDs without waves: each lane takes
-// fewer slices.  100k sources ran 43 us with 2 lanes and 38 us with 8, 3000 sources
-// 22 and 9 us; 250k sources and more run the same or slower with 4.
-constexpr int kBwdPartsSmall = 8;
-constexpr int64_t kBwdSmall = 131072;              // sources
 constexpr int kGroup = 8;                          // queries evaluated per pass over a group's candidates
 constexpr double kGroupWidth = 9.0;                // a forward group spans cells of one row over about this many px
 
@@ -1054,9 +1039,7 @@ __device__ __forceinline__ void walk(const int* __restrict__ cstart, int base, i
 // in lockstep leaves most lanes idle).  Taller neighbourhoods take the row-by-row walk.
 constexpr int kRowTab = 8;
 
-// ADAPT: a wave in which some lane's neighbourhood holds more than kLongWalk candidates takes steps of kStepLong
-// (more loads in flight per lane on long walks; short walks keep kStep, which leaves fewer lanes masked).
-template <bool ADAPT = false, typename Visit>
+template <typename Visit>
 __device__ __forceinline__ void walk_flat(const int* __restrict__ cstart, int base, int plane, float qx, float qy,
                                           float R, float R2, const FGeo& G, int2* tab, Visit&& visit) {
   const int rlo = cell_walk(qy - R, G.gy0, G.gy1, G.icf, G.GH), rhi = cell_walk(qy + R, G.gy0, G.gy1, G.icf, G.GH);
@@ -1079,35 +1062,21 @@ __device__ __forceinline__ void walk_flat(const int* __restrict__ cstart, int ba
   }
 #pragma unroll
   for (int i = 0; i < kRowTab; ++i) tab[i * kPairBlock] = make_int2(kk[i] - base, ee[i] - base);
-  auto steps = [&](auto step) {
-    constexpr int U = decltype(step)::value;
-    int ri = 0;                                    // row of cur; nxt holds row ri + 1 (read one row ahead)
-    int2 cur = make_int2(kk[0] - base, ee[0] - base);
-    int2 nxt = make_int2(kk[1] - base, ee[1] - base);
-    while (true) {
-      if (cur.x >= cur.y) {
-        do {
-          cur = nxt;
-          ++ri;
-          nxt = ri + 1 < nrows ? tab[(ri + 1) * kPairBlock] : make_int2(0, 0);
-        } while (cur.x >= cur.y && ri < nrows - 1);
-        if (cur.x >= cur.y) break;
-      }
-      visit(cur.x, cur.y, step);
-      cur.x += U;
+  int ri = 0;                                      // row of cur; nxt holds row ri + 1 (read one row ahead)
+  int2 cur = make_int2(kk[0] - base, ee[0] - base);
+  int2 nxt = make_int2(kk[1] - base, ee[1] - base);
+  while (true) {
+    if (cur.x >= cur.y) {
+      do {
+        cur = nxt;
+        ++ri;
+        nxt = ri + 1 < nrows ? tab[(ri + 1) * kPairBlock] : make_int2(0, 0);
+      } while (cur.x >= cur.y && ri < nrows - 1);
+      if (cur.x >= cur.y) break;
     }
-  };
-  bool lng = false;
-  if (ADAPT) {
-    int tot = 0;
-#pragma unroll
-    for (int i = 0; i < kRowTab; ++i) tot += ee[i] - kk[i];
-    lng = __any(tot > kLongWalk);                  // uniform over the wave's walking lanes
+    visit(cur.x, cur.y, Step<kStep>{});
+    cur.x += kStep;
   }
-  if (lng)
-    steps(Step<kStepLong>{});
-  else
-    steps(Step<kStep>{});
 }
 
 // Group walk: the candidates of the cells of plane `plane` that meet the R-neighbourhood of the box
@@ -1239,7 +1208,7 @@ __device__ __forceinline__ void fwd_pass(const FPlan& p, const FGeo& G, int plan
   };
   auto load = [&](int pos) {
     const uint32_t k = (uint32_t)max(pos, 0);
-    return Cand{ld(p.epos, k), ld(p.etim, k)};
+    return Cand{ld(p.epos, k), ld((const float*)p.etq, 2 * k)};
   };
   // The walk covers the R-neighbourhood of the box of these anchors' clamped positions (tighter than their
   // cells' box: every contributing candidate lies within R of its anchor, and clamping never increases a
@@ -1279,9 +1248,26 @@ __device__ __forceinline__ void fwd_pass(const FPlan& p, const FGeo& G, int plan
   }
 }
 
-// Forward: out[m] = S_m and, with COUNT, count[m] = n_m (number of pairs passing the tests).  Every lane
-// sums one candidate per chunk, the 64 lane partials are added in a tree (the reference's CPU path sums
-// sequentially in fp64; both stay well inside 1e-5 of the exact sum).
+// Minimum and maximum over the 64 lanes, wave-uniform.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dppk(float v) {   // rows outside ROWS keep their own value
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, ROWS, 0xF, false));
+}
+template <bool MAX>
+__device__ __forceinline__ float wave_ext(float v) {
+  auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : fminf(a, b); };
+  v = op(v, dppk<0xB1, 0xF>(v));
+  v = op(v, dppk<0x4E, 0xF>(v));
+  v = op(v, dppk<0x141, 0xF>(v));
+  v = op(v, dppk<0x140, 0xF>(v));
+  v = op(v, dppk<0x142, 0xA>(v));
+  v = op(v, dppk<0x143, 0xC>(v));
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// Finite and small enough that products of two such values stay finite.
+__device__ __forceinline__ bool bounded(float v) { return fabsf(v) < 1e30f; }
+
 // A wave takes kAnchorsPerWave consecutive anchors (lanes past them hold copies and idle through the group loop;
 // every lane takes candidates in the walks).  The wave's time follows the density around its anchors, and
 // smaller units let the hardware's wave queue even out dense and sparse regions: 16 anchors per wave run the
@@ -1290,7 +1276,91 @@ __device__ __forceinline__ void fwd_pass(const FPlan& p, const FGeo& G, int plan
 // 20k anchors ran 30 us with 16 and 15.6 us with 4, 3000 anchors 17 and 8 us.
 constexpr int kAnchorsPerWave = 16;
 __host__ inline int anchors_per_wave(int64_t M) { return M > 131072 ? kAnchorsPerWave : M > 65536 ? 8 : 4; }
-static_assert(kPairBlock == kWave, "one wave per workgroup of the pair walks");
+static_assert(kPairBlock == kWave && kWave % kAnchorsPerWave == 0, "one wave per workgroup, whole waves per 64 anchors");
+
+// Forward of kAnchorsPerWave anchors that stand close together, each in kFwdParts lanes: their common neighbourhood is
+// read once for the wave, 64 candidates at a time; the candidates that can lie within cut h of some anchor at its own
+// time are put into LDS, and an anchor's lanes evaluate every kFwdParts-th of them, the 16 lanes of a part reading one
+// address.  The passes of up to eight wave-uniform
+// anchors evaluate all candidates of their box's cells, 3.5 per contributing pair in a crowd; here it is half of that:
+// 4M events in blobs 46 -> 31 ms.  All 64 lanes with an anchor each took 100 ms: a wave then lasts four times as long
+// and the densest end last.  On the edges of 1M events neither wins; kCommonFwd = 4, 8 and 14 run 1085, 1082 and 1074
+// us a step, with h = 2 406, 405 and 413.
+// [x0, x1] x [y0, y1]: the box of the anchors.
+constexpr int kFwdParts = kWave / kAnchorsPerWave;
+constexpr float kCommonFwd = 8.f;
+constexpr int kFwdSlots = kWave + 4 * kFwdParts;   // candidates of a chunk, padded to four of every part
+template <bool COUNT>
+__device__ __forceinline__ void fwd_common(const FPlan& p, const FGeo& G, int plane, float R, float R2, float vmax,
+                                           const float4& A, int es, float x0, float x1, float y0, float y1, char* lds,
+                                           float& mine, int& mine_n) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const float a0 = wave_ext<false>(A.w), a1 = wave_ext<true>(A.w);
+  const float rg = G.cuth * 1.000001f + vmax * fmaxf(fabsf(a0), fabsf(a1)) * 1.000001f + 0.01f;
+  if (rg < R) {
+    R = unif(rg);
+    R2 = R * R;
+  }
+  const float cr = G.cuth * 1.000001f + 0.01f, cr2 = cr * cr;     // 0.01 px: fp32 rounding of positions, as in R
+  float4* sE = (float4*)lds;                       // the candidates: (y, v), t, position
+  float* sT = (float*)(sE + kFwdSlots);
+  int* sI = (int*)(sT + kFwdSlots);
+  const int part = lane / kAnchorsPerWave;
+  struct Cand {
+    float4 e;
+    float t;
+  };
+  auto load = [&](int k) {
+    const uint32_t i = (uint32_t)max(k, 0);
+    return Cand{ld(p.epos, i), ld((const float*)p.etq, 2 * i)};
+  };
+  float acc = 0.f;
+  int cnt = 0;
+  group_walk(p.start, 0, plane, x0, x1, y0, y1, R, R2, G, load, [&](const Cand& c, int k) {
+    // the candidate's positions at the anchors' times; a NaN compares to "keep", as the pair tests would visit it
+    const float px0 = c.e.z * a0, px1 = c.e.z * a1, py0 = c.e.w * a0, py1 = c.e.w * a1;
+    const float ex = fmaxf(fmaxf(x0 - (c.e.x + fmaxf(px0, px1)), (c.e.x + fminf(px0, px1)) - x1), 0.f);
+    const float ey = fmaxf(fmaxf(y0 - (c.e.y + fmaxf(py0, py1)), (c.e.y + fminf(py0, py1)) - y1), 0.f);
+    const bool keep = (k >= 0) & !(ex * ex + ey * ey > cr2);
+    const uint64_t m = __ballot(keep);
+    const int n = __popcll(m);
+    __syncthreads();                               // one wave: the last chunk's reads are done
+    if (keep) {
+      const int i = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+      sE[i] = c.e;
+      sT[i] = c.t;
+      sI[i] = k;
+    }
+    if (lane < 4 * kFwdParts) {                    // padding that no anchor counts: infinitely late
+      sE[n + lane] = make_float4(x0, y0, 0.f, 0.f);
+      sT[n + lane] = INFINITY;
+      sI[n + lane] = -2;
+    }
+    __syncthreads();
+    for (int i = part; i < n + part; i += 4 * kFwdParts) {   // as many rounds in every part
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = i + u * kFwdParts;
+        float dt, rx, ry, d2;
+        const bool ok = pair_test(es, sI[c], A.z, sT[c], A.x, A.y, A.w, sE[c], G, dt, rx, ry, d2);
+        const float kern = __builtin_amdgcn_exp2f(d2 * G.kexp);
+        acc += ok ? kern : 0.f;
+        if (COUNT) cnt += ok ? 1 : 0;
+      }
+    }
+  });
+#pragma unroll
+  for (int d = kAnchorsPerWave; d < kWave; d <<= 1) {
+    acc += __shfl_xor(acc, d, kWave);
+    if (COUNT) cnt += __shfl_xor(cnt, d, kWave);
+  }
+  mine = acc;
+  mine_n = cnt;
+}
+
+// Forward: out[m] = S_m and, with COUNT, count[m] = n_m (number of pairs passing the tests).  Every lane
+// sums one candidate per chunk, the 64 lane partials are added in a tree (the reference's CPU path sums
+// sequentially in fp64; both stay well inside 1e-5 of the exact sum).
 
 // Register budgets (amdgpu_waves_per_eu: the compiler keeps the kernel within the registers of that many waves
 // per SIMD): the forward fits 8 waves without spills (53 VGPRs, 69 unconstrained), the backward 6 (80 VGPRs, three
@@ -1301,6 +1371,7 @@ static_assert(kPairBlock == kWave, "one wave per workgroup of the pair walks");
 template <bool COUNT>
 __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(8))) k_fast_fwd(FPlan p, FGeo G, int M, float* __restrict__ out,
                                                      int* __restrict__ count) {
+  __shared__ __align__(16) char lds[kFwdSlots * (sizeof(float4) + sizeof(float) + sizeof(int))];
   const int lb = xcd_block((M + G.apw - 1) / G.apw);
   if (lb < 0) return;
   const int lane = threadIdx.x & (kWave - 1);
@@ -1308,7 +1379,6 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
   const int E = uni(p.start[G.ncell_pad]);
   const int Mv = uni(p.start[2 * G.ncell_pad]) - E;
   if (wbase >= Mv) return;
-  const int n = min(G.apw, Mv - wbase);
   float R, R2;
   search_radius(p.P, G, R, R2);
   R = unif(R);
@@ -1316,13 +1386,36 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
   const float vmax = unif(ordered_to_float(p.P->vmax));
   const int* vpl = plane_vmax(p.P);
   const bool planes = G.vplanes && uni(p.P->planes) != 0;
+  const int n = min(G.apw, Mv - wbase);
   const bool have = lane < n;
-  const int q = wbase + min(lane, n - 1);
+  const int q = wbase + min(lane & (kAnchorsPerWave - 1), n - 1);
   const Rec AR = p.arec[q];
   const float4 A = AR.f;
   const int4 ai = AR.i;
   const int key = ai.z;
   const int es = p.eself[ai.x];                  // the anchor event's own entry in this slice, -1 if none
+  if (n == kAnchorsPerWave) {                    // anchors close together, in one plane: all of them at once
+    const int cell = (ai.w >> 16) * G.GW + (ai.w & 0xffff);
+    const int plane = uni(key - cell);
+    const bool plain = key - cell == plane && bounded(A.x) && bounded(A.y) && clampf(A.x, G.gx0, G.gx1) == A.x &&
+                       clampf(A.y, G.gy0, G.gy1) == A.y;
+    if (__ballot(!plain) == 0) {
+      const float x0 = wave_ext<false>(A.x), x1 = wave_ext<true>(A.x);
+      const float y0 = wave_ext<false>(A.y), y1 = wave_ext<true>(A.y);
+      const float bw = x1 - x0, bh = y1 - y0;
+      if (bw * bh + 2.f * G.cuth * (bw + bh) <= kCommonFwd * G.cuth * G.cuth) {
+        const float vg = planes ? fminf(vmax, ordered_to_float(vpl[plane / (G.GH * G.GW)])) : vmax;
+        float mine;
+        int mine_n;
+        fwd_common<COUNT>(p, G, plane, R, R2, vg, A, es, x0, x1, y0, y1, lds, mine, mine_n);
+        if (have) {
+          out[ai.y] = mine;
+          if (COUNT) count[ai.y] = mine_n;
+        }
+        return;
+      }
+    }
+  }
   const int plane_cells = G.GH * G.GW;
   float mine = 0.f;
   int mine_n = 0;
@@ -1362,9 +1455,6 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
   }
 }
 
-// Finite and small enough that products of two such values stay finite.
-__device__ __forceinline__ bool bounded(float v) { return fabsf(v) < 1e30f; }
-
 // Record range of slice s of (batch b, tile (tb, tx)) in the source records.
 __device__ __forceinline__ int2 src_tile_range(const FPlan& p, const FGeo& G, int b, int s, int tb, int tx, int EA) {
   const int T = G.stile;
@@ -1374,15 +1464,17 @@ __device__ __forceinline__ int2 src_tile_range(const FPlan& p, const FGeo& G, in
   return make_int2(sstart[k0] - EA, sstart[k0 + hb * wt] - EA);
 }
 
-// Backward records of the anchors in cell order, brec[q] = (x, y, t, gS / h^2): one 16-byte load per candidate in
-// the backward's per-lane walks (the anchor's at = t - c_s is recomputed there with the same fp32 operation).
-// Also checks that no event occurs twice among the anchors (self[id] then names only one of the records); an
-// index-free plan (every event once) skips that check.  Threads q < N clear gv[q] for the backward, which then
-// writes each source's total (sources without a record keep the zero).
+// Backward records of the anchors in cell order, brec[q] = (x, y, t, gS / h^2): one 16-byte load per candidate (the
+// anchor's at = t - c_s is recomputed with the same fp32 operation); bes[q]: the event's own entry in the slice, which
+// the leave-one-out test skips.  Threads q < N clear gv[q] and, with gcoef, the rows of C coefficients of events without
+// a source record: the backward writes every source's total, and only what it does not write has to be cleared.
 __global__ void __launch_bounds__(kBlock) k_fast_gather_gs(FPlan p, FGeo G, int M, const float* __restrict__ gS,
-                                                           int N, float2* __restrict__ gv) {
+                                                           int N, float2* __restrict__ gv,
+                                                           float* __restrict__ gcoef, int C) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (gv && q < N) gv[q] = make_float2(0.f, 0.f);
+  if (gcoef && q < N && (M == 0 || p.spos[q] < 0))
+    for (int c = 0; c < C; ++c) gcoef[(int64_t)q * C + c] = 0.f;
   const int Mv = p.start[2 * G.ncell_pad] - p.start[G.ncell_pad];
   // the walks' padding past the last record (Mv <= M: inside the M + kUnroll records): zeros
   if (q < kUnroll) p.brec[Mv + q] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1390,140 +1482,259 @@ __global__ void __launch_bounds__(kBlock) k_fast_gather_gs(FPlan p, FGeo G, int 
   const Rec r = p.arec[q];
   const float4 br = make_float4(r.f.x, r.f.y, r.f.z, gS[r.i.y] * G.invh2);
   p.brec[q] = br;
-  if (!p.P->unique && p.self[r.i.x] != q) p.P->dup = 1;
+  p.bes[q] = p.eself[r.i.x];
   if (!(bounded(br.x) && bounded(br.y) && bounded(br.z) && bounded(br.w))) p.P->nonfinite = 1;
 }
 
-// One source's walk over the anchors of every slice of its range (csrc/atl_cpu.cpp:240-248): returns
-// sum_i gS_i * k * dt / h^2 * r.  Leave-one-out (LOO): the pair of an event with its own anchor record has
-// dt = t_j - t_j = 0, so with finite records and source data its term is exactly zero and the test is skipped
-// (kLooNone); otherwise (kLooPos) the candidate's record position is compared with the position of the source's
-// own anchor record (sp), and with an event repeated among the anchors (kLooId) the event ids are compared, as
-// the reference does.
-enum { kLooNone = 0, kLooPos = 1, kLooId = 2 };
-template <int LOO, int PARTS>
-__device__ __forceinline__ float2 bwd_source(const FPlan& p, const FGeo& G, float R, float R2, float4 sr, int sid,
-                                             float tj, int key, int sp, int part, int2* tab) {
-  const int plane_cells = G.GH * G.GW;
+// Backward over the entries.  A wave takes 64 consecutive entries (cell order), in which each lane's entry sums the
+// terms of the anchors of its own slice: the linear model gS_i k dt / h^2 r, trajectories gS_i k r / h^2 and that
+// times at (csrc/atl_cpu.cpp:240-248).  The sums go to the slot (slice of the source's range, source record), which
+// only this entry writes, and k_slot_* adds a source's slots in slice order: no atomics.
+//
+// Two ways through the anchors.  Where the 64 entries stand close together (kCommon), their common neighbourhood is
+// read once for the wave, 64 anchors at a time; the anchors that can lie within cut h of some entry at their own time
+// (the entries' boxes of positions and velocities) are put into LDS, and every lane evaluates each of them, read at a
+// wave-uniform address.  Elsewhere every lane walks the cells around its own entry.  The lanes read one
+// address then, where each lane's own walk reads its own: dense crowds ran 75 ms with a lane per source walking all its
+// slices (4M events, 90% in five blobs of sigma 8 px) and run 24 ms; 1M events on 640 x 480 438 -> 339 us and 17 us
+// for the sums of the slots, trajectories of 4 x 500k events 1774 -> 1272 + 245 us.  kCommon, the box up to which the
+// common way is taken in units of (cut h)^2: 1126, 1087, 1077 and 1081 us a step at 4, 8, 20 and 40 on the 1M events,
+// where the entries of edges stand 10 to a square pixel, and 401, 405, 406 and 411 us with the wide kernel of h = 2.
+//
+// Leave-one-out: an anchor's own entry is skipped by position (bes).  The linear model's own pair has dt = 0, so its
+// term is exactly zero when every number is finite, and the test is dropped there (LOO false).
+constexpr float kCommon = 16.f;
+
+template <bool TRAJ>
+using EntSum = std::conditional_t<TRAJ, float4, float2>;
+
+template <bool TRAJ, bool LOO>
+__device__ __forceinline__ EntSum<TRAJ> entry_sum(const FPlan& p, const FGeo& G, float R, float R2, float atmax,
+                                                  const float4& sv, float tj, int pos, int pl, int sl, bool active,
+                                                  bool finite, char* lds) {
+  const int lane = threadIdx.x & (kWave - 1);
   const int* astart = p.start + G.ncell_pad;
   const int E = uni(p.start[G.ncell_pad]);
-  const int* aid = (const int*)p.arec + 4;         // event id of record k: aid[8 * k]
-  int lo_l, hi_l;
-  slice_range(tj, G, lo_l, hi_l);
-  {                                                // part p of PARTS: its share of the slices, in order
-    const int L = max(hi_l - lo_l + 1, 0);
-    const int a = lo_l + (part * L) / PARTS, b = lo_l + ((part + 1) * L) / PARTS - 1;
-    lo_l = a;
-    hi_l = b;
-  }
-  const int bj = key / (G.S * plane_cells);
-  float mgx = 0.f, mgy = 0.f;
-  float4 sv;                                       // the current slice's entry (y, v) and centre
-  float cs;
-  auto visit = [&](int k, int e, auto step) {
-    constexpr int U = decltype(step)::value;
-    float4 A[U];
-    int id[U];
-    // one lane offset for the U loads, the step within the record run folded into the (scalar) base
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      A[u] = ld((const float4*)p.brec + u, (uint32_t)k);
-      if (LOO == kLooId) id[u] = ld(aid + 8 * u, 8u * (uint32_t)k);
-    }
-    const int rem = e - k, self_u = sp - k;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const float at = A[u].z - cs;
-      const float dt = A[u].z - tj;
-      const float rx = A[u].x - (sv.x + sv.z * at);
-      const float ry = A[u].y - (sv.y + sv.w * at);
-      const float d2 = rx * rx + ry * ry;
-      const bool other = LOO == kLooId ? id[u] != sid : LOO == kLooPos ? u != self_u : true;
-      const bool ok = other & !(fabsf(dt) > G.tau) & !(d2 > G.r2max) & (u < rem);
-      const float kern = __builtin_amdgcn_exp2f(d2 * G.kexp);
-      const float f = A[u].w * kern * dt;           // A.w = gS / h^2
-      if (LOO == kLooNone) {                         // every record and the source are finite and below
-        float fo = ok ? f : 0.f;                     // 1e30 (checked), so a zero factor adds exactly nothing
+  const int plane = pl * (G.GH * G.GW);
+  const float cs = slice_centre(sl, G.delta);
+  float g0 = 0.f, g1 = 0.f, g2 = 0.f, g3 = 0.f;
+  // one pair; `other` folds in the caller's own conditions
+  auto term = [&](const float4& A, bool other) {
+    const float at = A.z - cs;
+    const float dt = A.z - tj;
+    const float rx = A.x - (sv.x + sv.z * at);
+    const float ry = A.y - (sv.y + sv.w * at);
+    const float d2 = rx * rx + ry * ry;
+    const bool ok = other & !(fabsf(dt) > G.tau) & !(d2 > G.r2max);
+    const float kern = __builtin_amdgcn_exp2f(d2 * G.kexp);
+    if (TRAJ) {
+      const float f = A.w * kern;                    // A.w = gS / h^2
+      const float fx = f * rx, fy = f * ry;
+      g0 = ok ? g0 + fx : g0;                        // selects: a record may hold anything, NaN included
+      g1 = ok ? g1 + fy : g1;
+      g2 = ok ? fmaf(fx, at, g2) : g2;
+      g3 = ok ? fmaf(fy, at, g3) : g3;
+    } else {
+      const float f = A.w * kern * dt;
+      if (!LOO) {                                    // every record and the entry are finite and below 1e30
+        float fo = ok ? f : 0.f;                     // (checked), so a zero factor adds exactly nothing
         asm volatile("" : "+v"(fo));                 // keep one select (not folded into two after the FMAs)
-        mgx = fmaf(fo, rx, mgx);
-        mgy = fmaf(fo, ry, mgy);
-      } else {                                       // selects: a record may hold anything, NaN included
-        mgx = ok ? fmaf(f, rx, mgx) : mgx;
-        mgy = ok ? fmaf(f, ry, mgy) : mgy;
+        g0 = fmaf(fo, rx, g0);
+        g1 = fmaf(fo, ry, g1);
+      } else {
+        g0 = ok ? fmaf(f, rx, g0) : g0;
+        g1 = ok ? fmaf(f, ry, g1) : g1;
       }
     }
   };
-  auto entry = [&](int s, float4& e4, float& c) {
-    entry_key(make_float2(sr.x, sr.y), make_float2(sr.z, sr.w), tj, bj, s, G, e4.x, e4.y);
-    e4.z = sr.z;
-    e4.w = sr.w;
-    c = slice_centre(s, G.delta);
-  };
-  for (int s = lo_l; s <= hi_l; ++s) {
-    entry(s, sv, cs);
-    const float qx = clampf(sv.x, G.gx0, G.gx1), qy = clampf(sv.y, G.gy0, G.gy1);
-    walk_flat<true>(astart, E, (bj * G.S + s) * plane_cells, qx, qy, R, R2, G, tab, visit);
+  const float qx = clampf(sv.x, G.gx0, G.gx1), qy = clampf(sv.y, G.gy0, G.gy1);
+  float bx0 = 0.f, bx1 = 0.f, by0 = 0.f, by1 = 0.f;
+  // positions clamped into the grid's box or not finite: every lane on its own
+  bool common = __ballot(active && !(finite && qx == sv.x && qy == sv.y)) == 0 && uni(p.P->nonfinite) == 0;
+  if (common) {
+    bx0 = wave_ext<false>(active ? sv.x : INFINITY);
+    bx1 = wave_ext<true>(active ? sv.x : -INFINITY);
+    by0 = wave_ext<false>(active ? sv.y : INFINITY);
+    by1 = wave_ext<true>(active ? sv.y : -INFINITY);
+    const float bw = bx1 - bx0, bh = by1 - by0;
+    common = bw * bh + 2.f * G.cuth * (bw + bh) <= kCommon * G.cuth * G.cuth;
   }
-  return make_float2(mgx, mgy);
+  if (common) {
+    const float vx0 = wave_ext<false>(active ? sv.z : INFINITY), vx1 = wave_ext<true>(active ? sv.z : -INFINITY);
+    const float vy0 = wave_ext<false>(active ? sv.w : INFINITY), vy1 = wave_ext<true>(active ? sv.w : -INFINITY);
+    const float vxm = fmaxf(fabsf(vx0), fabsf(vx1)), vym = fmaxf(fabsf(vy0), fabsf(vy1));
+    const float rw = G.cuth * 1.000001f + sqrtf(vxm * vxm + vym * vym) * atmax * 1.000001f + 0.01f;
+    const float Rw = unif(fminf(rw, R));             // no entry is faster than the plan's bound
+    const float cr = G.cuth * 1.000001f + 0.01f, cr2 = cr * cr;   // 0.01 px: fp32 rounding of positions, as in R
+    float4* sA = (float4*)lds;                       // up to 64 anchors and three of padding
+    int* sI = (int*)(sA + kWave + 4);
+    struct Cand {
+      float4 A;
+      int own;
+    };
+    auto load = [&](int k) {
+      const uint32_t i = (uint32_t)max(k, 0);
+      return Cand{ld((const float4*)p.brec, i), LOO ? ld((const int*)p.bes, i) : -1};
+    };
+    group_walk(astart, E, plane, bx0, bx1, by0, by1, Rw, Rw * Rw, G, load, [&](const Cand& c, int k) {
+      const float at = c.A.z - cs;
+      // the entries' positions at the anchor's time lie in this box
+      const float ex = fmaxf(fmaxf(bx0 + fminf(vx0 * at, vx1 * at) - c.A.x, c.A.x - (bx1 + fmaxf(vx0 * at, vx1 * at))), 0.f);
+      const float ey = fmaxf(fmaxf(by0 + fminf(vy0 * at, vy1 * at) - c.A.y, c.A.y - (by1 + fmaxf(vy0 * at, vy1 * at))), 0.f);
+      const bool keep = (k >= 0) & (ex * ex + ey * ey <= cr2);
+      const uint64_t m = __ballot(keep);
+      const int n = __popcll(m);
+      __syncthreads();                               // one wave: the last chunk's reads are done
+      if (keep) {
+        const int i = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+        sA[i] = c.A;
+        if (LOO) sI[i] = c.own;
+      }
+      if (lane < 3) {                                // padding of weight zero, near the entries
+        sA[n + lane] = make_float4(bx0, by0, cs, 0.f);
+        if (LOO) sI[n + lane] = -1;
+      }
+      __syncthreads();
+      for (int i = 0; i < n; i += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) term(sA[i + u], LOO ? sI[i + u] != pos : true);
+      }
+    });
+  } else if (active) {
+    const float rj = G.cuth * 1.000001f + sqrtf(sv.z * sv.z + sv.w * sv.w) * atmax * 1.000001f + 0.01f;
+    if (rj < R) {                                    // false for NaN / inf velocities: keep the whole-slice walk
+      R = rj;
+      R2 = rj * rj;
+    }
+    walk_flat(astart, E, plane, qx, qy, R, R2, G, (int2*)lds + lane, [&](int k, int e, auto step) {
+      constexpr int U = decltype(step)::value;
+      float4 A[U];
+      int own[U];
+      // one lane offset for the U loads, the step within the record run folded into the (scalar) base
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        A[u] = ld((const float4*)p.brec + u, (uint32_t)k);
+        if (LOO) own[u] = ld((const int*)p.bes + u, (uint32_t)k);
+      }
+      const int rem = e - k;
+#pragma unroll
+      for (int u = 0; u < U; ++u) term(A[u], (u < rem) & (LOO ? own[u] != pos : true));
+    });
+  }
+  if constexpr (TRAJ)
+    return make_float4(g0, g1, g2, g3);
+  else
+    return make_float2(g0, g1);
 }
 
-// Backward: every source (one lane each, own-slice tile order) sums, over the anchors of each slice of its
-// range within R of its slice-centre position, gS_i * k * dt / h^2 * r (csrc/atl_cpu.cpp:240-248);
-// gv[j] = the total (each source has one record: no atomics).
-template <int PARTS>
-__global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(6))) k_fast_bwd(FPlan p, FGeo G, int N, float2* __restrict__ gv,
-                                                      float2* __restrict__ gvr) {
-  __shared__ int2 tab[kRowTab * kPairBlock];           // per-lane row spans of the current slice (column threadIdx.x)
-  constexpr int kSrcPerWave = kWave / PARTS;
-  const int lb = xcd_block((N + kPairBlock / PARTS - 1) / (kPairBlock / PARTS));
+template <bool TRAJ>
+__global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(TRAJ ? 5 : 5))) k_entry_bwd(
+    FPlan p, FGeo G, int N, int ecap, EntSum<TRAJ>* __restrict__ slots) {
+  __shared__ __align__(16) char lds[kRowTab * kPairBlock * sizeof(int2)];
+  static_assert(sizeof(lds) >= (kWave + 4) * (sizeof(float4) + sizeof(int)), "the compact anchors share the row table");
+  const int lb = xcd_block((ecap + kWave - 1) / kWave);
   if (lb < 0) return;
   const int lane = threadIdx.x & (kWave - 1);
-  const int part = lane / kSrcPerWave, ls = lane - part * kSrcPerWave;
-  const int wbase = (lb * (kPairBlock / kWave) + (int)(threadIdx.x / kWave)) * kSrcPerWave;
-  const int EA = uni(p.start[2 * G.ncell_pad]);
-  const int Nv = uni(p.start[3 * G.ncell_pad]) - EA;
-  if (wbase >= Nv) return;
-  const int n = min(kSrcPerWave, Nv - wbase);
+  // loads ahead of the check against the entry count, so that they are in flight with it: positions up to ecap are
+  // allocated, and what lies past the entries is not used
+  const int p0 = lb * kWave, pos = min(p0 + lane, ecap - 1);
+  const float4 sv = p.epos[pos];
+  const float2 tq = p.etq[pos];
+  const float tj = tq.x;
+  int q = __float_as_int(tq.y);
+  const int E = uni(p.start[G.ncell_pad]);
+  if (p0 >= E) return;
+  const int p1 = min(p0 + kWave, E);
+  if (TRAJ) q = pos < p1 ? p.spos[q] : 0;            // past the entries q may hold anything
   float R, R2;
   search_radius(p.P, G, R, R2);
   R = unif(R);
   R2 = unif(R2);
-  const bool have = ls < n;
-  const Rec SR = p.srec[wbase + min(ls, n - 1)];
-  const int4 si = SR.i;
-  const float tj = __int_as_float(si.x);
-  // this source's own search radius: its entries all move with its own velocity, |v_j| * max|at| <= vmax * max|at|
-  {
-    const float vj = sqrtf(SR.f.z * SR.f.z + SR.f.w * SR.f.w);
-    const float rj = G.cuth * 1.000001f + vj * ordered_to_float(p.P->atmax) * 1.000001f + 0.01f;
-    if (rj < R) {                                  // false for NaN / inf velocities: keep the whole-slice walk
-      R = rj;
-      R2 = rj * rj;
+  const float atmax = unif(ordered_to_float(p.P->atmax));
+  const bool finite = bounded(sv.x) && bounded(sv.y) && bounded(sv.z) && bounded(sv.w) && bounded(tj);
+  // the own pair's test can go where every term of an entry with its own anchor is exactly zero
+  const bool loo = TRAJ || uni(p.P->nonfinite) != 0 || __ballot(pos < p1 && !finite) != 0;
+  const int plane_cells = G.GH * G.GW, nplanes = (int)G.B * G.S;
+  int lo, hi;
+  slice_range(tj, G, lo, hi);
+  EntSum<TRAJ> sum{};
+  int pl = 0;
+  for (int a = p0; a < p1;) {                        // the wave's entries plane by plane (mostly one plane)
+    // the last plane that starts at or before position a (empty planes start where the next one does)
+    for (int base = pl;; base += kWave) {
+      const int c = base + lane;
+      const int n = __popcll(__ballot(c < nplanes && p.start[min(c, nplanes - 1) * plane_cells] <= a));
+      pl = base + n - 1;
+      if (n < kWave) break;
+    }
+    const int e = min(p1, pl + 1 < nplanes ? uni(p.start[(pl + 1) * plane_cells]) : E);
+    const bool active = p0 + lane >= a && p0 + lane < e;
+    const int sl = pl % G.S;
+    const EntSum<TRAJ> r = loo ? entry_sum<TRAJ, true>(p, G, R, R2, atmax, sv, tj, pos, pl, sl, active, finite, lds)
+                               : entry_sum<TRAJ, TRAJ>(p, G, R, R2, atmax, sv, tj, pos, pl, sl, active, finite, lds);
+    if (active) {
+      sum = r;
+      slots[(int64_t)(sl - lo) * N + q] = sum;
+    }
+    a = e;
+  }
+}
+
+// A source's gradient from its entries' slots, in slice order: by event (gv) or by source record (gvr).
+__global__ void __launch_bounds__(kBlock) k_slot_sum(FPlan p, FGeo G, int N, const float2* __restrict__ slots,
+                                                     float2* __restrict__ gv, float2* __restrict__ gvr) {
+  const int q = blockIdx.x * kBlock + threadIdx.x;
+  if (q >= p.start[3 * G.ncell_pad] - p.start[2 * G.ncell_pad]) return;
+  const int4 si = p.srec[q].i;
+  int lo, hi;
+  slice_range(__int_as_float(si.x), G, lo, hi);
+  float gx = 0.f, gy = 0.f;
+#pragma unroll 4
+  for (int k = 0; k <= hi - lo; ++k) {
+    const float2 g = slots[(int64_t)k * N + q];
+    gx += g.x;
+    gy += g.y;
+  }
+  if (gv) gv[si.y] = make_float2(gx, gy);
+  if (gvr) gvr[q] = make_float2(gx, gy);
+}
+
+// The trajectory model's: y_s = p + sum_k cf_k g_k(c_s) and v_s = sum_k cf_k g_k'(c_s) chain the slots (Gy_s, Gv_s)
+// into gp[j] = sum_s Gy_s and gcoef[j, k] = sum_s (Gy_s g_k(c_s) + Gv_s g_k'(c_s)) per axis (channels
+// [y_1..y_K, x_1..x_K]).
+template <int K>
+__global__ void __launch_bounds__(kBlock) k_slot_traj(FPlan p, FGeo G, int N, const float4* __restrict__ slots,
+                                                      const float* __restrict__ tab, float2* __restrict__ gp,
+                                                      float* __restrict__ gcoef) {
+  const int q = blockIdx.x * kBlock + threadIdx.x;
+  if (q >= p.start[3 * G.ncell_pad] - p.start[2 * G.ncell_pad]) return;
+  const int4 si = p.srec[q].i;
+  int lo, hi;
+  slice_range(__int_as_float(si.x), G, lo, hi);
+  float gx = 0.f, gy = 0.f, gc[2 * K];
+#pragma unroll
+  for (int c = 0; c < 2 * K; ++c) gc[c] = 0.f;
+  for (int s = lo; s <= hi; ++s) {
+    const float4 g = slots[(int64_t)(s - lo) * N + q];
+    const float* row = tab + s * 2 * K;
+    gx += g.x;
+    gy += g.y;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const float b = row[k], d = row[K + k];
+      gc[k] = fmaf(g.y, b, fmaf(g.w, d, gc[k]));
+      gc[K + k] = fmaf(g.x, b, fmaf(g.z, d, gc[K + k]));
     }
   }
-  const int sp = p.self[si.y];
-  int2* mytab = tab + threadIdx.x;
-  float2 m = make_float2(0.f, 0.f);
-  // the leave-one-out test can be skipped when every term of a source with its own anchor is exactly zero
-  const bool src_finite = bounded(SR.f.x) && bounded(SR.f.y) && bounded(SR.f.z) && bounded(SR.f.w) && bounded(tj);
-  const int loo = uni(p.P->dup) ? kLooId : (uni(p.P->nonfinite) || __ballot(have && !src_finite)) ? kLooPos
-                                                                                                    : kLooNone;
-  if (have) {
-    if (loo == kLooId)
-      m = bwd_source<kLooId, PARTS>(p, G, R, R2, SR.f, si.y, tj, si.z, sp, part, mytab);
-    else if (loo == kLooPos)
-      m = bwd_source<kLooPos, PARTS>(p, G, R, R2, SR.f, si.y, tj, si.z, sp, part, mytab);
-    else
-      m = bwd_source<kLooNone, PARTS>(p, G, R, R2, SR.f, si.y, tj, si.z, sp, part, mytab);
-  }
+  gp[si.y] = make_float2(gx, gy);
+  if constexpr (K % 2 == 0) {                      // rows of whole 16-byte pieces: four stores of a quarter the lines
+    float4* o = (float4*)(gcoef + (int64_t)si.y * (2 * K));
 #pragma unroll
-  for (int o = kSrcPerWave; o < kWave; o <<= 1) {  // the parts of a source sit kSrcPerWave lanes apart
-    m.x += __shfl_xor(m.x, o);
-    m.y += __shfl_xor(m.y, o);
-  }
-  if (have && part == 0) {                         // by event (gv), or by source record (gvr, coalesced)
-    if (gv) gv[si.y] = m;
-    if (gvr) gvr[wbase + ls] = m;
+    for (int c = 0; c < K / 2; ++c) o[c] = make_float4(gc[4 * c], gc[4 * c + 1], gc[4 * c + 2], gc[4 * c + 3]);
+  } else {
+    float2* o = (float2*)(gcoef + (int64_t)si.y * (2 * K));
+#pragma unroll
+    for (int c = 0; c < K; ++c) o[c] = make_float2(gc[2 * c], gc[2 * c + 1]);
   }
 }
 
@@ -1741,141 +1952,6 @@ __global__ void __launch_bounds__(kAdjBlock) k_src_flow_adjoint(FPlan p, FGeo G,
   }
 }
 
-// Backward of the trajectory model: every source (one lane per part of its slices, own-slice tile order) sums
-// over the anchors of each slice s of its range, within R of its slice-centre position y_s, the gradients of the
-// entry's position and velocity, Gy_s = sum_i gS_i k r / h^2 and Gv_s = sum_i gS_i k r at_i / h^2
-// (r = x_i - (y_s + v_s at_i), the pair terms of the forward), and chains them in registers through
-// y_s = p + sum_k cf_k g_k(c_s), v_s = sum_k cf_k g_k'(c_s): gp[j] = sum_s Gy_s and
-// gcoef[j, k] = sum_s (Gy_s g_k(c_s) + Gv_s g_k'(c_s)) per axis (channels [y_1..y_K, x_1..x_K]).  Each source's
-// gradients are complete in its lanes and written once, without atomics.
-template <int K, bool DUP>
-__device__ __forceinline__ void bwd_traj_source(const FPlan& p, const FGeo& G, float R, float R2, float atmax, float px,
-                                                float py, const float (&cf)[2 * K], const float* __restrict__ tab,
-                                                int sid, float tj, int key, int sp, int part, int2* rowtab,
-                                                float (&gc)[2 * K], float& gpx, float& gpy) {
-  const int plane_cells = G.GH * G.GW;
-  const int* astart = p.start + G.ncell_pad;
-  const int E = uni(p.start[G.ncell_pad]);
-  const int* aid = (const int*)p.arec + 4;         // event id of record k: aid[8 * k]
-  int lo_l, hi_l;
-  slice_range(tj, G, lo_l, hi_l);
-  if (kBwdParts > 1) {
-    const int L = max(hi_l - lo_l + 1, 0);
-    const int a = lo_l + (part * L) / kBwdParts, b = lo_l + ((part + 1) * L) / kBwdParts - 1;
-    lo_l = a;
-    hi_l = b;
-  }
-  const int bj = key / (G.S * plane_cells);
-  for (int s = lo_l; s <= hi_l; ++s) {
-    float yx, yy, vx, vy;
-    traj_entry<K>(cf, px, py, tab, s, yx, yy, vx, vy);
-    const float cs = slice_centre(s, G.delta);
-    const float qx = clampf(yx, G.gx0, G.gx1), qy = clampf(yy, G.gy0, G.gy1);
-    // this entry's own search radius: its pairs lie within cut h + |v_s| max|at| of y_s (the global R takes the
-    // largest velocity of all entries); the same slack as search_radius
-    float Rs = R, R2s = R2;
-    {
-      const float rs = G.cuth * 1.000001f + sqrtf(vx * vx + vy * vy) * atmax * 1.000001f + 0.01f;
-      if (rs < R) {                                // false for NaN / inf velocities: keep the global walk
-        Rs = rs;
-        R2s = rs * rs;
-      }
-    }
-    float gyx = 0.f, gyy = 0.f, gvx = 0.f, gvy = 0.f;
-    walk_flat(astart, E, (bj * G.S + s) * plane_cells, qx, qy, Rs, R2s, G, rowtab, [&](int k, int e, auto step) {
-      constexpr int U = decltype(step)::value;
-      float4 A[U];
-      int id[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        A[u] = ld((const float4*)p.brec + u, (uint32_t)k);
-        if (DUP) id[u] = ld(aid + 8 * u, 8u * (uint32_t)k);
-      }
-      const int rem = e - k, self_u = sp - k;
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float at = A[u].z - cs;
-        const float dt = A[u].z - tj;
-        const float rx = A[u].x - (yx + vx * at);
-        const float ry = A[u].y - (yy + vy * at);
-        const float d2 = rx * rx + ry * ry;
-        const bool other = DUP ? id[u] != sid : u != self_u;
-        const bool ok = other & !(fabsf(dt) > G.tau) & !(d2 > G.r2max) & (u < rem);
-        // selects, not products with zero: records past the range end may hold anything, NaN included
-        const float f = A[u].w * __builtin_amdgcn_exp2f(d2 * G.kexp);   // A.w = gS / h^2
-        const float fx = f * rx, fy = f * ry;
-        gyx = ok ? gyx + fx : gyx;
-        gyy = ok ? gyy + fy : gyy;
-        gvx = ok ? fmaf(fx, at, gvx) : gvx;
-        gvy = ok ? fmaf(fy, at, gvy) : gvy;
-      }
-    });
-    gpx += gyx;
-    gpy += gyy;
-    const float* row = tab + s * 2 * K;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const float g = row[k], gd = row[K + k];
-      gc[k] = fmaf(gyy, g, fmaf(gvy, gd, gc[k]));
-      gc[K + k] = fmaf(gyx, g, fmaf(gvx, gd, gc[K + k]));
-    }
-  }
-}
-
-template <int K>
-__global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(4))) k_fast_bwd_traj(FPlan p, FGeo G, int N, const float* __restrict__ coef,
-                                                             const float* __restrict__ tab, float2* __restrict__ gp,
-                                                             float* __restrict__ gcoef) {
-  __shared__ int2 rowtab[kRowTab * kPairBlock];
-  constexpr int kSrcPerWave = kWave / kBwdParts;
-  const int lb = xcd_block((N + kPairBlock / kBwdParts - 1) / (kPairBlock / kBwdParts));
-  if (lb < 0) return;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int part = lane / kSrcPerWave, ls = lane - part * kSrcPerWave;
-  const int wbase = (lb * (kPairBlock / kWave) + (int)(threadIdx.x / kWave)) * kSrcPerWave;
-  const int EA = uni(p.start[2 * G.ncell_pad]);
-  const int Nv = uni(p.start[3 * G.ncell_pad]) - EA;
-  if (wbase >= Nv) return;
-  const int n = min(kSrcPerWave, Nv - wbase);
-  float R, R2;
-  search_radius(p.P, G, R, R2);
-  R = unif(R);
-  R2 = unif(R2);
-  const bool have = ls < n;
-  const Rec SR = p.srec[wbase + min(ls, n - 1)];
-  const int4 si = SR.i;
-  const float tj = __int_as_float(si.x);
-  float cf[2 * K], gc[2 * K];
-#pragma unroll
-  for (int c = 0; c < 2 * K; ++c) {
-    cf[c] = coef[(int64_t)si.y * (2 * K) + c];
-    gc[c] = 0.f;
-  }
-  const int sp = p.self[si.y];
-  float gpx = 0.f, gpy = 0.f;
-  if (have) {
-    const float atmax = unif(ordered_to_float(p.P->atmax));
-    if (uni(p.P->dup))
-      bwd_traj_source<K, true>(p, G, R, R2, atmax, SR.f.x, SR.f.y, cf, tab, si.y, tj, si.z, sp, part,
-                               rowtab + threadIdx.x, gc, gpx, gpy);
-    else
-      bwd_traj_source<K, false>(p, G, R, R2, atmax, SR.f.x, SR.f.y, cf, tab, si.y, tj, si.z, sp, part,
-                                rowtab + threadIdx.x, gc, gpx, gpy);
-  }
-#pragma unroll
-  for (int o = kSrcPerWave; o < kWave; o <<= 1) {  // the parts of a source sit kSrcPerWave lanes apart
-    gpx += __shfl_xor(gpx, o);
-    gpy += __shfl_xor(gpy, o);
-#pragma unroll
-    for (int c = 0; c < 2 * K; ++c) gc[c] += __shfl_xor(gc[c], o);
-  }
-  if (have && part == 0) {
-    gp[si.y] = make_float2(gpx, gpy);
-#pragma unroll
-    for (int c = 0; c < 2 * K; ++c) gcoef[(int64_t)si.y * (2 * K) + c] = gc[c];
-  }
-}
-
 // ------------------------------------------------------------------------------------------ host side
 int64_t align256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 
@@ -1928,12 +2004,13 @@ T* at_off(void* ws, int64_t off) { return (T*)((char*)ws + off); }
 FPlan make_plan(void* ws, const atl_fast_geometry* geo) {
   FPlan p;
   p.epos = at_off<float4>(ws, geo->off_epos);
-  p.etim = at_off<float>(ws, geo->off_etim);
+  p.etq = at_off<float2>(ws, geo->off_etim);
   p.eself = at_off<int>(ws, geo->off_eself);
   p.arec = at_off<Rec>(ws, geo->off_arec);
   p.srec = at_off<Rec>(ws, geo->off_srec);
   p.brec = at_off<float4>(ws, geo->off_brec);
-  p.self = at_off<int>(ws, geo->off_self);
+  p.bes = at_off<int>(ws, geo->off_brec + align256((geo->M + kUnroll) * (int64_t)sizeof(float4)));
+  p.spos = at_off<int>(ws, geo->off_self);
   p.start = at_off<int>(ws, geo->off_start);
   p.P = at_off<FParams>(ws, geo->off_params);
   return p;
@@ -1944,14 +2021,24 @@ unsigned xcd_grid(int64_t nblocks) {
   return (unsigned)(((nblocks + g - 1) / g) * g);
 }
 
-void launch_bwd(const FPlan& p, const FGeo& G, int64_t N, float2* gv, float2* gvr, hipStream_t stream) {
-  const int parts = N > kBwdSmall ? kBwdParts : kBwdPartsSmall;
-  const int spw = kWave / parts;                   // sources per wave
-  const dim3 grid(xcd_grid((N + spw - 1) / spw));
-  if (parts == kBwdParts)
-    hipLaunchKernelGGL(k_fast_bwd<kBwdParts>, grid, dim3(kPairBlock), 0, stream, p, G, (int)N, gv, gvr);
-  else
-    hipLaunchKernelGGL(k_fast_bwd<kBwdPartsSmall>, grid, dim3(kPairBlock), 0, stream, p, G, (int)N, gv, gvr);
+// The slots of the entries' sums in the sort-record region, after the flow adjoint's scratch.
+template <typename T>
+T* slots_of(void* ws, const atl_fast_geometry* geo) {
+  return at_off<T>(ws, geo->off_trec + align256(adj_scratch_bytes(geo->B, geo->N, geo->GW, geo->GH, geo->cell)));
+}
+
+template <bool TRAJ>
+void launch_entry_bwd(const FPlan& p, const FGeo& G, const atl_fast_geometry* geo, void* ws, hipStream_t stream) {
+  const int64_t nblocks = (geo->ecap + kWave - 1) / kWave;
+  hipLaunchKernelGGL(k_entry_bwd<TRAJ>, dim3(xcd_grid(nblocks)), dim3(kPairBlock), 0, stream, p, G, (int)geo->N,
+                     (int)geo->ecap, slots_of<EntSum<TRAJ>>(ws, geo));
+}
+
+void launch_bwd(const FPlan& p, const FGeo& G, const atl_fast_geometry* geo, void* ws, float2* gv, float2* gvr,
+                hipStream_t stream) {
+  launch_entry_bwd<false>(p, G, geo, ws, stream);
+  hipLaunchKernelGGL(k_slot_sum, dim3(grid_for(geo->N)), dim3(kBlock), 0, stream, p, G, (int)geo->N,
+                     (const float2*)slots_of<float2>(ws, geo), gv, gvr);
 }
 
 }  // namespace
@@ -2025,16 +2112,17 @@ int atl_fast_geometry_init(int64_t N, int64_t M, int64_t B, int64_t H, int64_t W
   g.off_start = off;   off += align256((3 * g.ncell_pad + 1) * 4);
   // the sort's records sit at their bucket positions in all three key spaces (the linear model's anchor and
   // source records after the entries' counted places), so the region holds ecap + M + N records; after the plan
-  // it also serves the flow adjoint's scratch (per-source gradients, chunk list, tile counts)
+  // it also serves the flow adjoint's scratch (per-source gradients, chunk list, tile counts) and the backward's slots
   g.off_trec = off;    off += align256(std::max((g.ecap + M + N) * (int64_t)sizeof(Rec),
-                                                adj_scratch_bytes(B, N, g.GW, g.GH, g.cell)));
+                                                align256(adj_scratch_bytes(B, N, g.GW, g.GH, g.cell)) +
+                                                    g.ecap * (int64_t)sizeof(float4)));
   // the walks read up to kUnroll - 1 records past a range end: entry and anchor arrays carry that padding
   g.off_epos = off;    off += align256((g.ecap + kUnroll) * (int64_t)sizeof(float4));
-  g.off_etim = off;    off += align256((g.ecap + kUnroll) * (int64_t)sizeof(float));
+  g.off_etim = off;    off += align256((g.ecap + kUnroll) * (int64_t)sizeof(float2));
   g.off_eself = off;   off += align256(N * (int64_t)sizeof(int));
   g.off_arec = off;    off += align256((M + kUnroll) * (int64_t)sizeof(Rec));
   g.off_srec = off;    off += align256(N * (int64_t)sizeof(Rec));
-  g.off_brec = off;    off += align256((M + kUnroll) * (int64_t)sizeof(float4));
+  g.off_brec = off;    off += align256((M + kUnroll) * (int64_t)sizeof(float4)) + align256((M + kUnroll) * 4);
   g.off_self = off;    off += align256(N * (int64_t)sizeof(int));
   g.ws_bytes = off;
   *geo = g;
@@ -2074,8 +2162,9 @@ int fast_plan_impl(const atl_fast_geometry* geo, const FGeo& G, const float* x, 
                        (const float2*)x, t, (const float2*)v, b, N, anchors, (const float2*)anchor_xy, M, G, cnt,
                        bpos, trec, (FParams*)nullptr, (int*)nullptr, (int*)nullptr, coef, tab);
   const SortOut out{at_off<int>(ws, geo->off_start), at_off<float4>(ws, geo->off_epos),
-                    at_off<float>(ws, geo->off_etim), at_off<int>(ws, geo->off_eself),
-                    at_off<Rec>(ws, geo->off_arec), at_off<Rec>(ws, geo->off_srec), at_off<int>(ws, geo->off_self)};
+                    at_off<float2>(ws, geo->off_etim), at_off<int>(ws, geo->off_eself),
+                    at_off<Rec>(ws, geo->off_arec), at_off<Rec>(ws, geo->off_srec),
+                    K > 0 ? at_off<int>(ws, geo->off_self) : nullptr};
   // the anchor and source spaces in groups of kSortGroupKeys keys; the entries' space (trajectory model) one
   // bucket per workgroup
   constexpr int kSortGroupKeys = 4096;
@@ -2179,9 +2268,9 @@ int atl_fast_pair_bwd(const atl_fast_geometry* geo, void* ws, const float* gS, f
   if (geo->N == 0) return 0;
   const FPlan p = make_plan(ws, geo);
   hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
-                     (int)geo->M, gS, (int)geo->N, (float2*)gv);
+                     (int)geo->M, gS, (int)geo->N, (float2*)gv, (float*)nullptr, 0);
   if (geo->M > 0)
-    launch_bwd(p, G, geo->N, (float2*)gv, nullptr, stream);
+    launch_bwd(p, G, geo, ws, (float2*)gv, nullptr, stream);
   return check_launch("fast_pair_bwd");
 }
 
@@ -2196,8 +2285,8 @@ int atl_fast_pair_bwd_src(const atl_fast_geometry* geo, void* ws, const float* g
   const FPlan p = make_plan(ws, geo);
   float2* gvr = at_off<float2>(ws, geo->off_trec);
   hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
-                     (int)geo->M, gS, (int)geo->N, (float2*)nullptr);
-  launch_bwd(p, G, geo->N, nullptr, gvr, stream);
+                     (int)geo->M, gS, (int)geo->N, (float2*)nullptr, (float*)nullptr, 0);
+  launch_bwd(p, G, geo, ws, nullptr, gvr, stream);
   return check_launch("fast_pair_bwd_src");
 }
 
@@ -2251,14 +2340,14 @@ int atl_fast_pair_bwd_traj(const atl_fast_geometry* geo, void* ws, const float* 
   if (!ws || (geo->N > 0 && (!gp || !gcoef || !coef || !tab)) || (geo->M > 0 && !gS)) { set_error("fast_pair_bwd_traj: null argument"); return 1; }
   if (geo->N == 0) return 0;
   const FPlan p = make_plan(ws, geo);
-  // gp cleared by the record pass, gcoef here: sources outside the plan keep zero gradients
-  hipLaunchKernelGGL(k_fill_zero, dim3(grid_for(geo->N * 2 * K)), dim3(kBlock), 0, stream, (int*)gcoef, geo->N * 2 * K);
+  // the record pass clears gp and the rows of gcoef that no source writes: they keep zero gradients
   hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
-                     (int)geo->M, gS, (int)geo->N, (float2*)gp);
+                     (int)geo->M, gS, (int)geo->N, (float2*)gp, gcoef, (int)(2 * K));
   if (geo->M > 0) {
-    const dim3 grid(xcd_grid((geo->N + kPairBlock / kBwdParts - 1) / (kPairBlock / kBwdParts))), block(kPairBlock);
+    launch_entry_bwd<true>(p, G, geo, ws, stream);
+    const float4* slots = slots_of<float4>(ws, geo);
     switch (K) {
-#define ATL_K(k) case k: hipLaunchKernelGGL(k_fast_bwd_traj<k>, grid, block, 0, stream, p, G, (int)geo->N, coef, tab, (float2*)gp, gcoef); break;
+#define ATL_K(k) case k: hipLaunchKernelGGL(k_slot_traj<k>, dim3(grid_for(geo->N)), dim3(kBlock), 0, stream, p, G, (int)geo->N, slots, tab, (float2*)gp, gcoef); break;
       ATL_K(1) ATL_K(2) ATL_K(3) ATL_K(4) ATL_K(5) ATL_K(6) ATL_K(7) ATL_K(8) ATL_K(9) ATL_K(10) ATL_K(11) ATL_K(12)
 #undef ATL_K
     }
