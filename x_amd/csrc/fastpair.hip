@@ -1680,14 +1680,10 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
   }
 }
 
-// A source's gradient from its entries' slots, in slice order: by event (gv) or by source record (gvr).
-__global__ void __launch_bounds__(kBlock) k_slot_sum(FPlan p, FGeo G, int N, const float2* __restrict__ slots,
-                                                     float2* __restrict__ gv, float2* __restrict__ gvr) {
-  const int q = blockIdx.x * kBlock + threadIdx.x;
-  if (q >= p.start[3 * G.ncell_pad] - p.start[2 * G.ncell_pad]) return;
-  const int4 si = p.srec[q].i;
+// A source's gradient from its entries' slots, in slice order; q its record, t its time.
+__device__ __forceinline__ float2 slot_sum(const FGeo& G, const float2* __restrict__ slots, int N, int q, float t) {
   int lo, hi;
-  slice_range(__int_as_float(si.x), G, lo, hi);
+  slice_range(t, G, lo, hi);
   float gx = 0.f, gy = 0.f;
 #pragma unroll 4
   for (int k = 0; k <= hi - lo; ++k) {
@@ -1695,17 +1691,30 @@ __global__ void __launch_bounds__(kBlock) k_slot_sum(FPlan p, FGeo G, int N, con
     gx += g.x;
     gy += g.y;
   }
-  if (gv) gv[si.y] = make_float2(gx, gy);
-  if (gvr) gvr[q] = make_float2(gx, gy);
+  return make_float2(gx, gy);
+}
+
+__global__ void __launch_bounds__(kBlock) k_slot_sum(FPlan p, FGeo G, int N, const float2* __restrict__ slots,
+                                                     float2* __restrict__ gv) {
+  const int q = blockIdx.x * kBlock + threadIdx.x;
+  if (q >= p.start[3 * G.ncell_pad] - p.start[2 * G.ncell_pad]) return;
+  const int4 si = p.srec[q].i;
+  gv[si.y] = slot_sum(G, slots, N, q, __int_as_float(si.x));
 }
 
 // The trajectory model's: y_s = p + sum_k cf_k g_k(c_s) and v_s = sum_k cf_k g_k'(c_s) chain the slots (Gy_s, Gv_s)
 // into gp[j] = sum_s Gy_s and gcoef[j, k] = sum_s (Gy_s g_k(c_s) + Gv_s g_k'(c_s)) per axis (channels
 // [y_1..y_K, x_1..x_K]).
+constexpr int kSlotRows = 64;
 template <int K>
 __global__ void __launch_bounds__(kBlock) k_slot_traj(FPlan p, FGeo G, int N, const float4* __restrict__ slots,
                                                       const float* __restrict__ tab, float2* __restrict__ gp,
                                                       float* __restrict__ gcoef) {
+  // the first rows of the basis table in LDS (one row per slice, all of them at the usual slice counts)
+  __shared__ float stab[kSlotRows * 2 * K];
+  const int nrow = min(G.S, kSlotRows);
+  for (int i = threadIdx.x; i < nrow * 2 * K; i += kBlock) stab[i] = tab[i];
+  __syncthreads();
   const int q = blockIdx.x * kBlock + threadIdx.x;
   if (q >= p.start[3 * G.ncell_pad] - p.start[2 * G.ncell_pad]) return;
   const int4 si = p.srec[q].i;
@@ -1714,16 +1723,24 @@ __global__ void __launch_bounds__(kBlock) k_slot_traj(FPlan p, FGeo G, int N, co
   float gx = 0.f, gy = 0.f, gc[2 * K];
 #pragma unroll
   for (int c = 0; c < 2 * K; ++c) gc[c] = 0.f;
-  for (int s = lo; s <= hi; ++s) {
-    const float4 g = slots[(int64_t)(s - lo) * N + q];
-    const float* row = tab + s * 2 * K;
-    gx += g.x;
-    gy += g.y;
+  constexpr int U = 4;                             // slots in flight
+  for (int s0 = lo; s0 <= hi; s0 += U) {
+    float4 g[U];
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const float b = row[k], d = row[K + k];
-      gc[k] = fmaf(g.y, b, fmaf(g.w, d, gc[k]));
-      gc[K + k] = fmaf(g.x, b, fmaf(g.z, d, gc[K + k]));
+    for (int u = 0; u < U; ++u) g[u] = slots[(int64_t)(min(s0 + u, hi) - lo) * N + q];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = s0 + u;
+      if (s > hi) break;
+      gx += g[u].x;
+      gy += g[u].y;
+      const float* row = s < kSlotRows ? stab + s * 2 * K : tab + s * 2 * K;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const float b = row[k], d = row[K + k];
+        gc[k] = fmaf(g[u].y, b, fmaf(g[u].w, d, gc[k]));
+        gc[K + k] = fmaf(g[u].x, b, fmaf(g[u].z, d, gc[K + k]));
+      }
     }
   }
   gp[si.y] = make_float2(gx, gy);
@@ -1803,7 +1820,7 @@ __global__ void __launch_bounds__(kAdjListBlock) k_src_adj_list(const int* __res
 __global__ void __launch_bounds__(kAdjBlock) k_src_flow_adjoint(FPlan p, FGeo G, FlowGeo F,
                                                              const int2* __restrict__ info,
                                                              const int* __restrict__ nchunk,
-                                                             const float2* __restrict__ gvr,
+                                                             const float2* __restrict__ slots, int N,
                                                              float* __restrict__ ggrid) {
   constexpr int T = kAdjT, L = T + 1;
   __shared__ int seg[kAdjMaxSlices + 1];          // prefix of the S slice ranges' lengths
@@ -1857,8 +1874,10 @@ __global__ void __launch_bounds__(kAdjBlock) k_src_flow_adjoint(FPlan p, FGeo G,
       while (seg[s + 1] <= r) ++s;
       q = sbase[s] + (r - seg[s]);
     }
-    const float4 f = live[u] ? p.srec[q].f : make_float4(0.f, 0.f, 0.f, 0.f);
-    g[u] = live[u] ? gvr[q] : make_float2(0.f, 0.f);
+    Rec R{};
+    if (live[u]) R = p.srec[q];
+    const float4 f = R.f;
+    g[u] = live[u] ? slot_sum(G, slots, N, q, __int_as_float(R.i.x)) : make_float2(0.f, 0.f);
     c[u] = grid_corners(f.x, f.y, F.Hg, F.Wg, F.sxw, F.syh, F.scale != 0);
     live[u] = live[u] && !(g[u].x == 0.f && g[u].y == 0.f);   // a zero row adds nothing
     if (live[u]) {
@@ -1958,13 +1977,12 @@ int64_t align256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 // Source tile edge in cells (about kSrcTilePx px) of a fine-cell size.
 inline int src_tile_cells(float cell) { return std::min(16, std::max(2, (int)std::lround(kSrcTilePx / (double)cell))); }
 
-// Bytes the flow adjoint keeps in the sort-record region: the per-source gradients, then its chunk list, chunk
-// count and tile record counts.
+// Bytes the flow adjoint keeps in the sort-record region: its chunk list, chunk count and tile record counts.
 inline int64_t adj_scratch_bytes(int64_t B, int64_t N, int64_t GW, int64_t GH, float cell) {
   const int64_t st = src_tile_cells(cell);
   const int64_t tiles = B * ((GW + st - 1) / st) * ((GH + st - 1) / st);
   const int64_t maxc = tiles + (N + kAdjChunk - 1) / kAdjChunk;
-  return align256(N * 8) + maxc * (int64_t)sizeof(int2) + 64 * 4 + tiles * 4;
+  return maxc * (int64_t)sizeof(int2) + 64 * 4 + tiles * 4;
 }
 
 bool make_geo(const atl_fast_geometry* geo, FGeo& G) {
@@ -2032,13 +2050,6 @@ void launch_entry_bwd(const FPlan& p, const FGeo& G, const atl_fast_geometry* ge
   const int64_t nblocks = (geo->ecap + kWave - 1) / kWave;
   hipLaunchKernelGGL(k_entry_bwd<TRAJ>, dim3(xcd_grid(nblocks)), dim3(kPairBlock), 0, stream, p, G, (int)geo->N,
                      (int)geo->ecap, slots_of<EntSum<TRAJ>>(ws, geo));
-}
-
-void launch_bwd(const FPlan& p, const FGeo& G, const atl_fast_geometry* geo, void* ws, float2* gv, float2* gvr,
-                hipStream_t stream) {
-  launch_entry_bwd<false>(p, G, geo, ws, stream);
-  hipLaunchKernelGGL(k_slot_sum, dim3(grid_for(geo->N)), dim3(kBlock), 0, stream, p, G, (int)geo->N,
-                     (const float2*)slots_of<float2>(ws, geo), gv, gvr);
 }
 
 }  // namespace
@@ -2270,23 +2281,25 @@ int atl_fast_pair_bwd(const atl_fast_geometry* geo, void* ws, const float* gS, f
   hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
                      (int)geo->M, gS, (int)geo->N, (float2*)gv, (float*)nullptr, 0);
   if (geo->M > 0)
-    launch_bwd(p, G, geo, ws, (float2*)gv, nullptr, stream);
+  {
+    launch_entry_bwd<false>(p, G, geo, ws, stream);
+    hipLaunchKernelGGL(k_slot_sum, dim3(grid_for(geo->N)), dim3(kBlock), 0, stream, p, G, (int)geo->N,
+                       (const float2*)slots_of<float2>(ws, geo), (float2*)gv);
+  }
   return check_launch("fast_pair_bwd");
 }
 
-// The flow path's backward in two steps: the pair backward writes each source's velocity gradient by source
-// record into the plan's temporary sort records (dead after the plan), and the adjoint accumulates them into the
-// flow grid.  atl_fast_pair_bwd_flow runs both.
+// The flow path's backward in two steps: the pair backward writes the entries' sums into the plan's temporary sort
+// records (dead after the plan), and the adjoint adds up each source's and accumulates them into the flow grid.  atl_fast_pair_bwd_flow runs both.
 int atl_fast_pair_bwd_src(const atl_fast_geometry* geo, void* ws, const float* gS, hipStream_t stream) {
   FGeo G;
   if (!make_geo(geo, G)) { set_error("fast_pair_bwd_src: geometry not initialised"); return 1; }
   if (!ws || (geo->M > 0 && !gS)) { set_error("fast_pair_bwd_src: null argument"); return 1; }
   if (geo->N == 0 || geo->M == 0) return 0;
   const FPlan p = make_plan(ws, geo);
-  float2* gvr = at_off<float2>(ws, geo->off_trec);
   hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
                      (int)geo->M, gS, (int)geo->N, (float2*)nullptr, (float*)nullptr, 0);
-  launch_bwd(p, G, geo, ws, nullptr, gvr, stream);
+  launch_entry_bwd<false>(p, G, geo, ws, stream);
   return check_launch("fast_pair_bwd_src");
 }
 
@@ -2302,7 +2315,6 @@ int atl_fast_flow_adjoint(const atl_fast_geometry* geo, void* ws, int64_t Hg, in
     return check_launch("fast_flow_adjoint");
   }
   const FPlan p = make_plan(ws, geo);
-  const float2* gvr = at_off<float2>(ws, geo->off_trec);
   FlowGeo F;
   F.Hg = (int)Hg;
   F.Wg = (int)Wg;
@@ -2311,7 +2323,7 @@ int atl_fast_flow_adjoint(const atl_fast_geometry* geo, void* ws, int64_t Hg, in
   F.syh = (float)(img_h - 1 > 1 ? img_h - 1 : 1);
   const int64_t tiles = geo->B * ((G.GW + G.stile - 1) / G.stile) * ((G.GH + G.stile - 1) / G.stile);
   const int64_t maxc = tiles + (geo->N + kAdjChunk - 1) / kAdjChunk;   // chunks, at most (adj_scratch_bytes)
-  int2* info = (int2*)(at_off<char>(ws, geo->off_trec) + align256(geo->N * 8));   // after the gradients
+  int2* info = at_off<int2>(ws, geo->off_trec);
   int* nchunk = (int*)(info + maxc);
   int* tilecnt = nchunk + 64;
   int SP = 1;
@@ -2322,7 +2334,7 @@ int atl_fast_flow_adjoint(const atl_fast_geometry* geo, void* ws, int64_t Hg, in
   hipLaunchKernelGGL(k_src_adj_list, dim3(1), dim3(kAdjListBlock), 0, stream, (const int*)tilecnt, (int)tiles, info,
                      nchunk);
   hipLaunchKernelGGL(k_src_flow_adjoint, dim3((unsigned)maxc), dim3(kAdjBlock), 0, stream, p, G, F,
-                     (const int2*)info, (const int*)nchunk, gvr, ggrid);
+                     (const int2*)info, (const int*)nchunk, (const float2*)slots_of<float2>(ws, geo), (int)geo->N, ggrid);
   return check_launch("fast_flow_adjoint");
 }
 

@@ -1187,42 +1187,62 @@ __global__ void __launch_bounds__(kBlock) k_window_counts_seq(const float* __res
     for (int64_t i = threadIdx.x; i < nB; i += kBlock) Bk[i] = bt_key(t, b, hif + i);
   }
   __syncthreads();
+  // A block whose anchors' bounds lie far apart (its anchors cross into another batch) searches the events: the
+  // thread's anchors and both bounds step together, 8 loads in flight instead of one (three windows of 84k events:
+  // 34 us, one anchor and bound after the other, as the last block of the launch; WC_AFTER us).
+  if (!fits) {
+    double lv[kWcPer], hv[kWcPer];
+    int64_t l0[kWcPer], l1[kWcPer], h0[kWcPer], h1[kWcPer];
+#pragma unroll
+    for (int u = 0; u < kWcPer; ++u) {
+      const double ki = bt_key(t, b, min(a0 + u * kBlock + (int64_t)threadIdx.x, a1));
+      lv[u] = ki - tau;
+      hv[u] = ki + tau;
+      l0[u] = lof; l1[u] = lol;                    // the block's first and last anchors bound the others
+      h0[u] = hif; h1[u] = hil;
+    }
+    bool more = true;
+    while (more) {
+      more = false;
+#pragma unroll
+      for (int u = 0; u < kWcPer; ++u) {
+        if (l0[u] < l1[u]) {
+          const int64_t mid = (l0[u] + l1[u]) >> 1;
+          if (bt_key(t, b, mid) < lv[u]) l0[u] = mid + 1; else l1[u] = mid;
+        }
+        if (h0[u] < h1[u]) {
+          const int64_t mid = (h0[u] + h1[u]) >> 1;
+          if (bt_key(t, b, mid) <= hv[u]) h0[u] = mid + 1; else h1[u] = mid;
+        }
+        more |= l0[u] < l1[u] || h0[u] < h1[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kWcPer; ++u) {
+      const int64_t a = a0 + u * kBlock + threadIdx.x;
+      const int64_t c = h0[u] - l0[u] - 1;
+      if (a <= a1) out[a] = (float)(c > 0 ? c : 0);
+    }
+    return;
+  }
   for (int u = 0; u < kWcPer; ++u) {
     const int64_t a = a0 + u * kBlock + threadIdx.x;
     if (a > a1) return;
     const double ki = bt_key(t, b, a);
     const double lo_v = ki - tau, hi_v = ki + tau;
-    int64_t first, last;
-    if (fits) {
-      int lo = 0, hi = (int)max(nA, (int64_t)0);
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (A[mid] < lo_v) lo = mid + 1; else hi = mid;
-      }
-      first = lof + lo;
-      lo = 0;
-      hi = (int)max(nB, (int64_t)0);
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (Bk[mid] <= hi_v) lo = mid + 1; else hi = mid;
-      }
-      last = hif + lo;
-    } else {
-      int64_t lo = 0, hi = N;
-      while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (bt_key(t, b, mid) < lo_v) lo = mid + 1; else hi = mid;
-      }
-      first = lo;
-      lo = first;
-      hi = N;
-      while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (bt_key(t, b, mid) <= hi_v) lo = mid + 1; else hi = mid;
-      }
-      last = lo;
+    int lo = 0, hi = (int)max(nA, (int64_t)0);
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (A[mid] < lo_v) lo = mid + 1; else hi = mid;
     }
-    const int64_t c = last - first - 1;
+    const int64_t first = lof + lo;
+    lo = 0;
+    hi = (int)max(nB, (int64_t)0);
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (Bk[mid] <= hi_v) lo = mid + 1; else hi = mid;
+    }
+    const int64_t c = hif + lo - first - 1;
     out[a] = (float)(c > 0 ? c : 0);
   }
 }
