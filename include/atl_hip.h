@@ -369,7 +369,7 @@ typedef struct atl_fast_geometry {
   int64_t N, M, B, H, W, S;
   double h, tau, cut;
   float gx0, gy0, gx1, gy1, cell;       /* clamp box and fine cell size (pixels) */
-  float reserved_f;
+  float direct;                /* non-zero: linear sums without a plan (atl_fast_geometry_direct) */
   int64_t GW, GH, ncell, ncell_pad, max_span, ecap;
   int64_t ws_bytes;                     /* workspace layout (byte offsets) */
   int64_t off_params, off_cnt, off_boff, off_part, off_start, off_trec, off_epos, off_etim, off_eself, off_arec,
@@ -399,6 +399,10 @@ int atl_fast_pair_bwd_src(const atl_fast_geometry* geo, void* ws, const float* g
 int atl_fast_flow_adjoint(const atl_fast_geometry* geo, void* ws, int64_t Hg, int64_t Wg, int64_t img_h,
                           int64_t img_w, float* ggrid, hipStream_t stream);
 
+/* Optional, between atl_fast_geometry_init and atl_fast_plan of the linear model: few enough anchors and sources take
+ * every pair directly instead of planning (the same entry points, sums and gradients; geo->direct tells).  Such a
+ * geometry is refused by the trajectory entries. */
+int atl_fast_geometry_direct(atl_fast_geometry* geo);
 /* The same fused pair sums for trajectory motion (the anchored score with PixelTrajectories, which the
  * reference's exact kernel does not take: atl/objectives/ats.py:77-78 requires motion linear at the event).
  * No counterpart in the reference's extension; it replaces atl_fast_plan / atl_fast_pair_bwd where each

@@ -302,3 +302,56 @@ def test_pair_sums_flow_full_size_matches_composed():
     # the same pairs; the within-cell record order follows the plan's LDS atomics, so sums differ in the last bits
     assert_sums_close(res[0][0], res[1][0])
     close_rel(res[0][1], res[1][1], 1e-4)
+
+
+class _PlannedSums(F.FastPairPlan):
+    """The fused path with its plan, also where few events would be summed directly."""
+
+    def _geometry(self, *sizes):
+        super()._geometry(*sizes)
+        self.geo.direct = 0.0
+
+
+@pytest.mark.parametrize("n,m,B,S,h,tau", [(1, None, 1, 16, 1.0, 0.2), (15, 7, 2, 1, 2.0, 0.4), (64, None, 1, 3, 1.0, 1.0),
+                                           (65, 130, 3, 16, 0.7, 0.05), (2049, None, 2, 16, 1.0, 0.2),
+                                           (16384, 2048, 4, 8, 1.5, 0.3)])
+def test_direct_sums_equal_the_planned_ones(n, m, B, S, h, tau):
+    print(f"direct sums n={n} m={m} B={B} S={S}", flush=True)
+    rng = np.random.default_rng(n)
+    H, W = 40, 48
+    x = (rng.random((n, 2)) * [W + 3, H + 3] + 12).astype(F32)   # none near the corner where the plan keeps a NaN
+    t = (rng.random(n) * 1.2 - 0.1).astype(F32)
+    v = (rng.normal(size=(n, 2)) * 15).astype(F32)
+    b = rng.integers(0, B, n)
+    if n > 60:
+        if S >= 8:                                 # outside every planned walk while these are short
+            x[3] = np.nan
+        x[5:9] = x[4]
+        t[5:9] = t[4]
+        b[10], b[11] = -1, B                       # left out
+        v[12] = 60.0
+    anchors = None if m is None else rng.integers(0, n, m)     # repeated events among them
+    xa = x if m is None else x[anchors]
+    xa = (xa + h * rng.normal(size=xa.shape)).astype(F32)
+    gS = rng.normal(size=xa.shape[0]).astype(F32)
+    res = []
+    for cls in (F.FastPairPlan, _PlannedSums):
+        p = cls(T(x), T(t), T(v), T(b), B, H, W, None if m is None else T(anchors), h, tau, 3.0, S, T(xa))
+        assert (p.geo.direct != 0) == (cls is F.FastPairPlan)
+        res.append((N(p.counts()), N(p.forward()), N(p.backward(T(gS))), N(p.backward_flow(T(gS), B, 7, 9, H, W))))
+    (c0, s0, g0, f0), (c1, s1, g1, f1) = res
+    assert np.array_equal(c0, c1)                  # the same pairs
+    # the same fp32 terms (all below 1) in another order
+    assert np.abs(s0 - s1).max() <= 2.0 ** -22 * max(c1.max(), 1)
+    # a source's term is at most |gS| tau r / h^2 with r <= 3 h; fp32 sums of up to m of them
+    bound = float(np.abs(gS).max()) * tau * 3.0 / h
+    assert np.abs(g0 - g1).max() <= 2.0 ** -21 * bound * max(c1.max(), 1) * 4
+    assert np.abs(f0 - f1).max() <= 2.0 ** -20 * max(np.abs(f1).max(), bound)
+
+
+def test_direct_sums_end_at_their_limits():
+    for n, m, direct in ((16384, 2048, True), (16385, 16, False), (5793, 5793, False), (5792, 5792, True)):
+        x = torch.zeros(n, 2, device=DEV)
+        a = torch.zeros(m, dtype=torch.int64, device=DEV)
+        p = F.FastPairPlan(x, x[:, 0], x, a.new_zeros(n), 1, 40, 48, a, 1.0, 0.2)
+        assert (p.geo.direct != 0) == direct

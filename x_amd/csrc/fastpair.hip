@@ -1971,6 +1971,210 @@ __global__ void __launch_bounds__(kAdjBlock) k_src_flow_adjoint(FPlan p, FGeo G,
   }
 }
 
+// ------------------------------------------------------------------------------------------ few events
+// Linear sums of at most kSmallPairs anchor x source pairs (kSmallMax of each) skip the plan: one launch packs the records, and forward and
+// backward take all sources (anchors) of the right slices, 64 at a time, compacted into LDS.  16 anchors (sources) share a
+// wave, each in four lanes, eight waves share them, every wave taking each eighth chunk; the waves' sums are added in
+// order.  The plan and its walks cost 12 launches and some 100 us of latency however few the events: SMALL_NOTE
+constexpr int64_t kSmallPairs = 1 << 25, kSmallMax = 16384;
+constexpr int kSmallWaves = 8, kSmallBlock = kSmallWaves * kWave;
+constexpr int kSmallParts = 4, kSmallQ = kWave / kSmallParts;      // lanes per query, queries per workgroup
+constexpr int kSmallSlots = kWave + 2 * kSmallParts;               // a chunk, padded to two of every part
+
+// Sources: f = (x, y, v), i = (t, -, hi << 16 | lo, window or -1).  Anchors: f = (x, y, t, slice centre), i = (event id,
+// slice, -, window or -1).  The window of what the plan would leave out is -1.
+// A NaN position meets nothing (the plan puts it into the corner cell, 16 px outside the sensor).
+__device__ __forceinline__ bool nowhere(float2 p) { return p.x != p.x || p.y != p.y; }
+
+__global__ void __launch_bounds__(kBlock) k_small_pack(const float2* __restrict__ x, const float* __restrict__ t,
+                                                       const float2* __restrict__ v, const int64_t* __restrict__ b,
+                                                       int N, const int64_t* __restrict__ anchors,
+                                                       const float2* __restrict__ anchor_xy, int M, FGeo G,
+                                                       Rec* __restrict__ srec, Rec* __restrict__ arec) {
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  if (k < N) {
+    const float2 xj = x[k], vj = v[k];
+    const float tj = t[k];
+    const int64_t bj = b[k];
+    int lo, hi;
+    slice_range(tj, G, lo, hi);
+    Rec r;
+    r.f = make_float4(xj.x, xj.y, vj.x, vj.y);
+    r.i = make_int4(__float_as_int(tj), 0, (int)((unsigned)hi << 16 | (unsigned)lo),
+                    bj >= 0 && bj < G.B && lo <= hi && !nowhere(xj) ? (int)bj : -1);
+    srec[k] = r;
+  }
+  if (k < M) {
+    Rec r;
+    int key;
+    r.f = make_float4(0.f, 0.f, 0.f, 0.f);
+    r.i = make_int4(-1, 0, 0, -1);
+    if (anchor_rec(k, x, t, b, anchors, anchor_xy, N, G, key, r)) {
+      const int s = anchor_slice(r.f.z, G);
+      r.f.w = slice_centre(s, G.delta);
+      r.i = make_int4(r.i.x, s, 0, nowhere(make_float2(r.f.x, r.f.y)) ? -1 : (int)b[r.i.x]);
+    }
+    arec[k] = r;
+  }
+}
+
+// Sum of a query's parts and waves, in a fixed order, in the first kSmallQ threads.
+template <typename T>
+__device__ __forceinline__ T small_sum(T v, T (&red)[kSmallWaves][kSmallQ]) {
+  v += __shfl_xor(v, kSmallQ, kWave);
+  v += __shfl_xor(v, 2 * kSmallQ, kWave);
+  const int lane = threadIdx.x & (kWave - 1);
+  __syncthreads();
+  if (lane < kSmallQ) red[threadIdx.x / kWave][lane] = v;
+  __syncthreads();
+  T s = 0;
+  if (threadIdx.x < kSmallQ)
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; ++w) s += red[w][threadIdx.x];
+  return s;
+}
+
+__device__ __forceinline__ int lane_rank(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
+
+template <bool COUNT>
+__global__ void __launch_bounds__(kSmallBlock) k_small_fwd(const Rec* __restrict__ srec, int N,
+                                                           const Rec* __restrict__ arec, int M, FGeo G,
+                                                           float* __restrict__ out, int* __restrict__ count) {
+  __shared__ float4 sE[kSmallWaves][kSmallSlots];
+  __shared__ int4 sI[kSmallWaves][kSmallSlots];      // (t, source id, hi << 16 | lo, window)
+  __shared__ float red[kSmallWaves][kSmallQ];
+  __shared__ int redc[COUNT ? kSmallWaves : 1][kSmallQ];
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  const int q = blockIdx.x * kSmallQ + (lane & (kSmallQ - 1)), part = lane / kSmallQ;
+  const Rec A = arec[min(q, M - 1)];
+  const int bq = q < M ? A.i.w : -1, sq = A.i.y;
+  const float cs = A.f.w, at = A.f.z - cs;
+  const int smin = wave_min_i(bq >= 0 ? sq : 0x7fffffff), smax = wave_max_i(bq >= 0 ? sq : -1);
+  const int bmin = wave_min_i(bq >= 0 ? bq : 0x7fffffff), bmax = wave_max_i(bq);
+  float acc = 0.f;
+  int cnt = 0;
+  for (int c0 = w * kWave; c0 < N; c0 += kSmallBlock) {
+    const int j = c0 + lane;
+    const Rec r = srec[min(j, N - 1)];
+    const bool keep = j < N && r.i.w >= max(bmin, 0) && r.i.w <= bmax && (r.i.z & 0xffff) <= smax &&
+                      (int)((unsigned)r.i.z >> 16) >= smin;
+    const uint64_t m = __ballot(keep);
+    const int n = __popcll(m);
+    __builtin_amdgcn_wave_barrier();
+    if (keep) {
+      const int i = lane_rank(m);
+      sE[w][i] = r.f;
+      sI[w][i] = make_int4(r.i.x, j, r.i.z, r.i.w);
+    }
+    if (lane < 2 * kSmallParts) {
+      sE[w][n + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+      sI[w][n + lane] = make_int4(0, -1, 0, -2);     // of no window
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int i = part; i < n + part; i += 2 * kSmallParts) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float4 f = sE[w][i + u * kSmallParts];
+        const int4 d = sI[w][i + u * kSmallParts];
+        const float ts = __int_as_float(d.x), ds = cs - ts;          // entry_key's operations
+        const float4 e = make_float4(f.x + f.z * ds, f.y + f.w * ds, f.z, f.w);
+        float dt, rx, ry, d2;
+        const bool ok = pair_test(A.i.x, d.y, A.f.z, ts, A.f.x, A.f.y, at, e, G, dt, rx, ry, d2) & (d.w == bq) &
+                        ((d.z & 0xffff) <= sq) & ((int)((unsigned)d.z >> 16) >= sq);
+        const float kern = __builtin_amdgcn_exp2f(d2 * G.kexp);
+        acc += ok ? kern : 0.f;
+        if (COUNT) cnt += ok ? 1 : 0;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  const float s = small_sum(acc, red);
+  int c = 0;
+  if constexpr (COUNT) c = small_sum(cnt, redc);
+  if (threadIdx.x < kSmallQ && bq >= 0) {
+    out[q] = s;
+    if (COUNT) count[q] = c;
+  }
+}
+
+// gv[j] of every source in order, zero for those outside the plan.
+__global__ void __launch_bounds__(kSmallBlock) k_small_bwd(const Rec* __restrict__ srec, int N,
+                                                           const Rec* __restrict__ arec, int M, FGeo G,
+                                                           const float* __restrict__ gS, float2* __restrict__ gv) {
+  __shared__ float4 sA[kSmallWaves][kSmallSlots];    // (x, y, t, slice centre)
+  __shared__ int4 sI[kSmallWaves][kSmallSlots];      // (event id, slice, gS / h^2, window)
+  __shared__ float red[kSmallWaves][kSmallQ];
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  const int j = blockIdx.x * kSmallQ + (lane & (kSmallQ - 1)), part = lane / kSmallQ;
+  const Rec S = srec[min(j, N - 1)];
+  const int bj = j < N ? S.i.w : -1, lo = S.i.z & 0xffff, hi = (int)((unsigned)S.i.z >> 16);
+  const float tj = __int_as_float(S.i.x);
+  const int smin = wave_min_i(bj >= 0 ? lo : 0x7fffffff), smax = wave_max_i(bj >= 0 ? hi : -1);
+  const int bmin = wave_min_i(bj >= 0 ? bj : 0x7fffffff), bmax = wave_max_i(bj);
+  float gx = 0.f, gy = 0.f;
+  for (int c0 = w * kWave; c0 < M; c0 += kSmallBlock) {
+    const int k = c0 + lane;
+    const Rec r = arec[min(k, M - 1)];
+    const float g = gS[min(k, M - 1)] * G.invh2;
+    const bool keep = k < M && r.i.w >= max(bmin, 0) && r.i.w <= bmax && r.i.y >= smin && r.i.y <= smax;
+    const uint64_t m = __ballot(keep);
+    const int n = __popcll(m);
+    __builtin_amdgcn_wave_barrier();
+    if (keep) {
+      const int i = lane_rank(m);
+      sA[w][i] = r.f;
+      sI[w][i] = make_int4(r.i.x, r.i.y, __float_as_int(g), r.i.w);
+    }
+    if (lane < 2 * kSmallParts) {
+      sA[w][n + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+      sI[w][n + lane] = make_int4(-2, 0, 0, -2);     // of no window
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int i = part; i < n + part; i += 2 * kSmallParts) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float4 a = sA[w][i + u * kSmallParts];
+        const int4 d = sI[w][i + u * kSmallParts];
+        const float cs = a.w, at = a.z - cs, ds = cs - tj;
+        const float4 e = make_float4(S.f.x + S.f.z * ds, S.f.y + S.f.w * ds, S.f.z, S.f.w);
+        float dt, rx, ry, d2;
+        const bool ok = pair_test(d.x, j, a.z, tj, a.x, a.y, at, e, G, dt, rx, ry, d2) & (d.w == bj) & (d.y >= lo) &
+                        (d.y <= hi);
+        const float f = __int_as_float(d.z) * __builtin_amdgcn_exp2f(d2 * G.kexp) * dt;
+        gx = ok ? fmaf(f, rx, gx) : gx;
+        gy = ok ? fmaf(f, ry, gy) : gy;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  const float sx = small_sum(gx, red), sy = small_sum(gy, red);
+  if (threadIdx.x < kSmallQ && j < N) gv[j] = make_float2(sx, sy);
+}
+
+// The flow adjoint of few sources: the corners of each added with global atomics.
+__global__ void __launch_bounds__(kBlock) k_small_adjoint(const Rec* __restrict__ srec, int N, FlowGeo F,
+                                                          const float2* __restrict__ gvr, float* __restrict__ ggrid) {
+  const int j = blockIdx.x * kBlock + threadIdx.x;
+  if (j >= N) return;
+  const Rec r = srec[j];
+  const float2 g = gvr[j];
+  if (r.i.w < 0 || (g.x == 0.f && g.y == 0.f)) return;   // a zero row adds nothing
+  const GridCorners c = grid_corners(r.f.x, r.f.y, F.Hg, F.Wg, F.sxw, F.syh, F.scale != 0);
+  const int64_t plane = (int64_t)F.Hg * F.Wg;
+  float* gb = ggrid + r.i.w * 2 * plane;
+  const int o[4] = {c.o00, c.o01, c.o10, c.o11};
+  const float w[4] = {c.w00, c.w01, c.w10, c.w11};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    atomicAdd(gb + o[k], g.x * w[k]);
+    atomicAdd(gb + plane + o[k], g.y * w[k]);
+  }
+}
+
 // ------------------------------------------------------------------------------------------ host side
 int64_t align256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 
@@ -2039,10 +2243,19 @@ unsigned xcd_grid(int64_t nblocks) {
   return (unsigned)(((nblocks + g - 1) / g) * g);
 }
 
+// Whether the linear model's sums run without a plan (atl_fast_geometry_direct).
+bool is_small(const atl_fast_geometry* geo) { return geo->direct != 0.f && geo->N > 0 && geo->M > 0; }
+
 // The slots of the entries' sums in the sort-record region, after the flow adjoint's scratch.
 template <typename T>
 T* slots_of(void* ws, const atl_fast_geometry* geo) {
   return at_off<T>(ws, geo->off_trec + align256(adj_scratch_bytes(geo->B, geo->N, geo->GW, geo->GH, geo->cell)));
+}
+
+void launch_small_bwd(const FPlan& p, const FGeo& G, const atl_fast_geometry* geo, const float* gS, float2* gv,
+                      hipStream_t stream) {
+  hipLaunchKernelGGL(k_small_bwd, dim3((unsigned)((geo->N + kSmallQ - 1) / kSmallQ)), dim3(kSmallBlock), 0, stream,
+                     p.srec, (int)geo->N, p.arec, (int)geo->M, G, gS, gv);
 }
 
 template <bool TRAJ>
@@ -2137,6 +2350,12 @@ int atl_fast_geometry_init(int64_t N, int64_t M, int64_t B, int64_t H, int64_t W
   g.off_self = off;    off += align256(N * (int64_t)sizeof(int));
   g.ws_bytes = off;
   *geo = g;
+  return 0;
+}
+
+int atl_fast_geometry_direct(atl_fast_geometry* geo) {
+  if (!geo || geo->version != ATL_HIP_ABI_VERSION) { set_error("fast_geometry_direct: geometry not initialised"); return 1; }
+  geo->direct = geo->N <= kSmallMax && geo->M <= kSmallMax && geo->N * geo->M <= kSmallPairs ? 1.f : 0.f;
   return 0;
 }
 
@@ -2238,6 +2457,12 @@ int atl_fast_plan(const atl_fast_geometry* geo, const float* x, const float* t, 
   if (!plan_args_ok(geo, G, ws, ws_bytes, "fast_plan")) return 1;
   const int64_t N = geo->N, M = geo->M;
   if ((N > 0 && (!x || !t || !v || !b)) || (M > 0 && !anchors && M != N)) { set_error("fast_plan: null input"); return 1; }
+  if (is_small(geo)) {
+    hipLaunchKernelGGL(k_small_pack, dim3(grid_for(std::max(N, M))), dim3(kBlock), 0, stream, (const float2*)x, t,
+                       (const float2*)v, b, (int)N, anchors, (const float2*)anchor_xy, (int)M, G,
+                       at_off<Rec>(ws, geo->off_srec), at_off<Rec>(ws, geo->off_arec));
+    return check_launch("fast_plan");
+  }
   fast_plan_impl<0>(geo, G, x, t, v, b, anchors, anchor_xy, nullptr, nullptr, ws, stream);
   return check_launch("fast_plan");
 }
@@ -2248,6 +2473,7 @@ int atl_fast_plan_traj(const atl_fast_geometry* geo, const float* p, const float
   FGeo G;
   if (!plan_args_ok(geo, G, ws, ws_bytes, "fast_plan_traj")) return 1;
   const int64_t N = geo->N, M = geo->M;
+  if (is_small(geo)) { set_error("fast_plan_traj: a geometry for direct linear sums"); return 1; }
   if (K < 1 || K > kTrajPairMaxK) { set_error("fast_plan_traj: K = %lld outside 1..%d", (long long)K, kTrajPairMaxK); return 1; }
   if ((N > 0 && (!p || !coef || !tab || !t || !b)) || (M > 0 && !anchors && M != N)) { set_error("fast_plan_traj: null input"); return 1; }
   switch (K) {
@@ -2264,6 +2490,13 @@ int atl_fast_pair_fwd(const atl_fast_geometry* geo, const void* ws, float* out, 
   if (!ws || (geo->M > 0 && !out)) { set_error("fast_pair_fwd: null argument"); return 1; }
   if (geo->M == 0) return 0;
   const FPlan p = make_plan((void*)ws, geo);
+  if (is_small(geo)) {
+    const Rec *srec = p.srec, *arec = p.arec;
+    const dim3 sgrid((unsigned)((geo->M + kSmallQ - 1) / kSmallQ));
+    auto fwd = count ? k_small_fwd<true> : k_small_fwd<false>;
+    hipLaunchKernelGGL(fwd, sgrid, dim3(kSmallBlock), 0, stream, srec, (int)geo->N, arec, (int)geo->M, G, out, count);
+    return check_launch("fast_pair_fwd");
+  }
   const unsigned grid = xcd_grid((geo->M + G.apw - 1) / G.apw);
   if (count)
     hipLaunchKernelGGL(k_fast_fwd<true>, dim3(grid), dim3(kPairBlock), 0, stream, p, G, (int)geo->M, out, count);
@@ -2278,6 +2511,10 @@ int atl_fast_pair_bwd(const atl_fast_geometry* geo, void* ws, const float* gS, f
   if (!ws || (geo->N > 0 && !gv) || (geo->M > 0 && !gS)) { set_error("fast_pair_bwd: null argument"); return 1; }
   if (geo->N == 0) return 0;
   const FPlan p = make_plan(ws, geo);
+  if (is_small(geo)) {
+    launch_small_bwd(p, G, geo, gS, (float2*)gv, stream);
+    return check_launch("fast_pair_bwd");
+  }
   hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
                      (int)geo->M, gS, (int)geo->N, (float2*)gv, (float*)nullptr, 0);
   if (geo->M > 0)
@@ -2297,6 +2534,10 @@ int atl_fast_pair_bwd_src(const atl_fast_geometry* geo, void* ws, const float* g
   if (!ws || (geo->M > 0 && !gS)) { set_error("fast_pair_bwd_src: null argument"); return 1; }
   if (geo->N == 0 || geo->M == 0) return 0;
   const FPlan p = make_plan(ws, geo);
+  if (is_small(geo)) {                             // the sources' gradients where the plan keeps the slots
+    launch_small_bwd(p, G, geo, gS, slots_of<float2>(ws, geo), stream);
+    return check_launch("fast_pair_bwd_src");
+  }
   hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
                      (int)geo->M, gS, (int)geo->N, (float2*)nullptr, (float*)nullptr, 0);
   launch_entry_bwd<false>(p, G, geo, ws, stream);
@@ -2321,6 +2562,13 @@ int atl_fast_flow_adjoint(const atl_fast_geometry* geo, void* ws, int64_t Hg, in
   F.scale = img_h > 0 && img_w > 0;
   F.sxw = (float)(img_w - 1 > 1 ? img_w - 1 : 1);
   F.syh = (float)(img_h - 1 > 1 ? img_h - 1 : 1);
+  if (is_small(geo)) {
+    const int64_t ng = geo->B * 2 * Hg * Wg;
+    hipLaunchKernelGGL(k_fill_zero, dim3(grid_for(ng)), dim3(kBlock), 0, stream, (int*)ggrid, ng);
+    hipLaunchKernelGGL(k_small_adjoint, dim3(grid_for(geo->N)), dim3(kBlock), 0, stream, p.srec, (int)geo->N, F,
+                       (const float2*)slots_of<float2>(ws, geo), ggrid);
+    return check_launch("fast_flow_adjoint");
+  }
   const int64_t tiles = geo->B * ((G.GW + G.stile - 1) / G.stile) * ((G.GH + G.stile - 1) / G.stile);
   const int64_t maxc = tiles + (geo->N + kAdjChunk - 1) / kAdjChunk;   // chunks, at most (adj_scratch_bytes)
   int2* info = at_off<int2>(ws, geo->off_trec);
@@ -2348,6 +2596,7 @@ int atl_fast_pair_bwd_traj(const atl_fast_geometry* geo, void* ws, const float* 
                            const float* tab, float* gp, float* gcoef, hipStream_t stream) {
   FGeo G;
   if (!make_geo(geo, G)) { set_error("fast_pair_bwd_traj: geometry not initialised"); return 1; }
+  if (is_small(geo)) { set_error("fast_pair_bwd_traj: a geometry for direct linear sums"); return 1; }
   if (K < 1 || K > kTrajPairMaxK) { set_error("fast_pair_bwd_traj: K = %lld outside 1..%d", (long long)K, kTrajPairMaxK); return 1; }
   if (!ws || (geo->N > 0 && (!gp || !gcoef || !coef || !tab)) || (geo->M > 0 && !gS)) { set_error("fast_pair_bwd_traj: null argument"); return 1; }
   if (geo->N == 0) return 0;

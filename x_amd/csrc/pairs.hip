@@ -1189,7 +1189,7 @@ __global__ void __launch_bounds__(kBlock) k_window_counts_seq(const float* __res
   __syncthreads();
   // A block whose anchors' bounds lie far apart (its anchors cross into another batch) searches the events: the
   // thread's anchors and both bounds step together, 8 loads in flight instead of one (three windows of 84k events:
-  // 34 us, one anchor and bound after the other, as the last block of the launch; WC_AFTER us).
+  // 34 us, one anchor and bound after the other, as the last block of the launch; 30 us).
   if (!fits) {
     double lv[kWcPer], hv[kWcPer];
     int64_t l0[kWcPer], l1[kWcPer], h0[kWcPer], h1[kWcPer];

@@ -105,6 +105,7 @@ _SIGS = {
     "atl_fast_plan": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _P],
     "atl_fast_pair_fwd": [_P, _P, _P, _P, _P],
     "atl_fast_pair_bwd": [_P, _P, _P, _P, _P],
+    "atl_fast_geometry_direct": [_P],
     "atl_fast_plan_traj": [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _P],
     "atl_fast_pair_bwd_traj": [_P, _P, _P, _P, _I, _P, _P, _P, _P],
     "atl_standardise_nonzero_ws_bytes": [_I, _I],
@@ -140,7 +141,7 @@ class FastGeometry(ctypes.Structure):
     _fields_ = ([("version", ctypes.c_int32), ("bucket_shift", ctypes.c_int32)] +
                 [(n, ctypes.c_int64) for n in ("N", "M", "B", "H", "W", "S")] +
                 [(n, ctypes.c_double) for n in ("h", "tau", "cut")] +
-                [(n, ctypes.c_float) for n in ("gx0", "gy0", "gx1", "gy1", "cell", "reserved_f")] +
+                [(n, ctypes.c_float) for n in ("gx0", "gy0", "gx1", "gy1", "cell", "direct")] +
                 [(n, ctypes.c_int64) for n in ("GW", "GH", "ncell", "ncell_pad", "max_span", "ecap", "ws_bytes",
                                                "off_params", "off_cnt", "off_boff", "off_part", "off_start",
                                                "off_trec", "off_epos", "off_etim", "off_eself", "off_arec", "off_srec", "off_brec",

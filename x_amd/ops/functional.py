@@ -855,10 +855,7 @@ class FastPairPlan:
             raise ValueError("anchor_xy must be (M, 2)")
         self.N, self.M, self.device = N, M, dev
         self.geo = FastGeometry()
-        lib = load_library()
-        if lib.atl_fast_geometry_init(N, M, int(B), int(H), int(W), int(n_slices), float(h), float(tau), float(cut),
-                                      ctypes.byref(self.geo)) != 0:
-            raise HipLibraryError("atl_fast_geometry_init: " + lib.atl_last_error().decode(errors="replace"))
+        self._geometry(N, M, int(B), int(H), int(W), int(n_slices), float(h), float(tau), float(cut))
         self.ws = torch.empty(int(self.geo.ws_bytes), dtype=torch.uint8, device=dev)
         with on_device(dev):
             if self.traj:
@@ -868,6 +865,13 @@ class FastPairPlan:
             else:
                 call("atl_fast_plan", ctypes.byref(self.geo), ptr(self.x), ptr(self.t), ptr(self.v), ptr(self.b),
                      ptr(self.anchors), ptr(self.anchor_xy), ptr(self.ws), int(self.geo.ws_bytes), stream_of(self.x))
+
+    def _geometry(self, *sizes):
+        lib = load_library()
+        if lib.atl_fast_geometry_init(*sizes, ctypes.byref(self.geo)) != 0:
+            raise HipLibraryError("atl_fast_geometry_init: " + lib.atl_last_error().decode(errors="replace"))
+        if not self.traj:                # few events: every pair directly, without a plan
+            lib.atl_fast_geometry_direct(ctypes.byref(self.geo))
 
     def forward(self, count: Optional[torch.Tensor] = None) -> torch.Tensor:
         out = torch.zeros(self.M, dtype=F32, device=self.device)
