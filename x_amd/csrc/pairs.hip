@@ -158,7 +158,7 @@ __global__ void __launch_bounds__(kBlock) k_plan_fill(const float2* __restrict__
 
 // The same plan by a two-level counting sort instead of one global atomic per entry for the counts and another
 // for the cursor (k_plan_count, k_plan_fill: about 25 G scattered atomics/s on this part).  Buckets of 2^shift
-// consecutive cell keys.  Pass A (COUNT): every block of kPsPer * kPsBlock sources counts its entries per bucket
+// consecutive cell keys.  Pass A (COUNT): every block of pass_a_per * kPsBlock sources counts its entries per bucket
 // in LDS, writes the row (cnt, block-major) and adds its non-zero counts into the bucket totals; one workgroup
 // scans the totals into bucket positions.  Pass A (SCATTER): the block reserves its run of every bucket it feeds
 // with one atomic add on the bucket's position (which ends as the bucket's end) and writes one 32-byte record per
@@ -167,7 +167,10 @@ __global__ void __launch_bounds__(kBlock) k_plan_fill(const float2* __restrict__
 // cell_start (the CSR offsets of the old path, bit for bit) and writes every entry at its cell's next slot.
 // Entry order within a cell is arrival order, unspecified as before.
 constexpr int kPsBlock = 512;
-constexpr int kPsPer = 8;                          // sources per thread and pass-A block
+constexpr int kPsPer = 8;                          // sources per thread of a pass-A block, at most
+// Fewer of them where the blocks would leave CUs idle: 400k events ran 46 + 20 us in 98 blocks of eight per thread and
+// run 35 + 12 us in 391 of two (the anchors' pass A alike: 12.6 + 6.6 and 10.4 + 4.9 us).
+__host__ inline int pass_a_per(int64_t n) { return n > 786432 ? 8 : n > 524288 ? 4 : n > 196608 ? 2 : 1; }
 constexpr int kPsScanBlock = 1024;
 constexpr int kPsMaxBuckets = 16 * kPsScanBlock;
 constexpr int kPsMinShift = 7;                     // 128 cells per bucket at least: many pass-B workgroups
@@ -184,7 +187,7 @@ template <bool SCATTER>
 __global__ void __launch_bounds__(kPsBlock) k_psort_pass_a(const float2* __restrict__ x, const float* __restrict__ t,
                                                          const float2* __restrict__ v,
                                                          const int64_t* __restrict__ b, int64_t N, PlanGeo g,
-                                                         int shift, int nbuckets, int* __restrict__ cnt,
+                                                         int per, int shift, int nbuckets, int* __restrict__ cnt,
                                                          int* __restrict__ tot_or_pos, PsRec* __restrict__ rec) {
   extern __shared__ int hist[];
   const int blk = blockIdx.x;
@@ -198,13 +201,14 @@ __global__ void __launch_bounds__(kPsBlock) k_psort_pass_a(const float2* __restr
     hist[i] = h;
   }
   __syncthreads();
-  const int64_t j0 = (int64_t)blk * (kPsPer * kPsBlock) + threadIdx.x;
+  const int64_t j0 = (int64_t)blk * (per * kPsBlock) + threadIdx.x;
   // the thread's sources are read before any is binned, so that all their loads are in flight together
   int64_t bb[kPsPer];
   float tt[kPsPer];
   float2 xx[kPsPer], vv[kPsPer];
 #pragma unroll
   for (int u = 0; u < kPsPer; ++u) {
+    if (u >= per) break;
     const int64_t j = min(j0 + (int64_t)u * kPsBlock, N - 1);
     bb[u] = b[j];
     tt[u] = t[j];
@@ -214,7 +218,7 @@ __global__ void __launch_bounds__(kPsBlock) k_psort_pass_a(const float2* __restr
 #pragma unroll
   for (int u = 0; u < kPsPer; ++u) {
     const int64_t j = j0 + (int64_t)u * kPsBlock;
-    if (j >= N) break;
+    if (u >= per || j >= N) break;
     const int64_t bj = bb[u];
     if (bj < 0 || bj >= g.B) continue;
     const float tj = tt[u];
@@ -359,7 +363,8 @@ bool psort_layout(int64_t N, int64_t ecap, int64_t ncell, PsortLayout& L) {
   if (shift > kPsMaxShift) return false;
   L.shift = shift;
   L.nbuckets = (int)((ncell + ((int64_t)1 << shift) - 1) >> shift);
-  L.nblk = (int)((N + kPsPer * kPsBlock - 1) / (kPsPer * kPsBlock));
+  const int per_block = pass_a_per(N) * kPsBlock;
+  L.nblk = (int)((N + per_block - 1) / per_block);
   auto a256 = [](int64_t n) { return (n + 255) & ~(int64_t)255; };
   int64_t off = 0;
   L.cnt = off;  off += a256((int64_t)L.nblk * L.nbuckets * 4);
@@ -709,7 +714,7 @@ __global__ void __launch_bounds__(kBlock) k_anchor_place(PairRef a, int64_t M, c
 }
 
 // The same binning by a two-level counting sort (the plan's scheme: buckets of 2^shift consecutive cells): pass
-// A counts the anchors of every block of kAbPer * kAbBlock per bucket in LDS (one block-major row of counts,
+// A counts the anchors of every block of pass_a_per * kAbBlock per bucket in LDS (one block-major row of counts,
 // added into the bucket totals), one workgroup scans the totals, and pass A again reserves the block's run of
 // each bucket with one atomic add on the bucket's position and writes the anchors' records there; pass B ranks
 // each bucket's records by cell in LDS, writes the cells' CSR starts and the records at their final places.
@@ -718,7 +723,7 @@ constexpr int kAbBlock = 512;
 constexpr int kAbPer = 8;                          // anchors per thread of pass A, records per thread of pass B
 
 template <bool SCATTER>
-__global__ void __launch_bounds__(kAbBlock) k_abin_a(PairRef a, int64_t M, const float* __restrict__ gS, int shift,
+__global__ void __launch_bounds__(kAbBlock) k_abin_a(PairRef a, int64_t M, int per, const float* __restrict__ gS, int shift,
                                                      int nbuckets, int* __restrict__ cnt,
                                                      int* __restrict__ tot_or_pos, AnchorRec* __restrict__ tmp) {
   extern __shared__ int hist[];
@@ -732,7 +737,7 @@ __global__ void __launch_bounds__(kAbBlock) k_abin_a(PairRef a, int64_t M, const
     hist[i] = h;
   }
   __syncthreads();
-  const int64_t i0 = (int64_t)blockIdx.x * (kAbPer * kAbBlock) + threadIdx.x;
+  const int64_t i0 = (int64_t)blockIdx.x * (per * kAbBlock) + threadIdx.x;
   int key[kAbPer];
   float gi[kAbPer];
 #pragma unroll
@@ -740,7 +745,7 @@ __global__ void __launch_bounds__(kAbBlock) k_abin_a(PairRef a, int64_t M, const
     const int64_t i = i0 + (int64_t)u * kAbBlock;
     key[u] = -1;
     gi[u] = 0.f;
-    if (i < M) {
+    if (u < per && i < M) {
       gi[u] = gS ? gS[i] : 0.f;
       if (!(gS && gi[u] == 0.f)) key[u] = (int)anchor_key(i, a);   // -1 outside the grid
     }
@@ -1554,7 +1559,8 @@ PairWs pair_ws_layout(void* base, int64_t E, int64_t ncell, int64_t M, int64_t G
   w.fwork = (int64_t*)take(8 * atl_scan_work_size(ncell));
   w.fitems = (int2*)take(8 * w.max_fitems);
   // buckets of about kAbPer * kAbBlock / 2 anchors on average (pass B's workgroups hold up to twice that in
-  // registers), at least kPsMinShift and at most kPsMaxShift cells, and few enough for one scan workgroup
+  // registers; a quarter of that ran 28 against 25 us at 400k), at least kPsMinShift and at most kPsMaxShift cells, and
+  // few enough for one scan workgroup
   w.ab_shift = -1;
   for (int s = kPsMinShift; s <= kPsMaxShift; ++s)
     if (((ncell + ((int64_t)1 << s) - 1) >> s) <= kPsMaxBuckets &&
@@ -1563,7 +1569,8 @@ PairWs pair_ws_layout(void* base, int64_t E, int64_t ncell, int64_t M, int64_t G
       break;
     }
   w.ab_nbuckets = w.ab_shift < 0 ? 0 : (int)((ncell + ((int64_t)1 << w.ab_shift) - 1) >> w.ab_shift);
-  w.ab_nblk = (int)((M + kAbPer * kAbBlock - 1) / (kAbPer * kAbBlock));
+  const int per_block = pass_a_per(M) * kAbBlock;
+  w.ab_nblk = (int)((M + per_block - 1) / per_block);
   if (w.ab_shift >= 0) {
     w.abcnt = (int*)take(4 * (int64_t)w.ab_nblk * w.ab_nbuckets);
     w.abtot = (int*)take(4 * (int64_t)w.ab_nbuckets);
@@ -1590,11 +1597,11 @@ int bin_anchors(const PairRef& a, int64_t M, int64_t ncell, const float* gS, con
     const size_t lds = (size_t)w.ab_nbuckets * sizeof(int);
     hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(w.ab_nbuckets)), dim3(kBlock), 0, stream, w.abtot,
                        (int64_t)w.ab_nbuckets, 0);
-    hipLaunchKernelGGL(k_abin_a<false>, dim3(w.ab_nblk), dim3(kAbBlock), lds, stream, a, M, gS, w.ab_shift,
+    hipLaunchKernelGGL(k_abin_a<false>, dim3(w.ab_nblk), dim3(kAbBlock), lds, stream, a, M, pass_a_per(M), gS, w.ab_shift,
                        w.ab_nbuckets, w.abcnt, w.abtot, (AnchorRec*)nullptr);
     hipLaunchKernelGGL(k_psort_scan, dim3(1), dim3(kPsScanBlock), 0, stream, (const int*)w.abtot, w.ab_nbuckets,
                        w.abpos);
-    hipLaunchKernelGGL(k_abin_a<true>, dim3(w.ab_nblk), dim3(kAbBlock), lds, stream, a, M, gS, w.ab_shift,
+    hipLaunchKernelGGL(k_abin_a<true>, dim3(w.ab_nblk), dim3(kAbBlock), lds, stream, a, M, pass_a_per(M), gS, w.ab_shift,
                        w.ab_nbuckets, w.abcnt, w.abpos, w.abtmp);
     hipLaunchKernelGGL(k_abin_b, dim3(w.ab_nbuckets), dim3(kAbBlock), 0, stream, (const AnchorRec*)w.abtmp,
                        (const int*)w.abpos, (const int*)w.abtot, w.ab_shift, ncell, w.ab_nbuckets, (int)a.GW,
@@ -1705,11 +1712,11 @@ int atl_plan_sort(const float* x, const float* t, const float* v, const int64_t*
   const size_t lds = (size_t)L.nbuckets * sizeof(int);
   if (L.nblk > 0)
     hipLaunchKernelGGL(k_psort_pass_a<false>, dim3(L.nblk), dim3(kPsBlock), lds, stream, (const float2*)x, t,
-                       (const float2*)v, b, N, g, L.shift, L.nbuckets, cnt, tot, (PsRec*)nullptr);
+                       (const float2*)v, b, N, g, pass_a_per(N), L.shift, L.nbuckets, cnt, tot, (PsRec*)nullptr);
   hipLaunchKernelGGL(k_psort_scan, dim3(1), dim3(kPsScanBlock), 0, stream, (const int*)tot, L.nbuckets, pos);
   if (L.nblk > 0)
     hipLaunchKernelGGL(k_psort_pass_a<true>, dim3(L.nblk), dim3(kPsBlock), lds, stream, (const float2*)x, t,
-                       (const float2*)v, b, N, g, L.shift, L.nbuckets, cnt, pos, rec);
+                       (const float2*)v, b, N, g, pass_a_per(N), L.shift, L.nbuckets, cnt, pos, rec);
   hipLaunchKernelGGL(k_psort_pass_b, dim3(L.nbuckets), dim3(kPsBlock), 0, stream, (const PsRec*)rec,
                      (const int*)pos, (const int*)tot, L.shift, ncell, L.nbuckets, start, (float2*)src_y,
                      (float2*)src_v, src_t, src_id);
