@@ -479,6 +479,9 @@ int atl_lut_table_fwd(const float* tr, int64_t B, int64_t T, int64_t n, double x
 int atl_lut_table_bwd(const float* gtable, int64_t B, int64_t T, int64_t n, double x0, double y0, double step,
                       int64_t nx, int64_t ny, int64_t k, const void* ws, int64_t ws_bytes, float* gtr,
                       hipStream_t stream);
+/* Basis table of the trajectory pair sums: out (S, 2K) rows [g_1..g_K(c_s), g_1'..g_K'(c_s)] at c_s = (s + 1/2) / S,
+ * evaluated in fp64; basis as atl_traj_displacement's, K <= 16. */
+int atl_slice_table(int64_t S, int64_t K, int64_t basis, float* out, hipStream_t stream);
 /* Positions (B, nt, Hq * Wq, 2) of every tile trajectory at nt times (atl/motion/trajectories.py:88-97): coef
  * (B, 2K, Hq, Wq) with element strides sb, sc, sy, sx; tile centres tile * i + offset; basis as
  * atl_traj_displacement's.  nt K <= 4096.  The backward writes gcoef (B, 2K, Hq, Wq) contiguous. */

@@ -779,3 +779,14 @@ def _splat64_one(y, w, H, W):
             if 0 <= x0 + dx < W and 0 <= y0 + dy < H:
                 img[y0 + dy, x0 + dx] += w * wx * wy
     return img
+
+
+@pytest.mark.parametrize("K,kind,S", [(1, "bspline", 16), (2, "bspline", 1), (3, "bezier", 5), (10, "bspline", 16),
+                                      (16, "polynomial", 64), (16, "bezier", 65), (12, "bspline", 1000)])
+def test_slice_table_matches_the_host_table(K, kind, S):
+    from x_amd.motion import PixelTrajectories
+    c = torch.zeros(1, 2 * K, 4, 5)
+    want = PixelTrajectories(c, K, kind, tile=1).slice_tables(S, "cpu")
+    got = PixelTrajectories(c.to(DEV), K, kind, tile=1).slice_tables(S, DEV).cpu()
+    # both round an fp64 value once; the last fp32 bit may differ where that value lies at a tie
+    assert (got - want).abs().max() <= 2.0 ** -23 * want.abs().max()

@@ -711,6 +711,66 @@ __global__ void __launch_bounds__(kBlock) k_traj_displacement(const float4* __re
   if (live && q == 0) out[n] = make_float2(sx, sy);
 }
 
+// Rows [g_1..g_K(c_s), g_1'..g_K'(c_s)] of the basis at the slice centres c_s = (s + 1/2) / S (fp32, as the pair kernels
+// compute them), evaluated in fp64 by the formulas of the model's host table (basis_table) and rounded once; one thread
+// per slice and function.  The host's table came with a copy from pageable memory, which waits for the GPU: a step of 4
+// windows of 500k events held the host for 9.5 ms, now 0.9 ms, and left the device idle behind it.
+constexpr int kTableMaxK = 16;
+
+__global__ void __launch_bounds__(kWave) k_slice_table(int S, int K, int basis, float* __restrict__ out) {
+  const int id = blockIdx.x * kWave + threadIdx.x;
+  const int s = id / K, k = id - s * K + 1;
+  if (s >= S) return;
+  const double t = (double)(((float)s + 0.5f) * (float)(1.0 / (double)S));
+  double val, der;
+  if (basis == 2) {
+    // Cox and de Boor over the functions k .. k + P that N_k,P is made of; knots u_i = clip(i - P, 0, L) / L
+    const int P = K < 3 ? K : 3, L = K + 1 - P;
+    auto knot = [&](int i) { return (double)min(max(i - P, 0), L) / (double)L; };
+    const int j = min(max((int)floor(t * L), 0), L - 1);
+    double n[4], low0 = 0.0, low1 = 0.0;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) n[d] = k + d == j + P ? 1.0 : 0.0;
+#pragma unroll
+    for (int q = 1; q <= 3; ++q) {
+      if (q > P) break;
+      if (q == P) { low0 = n[0]; low1 = n[1]; }      // N_k and N_k+1 of degree P - 1
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        if (d > P - q) break;
+        const int i = k + d;
+        const double a = knot(i + q) - knot(i), c = knot(i + q + 1) - knot(i + 1);
+        double v = 0.0;
+        if (a > 0) v += (t - knot(i)) / a * n[d];
+        if (c > 0) v += (knot(i + q + 1) - t) / c * n[d + 1];
+        n[d] = v;
+      }
+    }
+    val = n[0];
+    const double a = knot(k + P) - knot(k), c = knot(k + P + 1) - knot(k + 1);
+    der = 0.0;
+    if (a > 0) der += low0 / a;
+    if (c > 0) der -= low1 / c;
+    der *= P;
+  } else {
+    auto power = [](double x, int e) {
+      double r = 1.0;
+      for (int i = 0; i < e; ++i) r *= x;
+      return r;
+    };
+    auto bern = [&](int n, int i) {
+      if (i < 0 || i > n) return 0.0;
+      double b = 1.0;
+      for (int q = 1; q <= i; ++q) b = b * (n - i + q) / q;
+      return b * power(t, i) * power(1.0 - t, n - i);
+    };
+    val = basis == 0 ? power(t, k) : bern(K, k);
+    der = basis == 0 ? k * power(t, k - 1) : K * (bern(K - 1, k - 1) - bern(K - 1, k));
+  }
+  out[(int64_t)s * 2 * K + k - 1] = (float)val;
+  out[(int64_t)s * 2 * K + K + k - 1] = (float)der;
+}
+
 // Positions of every tile trajectory at nt times (PixelTrajectories.tile_trajectories): out (B, nt, n, 2) = tile
 // centre + sum_k c_k g_k(t), the coefficients read through the strides of the tile-centre view (B, 2K, Hq, Wq).
 // One thread per trajectory and group of kTileTimes times (blockIdx.y), so that 19200 trajectories still give 300
@@ -1438,6 +1498,17 @@ int atl_traj_displacement(const float* field_cl, int64_t B, int64_t C, int64_t K
 #undef ATL_TRAJ_CASE
   }
   return check_launch("traj_displacement");
+}
+
+int atl_slice_table(int64_t S, int64_t K, int64_t basis, float* out, hipStream_t stream) {
+  if (S < 0 || S > ((int64_t)1 << 24) || K < 1 || K > kTableMaxK || basis < 0 || basis > 2) {
+    set_error("slice_table: bad sizes (1 <= K <= %d, basis 0, 1 or 2)", kTableMaxK);
+    return 1;
+  }
+  if (S == 0) return 0;
+  if (!out) { set_error("slice_table: null argument"); return 1; }
+  hipLaunchKernelGGL(k_slice_table, dim3(grid_for(S * K, kWave)), dim3(kWave), 0, stream, (int)S, (int)K, (int)basis, out);
+  return check_launch("slice_table");
 }
 
 static int tile_traj_bad(const char* what, int64_t B, int64_t K, int64_t Hq, int64_t Wq, int64_t nt, int64_t basis) {

@@ -1518,8 +1518,10 @@ __device__ __forceinline__ EntSum<TRAJ> entry_sum(const FPlan& p, const FGeo& G,
   const int plane = pl * (G.GH * G.GW);
   const float cs = slice_centre(sl, G.delta);
   float g0 = 0.f, g1 = 0.f, g2 = 0.f, g3 = 0.f;
-  // one pair; `other` folds in the caller's own conditions
-  auto term = [&](const float4& A, bool other) {
+  // one pair; `other` folds in the caller's own conditions.  FIN: every record and the entry are finite and below 1e30
+  // (checked), so a zero factor adds exactly nothing and one select does for all sums.
+  auto term = [&](const float4& A, bool other, auto fin) {
+    constexpr bool FIN = decltype(fin)::value;
     const float at = A.z - cs;
     const float dt = A.z - tj;
     const float rx = A.x - (sv.x + sv.z * at);
@@ -1528,7 +1530,17 @@ __device__ __forceinline__ EntSum<TRAJ> entry_sum(const FPlan& p, const FGeo& G,
     const bool ok = other & !(fabsf(dt) > G.tau) & !(d2 > G.r2max);
     const float kern = __builtin_amdgcn_exp2f(d2 * G.kexp);
     if (TRAJ) {
-      const float f = A.w * kern;                    // A.w = gS / h^2
+      float f = A.w * kern;                          // A.w = gS / h^2
+      if (FIN) {
+        f = ok ? f : 0.f;
+        asm volatile("" : "+v"(f));                  // keep one select (not folded into the four sums)
+        const float fx = f * rx, fy = f * ry;
+        g0 = g0 + fx;
+        g1 = g1 + fy;
+        g2 = fmaf(fx, at, g2);
+        g3 = fmaf(fy, at, g3);
+        return;
+      }
       const float fx = f * rx, fy = f * ry;
       g0 = ok ? g0 + fx : g0;                        // selects: a record may hold anything, NaN included
       g1 = ok ? g1 + fy : g1;
@@ -1536,8 +1548,8 @@ __device__ __forceinline__ EntSum<TRAJ> entry_sum(const FPlan& p, const FGeo& G,
       g3 = ok ? fmaf(fy, at, g3) : g3;
     } else {
       const float f = A.w * kern * dt;
-      if (!LOO) {                                    // every record and the entry are finite and below 1e30
-        float fo = ok ? f : 0.f;                     // (checked), so a zero factor adds exactly nothing
+      if (FIN) {
+        float fo = ok ? f : 0.f;
         asm volatile("" : "+v"(fo));                 // keep one select (not folded into two after the FMAs)
         g0 = fmaf(fo, rx, g0);
         g1 = fmaf(fo, ry, g1);
@@ -1597,7 +1609,7 @@ __device__ __forceinline__ EntSum<TRAJ> entry_sum(const FPlan& p, const FGeo& G,
       __syncthreads();
       for (int i = 0; i < n; i += 4) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) term(sA[i + u], LOO ? sI[i + u] != pos : true);
+        for (int u = 0; u < 4; ++u) term(sA[i + u], LOO ? sI[i + u] != pos : true, std::true_type{});
       }
     });
   } else if (active) {
@@ -1618,7 +1630,7 @@ __device__ __forceinline__ EntSum<TRAJ> entry_sum(const FPlan& p, const FGeo& G,
       }
       const int rem = e - k;
 #pragma unroll
-      for (int u = 0; u < U; ++u) term(A[u], (u < rem) & (LOO ? own[u] != pos : true));
+      for (int u = 0; u < U; ++u) term(A[u], (u < rem) & (LOO ? own[u] != pos : true), std::bool_constant<!LOO>{});
     });
   }
   if constexpr (TRAJ)

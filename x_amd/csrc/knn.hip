@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(kBlock) k_knn_query(const float2* __restrict__
 // order: a query first brackets its k-th distance, counting its candidates under seven thresholds at a time (14
 // instructions a candidate, nothing kept), then adds up the points under the bracket and picks the few inside it by
 // (distance, index).  The sorted insertion of k_knn_query costs 350 instructions a candidate, and took 560 us for 15
-// planes of 19200 points, k = 32; with the bracketing the whole forward takes 164 us on an even point set and 237 us
+// planes of 19200 points, k = 32; with the bracketing the whole forward takes 149 us on an even point set and 211 us
 // where trajectories of up to 25 px leave parts of the sensor empty (picking the bracket's points one pass each
 // instead of kPick a pass: 190 and 267 us).  One thread per query, a wave on an 8 x 8 patch,
 // so that its lanes read the same cells.
@@ -222,6 +222,7 @@ __global__ void __launch_bounds__(kBlock) k_knn_query(const float2* __restrict__
 // each block, so that a point tests about ten blocks (61 us; 88 us with a gradient loaded per taken query; torch's
 // scatter of 9.2M rows through atomics took 180 us, and the gather and mean forward another 130).
 constexpr int kQB = 4;                           // queries per block side
+constexpr int kQStep = 8;                        // candidates a query reads at once (2: 238, 4: 216, 8: 211 us)
 constexpr int kPick = 4;                         // points picked from the bracket in one pass
 constexpr int kPatch = 16;                       // queries per workgroup side: 4 waves of 8 x 8
 
@@ -309,14 +310,17 @@ __global__ void __launch_bounds__(kBlock) k_lut_query(float x0, float y0, float 
   if (live) {
     const int qcx = cell_of(qx, g.ox, g.icx, g.GX), qcy = cell_of(qy, g.oy, g.icy, g.GY);
     const float slack = 1e-4f * (g.csx + g.csy) + 1e-5f * (fabsf(g.ox) + fabsf(g.oy) + fabsf(qx) + fabsf(qy));
-    // f(d, slot) over the points of a row range of cells, two loads in flight
+    // f(d, slot) over the points of a row range of cells, kQStep loads in flight
     auto row = [&](int b, int e, auto&& f) {
-      for (int t = b; t < e; t += 2) {
-        const int t2 = min(t + 1, e - 1);
-        const float2 p = xy[(uint32_t)t], p2 = xy[(uint32_t)t2];
-        const float dx = qx - p.x, dy = qy - p.y, dx2 = qx - p2.x, dy2 = qy - p2.y;
-        f(dx * dx + dy * dy, t);
-        if (t2 != t) f(dx2 * dx2 + dy2 * dy2, t2);
+      for (int t = b; t < e; t += kQStep) {
+        float2 p[kQStep];
+#pragma unroll
+        for (int u = 0; u < kQStep; ++u) p[u] = xy[(uint32_t)min(t + u, e - 1)];
+#pragma unroll
+        for (int u = 0; u < kQStep; ++u) {
+          const float dx = qx - p[u].x, dy = qy - p[u].y;
+          if (t + u < e) f(dx * dx + dy * dy, t + u);
+        }
       }
     };
     // over every cell that can hold a point closer than sqrt(hi): a point can be binned one rounding away

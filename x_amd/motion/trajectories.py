@@ -25,7 +25,7 @@ import math
 import numpy as np
 import torch
 
-from ..ops.functional import TRAJ_BASES, TRAJ_MAX_K, _tile_plan_ok, tile_trajectories, traj_displacement, traj_origin
+from ..ops.functional import TRAJ_BASES, TRAJ_MAX_K, _tile_plan_ok, slice_table, tile_trajectories, traj_displacement, traj_origin
 from .base import Motion, as_time
 from .parametric import sample_grid
 
@@ -213,6 +213,8 @@ class PixelTrajectories(Motion):
     def slice_tables(self, n_slices: int, device) -> torch.Tensor:
         """(S, 2K) float32 table of the basis at the slice centres c_s = (s + 1/2) / S (fp32, as the pair kernels
         compute them): row s = [g_1..g_K(c_s), g_1'..g_K'(c_s)], evaluated in float64."""
+        if torch.device(device).type == "cuda" and self.K <= TRAJ_MAX_K and n_slices > 0:
+            return slice_table(n_slices, self.K, self.basis_kind, device)   # no copy that waits for the device
         cs = (np.arange(n_slices, dtype=np.float32) + np.float32(0.5)) * np.float32(1.0 / n_slices)
         val, der = basis_table(cs.astype(np.float64), self.K, self.basis_kind)
         return torch.as_tensor(np.concatenate([val, der], 1).astype(np.float32), device=device)

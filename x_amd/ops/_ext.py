@@ -114,6 +114,7 @@ _SIGS = {
     "atl_lut_table_ws_bytes": [_I, _I, _I, _I, _I],
     "atl_lut_table_fwd": [_P, _I, _I, _I, _D, _D, _D, _I, _I, _I, _P, _P, _I, _P],
     "atl_lut_table_bwd": [_P, _I, _I, _I, _D, _D, _D, _I, _I, _I, _P, _I, _P, _P],
+    "atl_slice_table": [_I, _I, _I, _P, _P],
     "atl_tile_trajectories": [_P, _I, _I, _I, _I, _I, _I, _I, _I, _D, _I, _P, _I, _I, _P, _P],
     "atl_tile_trajectories_bwd": [_P, _I, _I, _I, _I, _P, _I, _I, _P, _P],
     "atl_voxel_ws_bytes": [_I, _I, _I, _I, _I],

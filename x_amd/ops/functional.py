@@ -1413,6 +1413,14 @@ def tile_trajectories(coef: torch.Tensor, times: torch.Tensor, K: int, kind: str
     return _TileTrajectories.apply(coef, times.contiguous(), int(K), kind, float(offset), int(tile))
 
 
+def slice_table(n_slices: int, K: int, kind: str, device) -> torch.Tensor:
+    """(S, 2K) basis values and derivatives at the slice centres, evaluated in fp64 on the device."""
+    out = torch.empty(int(n_slices), 2 * int(K), dtype=F32, device=device)
+    with on_device(out.device):
+        call("atl_slice_table", int(n_slices), int(K), TRAJ_BASES[kind], ptr(out), stream_of(out))
+    return out
+
+
 def lut_table_torch(tr: torch.Tensor, centres: torch.Tensor, k: int) -> torch.Tensor:
     """(B, T, Q, 2) mean displacement (row 0 of ``tr`` (B, 1 + T, n, 2) minus row 1 + s) of the k points of bin s
     nearest to each centre (Q, 2), as torch operations on knn_indices' choice (atl/objectives/mpcm.py:67-77)."""
