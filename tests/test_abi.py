@@ -68,3 +68,14 @@ def test_workspace_and_trajectory_entries_reject_before_launch(lib):
     assert rc == 1 and b"expected 2K" in L.atl_last_error()
     rc = L.atl_traj_origin_bwd(None, 1, 8, 4, 8, 8, None, None, None, 5, 0, 1, None, None, None, None)
     assert rc == 1 and b"traj_origin_bwd" in L.atl_last_error()
+
+
+def test_pair_geometry_refuses_what_32_bit_offsets_cannot_reach(lib):
+    from x_amd.ops import _ext
+    L = _ext.load_library()
+    most = (1 << 28) - 64                          # anchor records of 16 bytes within 4 GiB, and the walks' padding
+    for m, ok in ((most, True), (most + 1, False)):
+        g = _ext.FastGeometry()
+        rc = L.atl_fast_geometry_init(16, m, 1, 40, 48, 1, 1.0, 0.2, 3.0, ctypes.byref(g))
+        assert (rc == 0) == ok, m
+        assert ok or b"too large" in L.atl_last_error()

@@ -355,3 +355,29 @@ def test_direct_sums_end_at_their_limits():
         a = torch.zeros(m, dtype=torch.int64, device=DEV)
         p = F.FastPairPlan(x, x[:, 0], x, a.new_zeros(n), 1, 40, 48, a, 1.0, 0.2)
         assert (p.geo.direct != 0) == direct
+
+
+def test_entries_past_32_bit_offsets():
+    """A second window whose entries stand behind 2^28 others of 16 bytes (byte offsets past 32 bits): its sums, counts
+    and gradients are those of the window alone."""
+    n0, n1, H, W, h, tau, S = 1 << 24, 3000, 512, 512, 1.0, 1.0, 16
+    print(f"entries past 32-bit offsets: {n0 * S} in front", flush=True)
+    rng = np.random.default_rng(8)
+    xs = (rng.random((n1, 2)) * 40 + 200).astype(F32)
+    t = np.sort(rng.random(n1)).astype(F32)
+    v = (rng.normal(size=(n1, 2)) * 4).astype(F32)
+    p = O.build_pair_plan(xs, t, v, np.zeros(n1, np.int64), 1, H, W, np.arange(n1), h, tau, 3.0, S)
+    want, wcnt = O.ats_pair_fwd(p, h, tau, 3.0, with_counts=True)
+    gS = rng.normal(size=n1).astype(F32)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    x_all = torch.cat([torch.rand(n0, 2, device=DEV, generator=gen) * H, T(xs)])
+    t_all = torch.cat([torch.rand(n0, device=DEV, generator=gen), T(t)])
+    v_all = torch.cat([torch.zeros(n0, 2, device=DEV), T(v)])
+    b_all = torch.cat([torch.zeros(n0, dtype=torch.int64, device=DEV), torch.ones(n1, dtype=torch.int64, device=DEV)])
+    anchors = torch.arange(n0, n0 + n1, device=DEV)
+    plan = F.FastPairPlan(x_all, t_all, v_all, b_all, 2, H, W, anchors, h, tau, 3.0, S)
+    assert np.array_equal(N(plan.counts()), wcnt)
+    assert_sums_close(N(plan.forward()), want)
+    gv = plan.backward(T(gS))
+    close_rel(N(gv[n0:]), O.ats_pair_bwd(gS, p, h, tau, 3.0, n1), 1e-4)
+    assert not gv[:n0].any()

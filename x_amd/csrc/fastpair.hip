@@ -45,6 +45,7 @@ namespace {
 constexpr int kMinBucketShift = 10;
 constexpr int kMaxBucketShift = 13;
 constexpr int kMaxBuckets = 16384;
+constexpr int64_t kMaxAnchors = ((int64_t)1 << 28) - 64;   // the backward reads their records through ld
 static_assert(kMaxBuckets <= kScanSmallMax, "bucket totals are scanned by one workgroup");
 constexpr int kSortBlock = 512;                    // pass-2 workgroup
 constexpr int kP1Block = 1024;                     // pass-1 workgroup
@@ -137,7 +138,8 @@ __device__ __forceinline__ int cell_walk(float p, float lo, float hi, float icf,
 }
 
 // Element i of an array through a 32-bit byte offset from a uniform base (lets the compiler use the
-// scalar-base + vector-offset addressing form instead of per-lane 64-bit address arithmetic).
+// scalar-base + vector-offset addressing form instead of per-lane 64-bit address arithmetic): the array
+// holds less than 4 GiB (kMaxAnchors records of 16 bytes).
 template <typename T>
 __device__ __forceinline__ T ld(const T* base, uint32_t i) {
   return *(const T*)((const char*)base + i * (uint32_t)sizeof(T));
@@ -1207,8 +1209,8 @@ __device__ __forceinline__ void fwd_pass(const FPlan& p, const FGeo& G, int plan
     float t;
   };
   auto load = [&](int pos) {
-    const uint32_t k = (uint32_t)max(pos, 0);
-    return Cand{ld(p.epos, k), ld((const float*)p.etq, 2 * k)};
+    const uint32_t k = (uint32_t)max(pos, 0);     // not ld: the entries may fill more than 4 GiB
+    return Cand{p.epos[k], p.etq[k].x};
   };
   // The walk covers the R-neighbourhood of the box of these anchors' clamped positions (tighter than their
   // cells' box: every contributing candidate lies within R of its anchor, and clamping never increases a
@@ -1311,8 +1313,8 @@ __device__ __forceinline__ void fwd_common(const FPlan& p, const FGeo& G, int pl
     float t;
   };
   auto load = [&](int k) {
-    const uint32_t i = (uint32_t)max(k, 0);
-    return Cand{ld(p.epos, i), ld((const float*)p.etq, 2 * i)};
+    const uint32_t i = (uint32_t)max(k, 0);       // not ld: the entries may fill more than 4 GiB
+    return Cand{p.epos[i], p.etq[i].x};
   };
   float acc = 0.f;
   int cnt = 0;
@@ -2330,9 +2332,10 @@ int atl_fast_geometry_init(int64_t N, int64_t M, int64_t B, int64_t H, int64_t W
   const int spb = src_per_block(N);
   const double nblk = std::ceil((double)N / spb) + std::ceil((double)M / (2 * spb));
   // GW, GH < 32768: anchor records pack (cy, cx) into 16-bit halves
-  if (3 * ncell_pad + 1 >= 2.0e9 || ecap + M + N >= 2.0e9 || nbuckets > kMaxBuckets || nbuckets * nblk + 1 >= 2.0e9 ||
+  if (3 * ncell_pad + 1 >= 2.0e9 || ecap + M + N >= 2.0e9 || M > kMaxAnchors || nbuckets > kMaxBuckets || nbuckets * nblk + 1 >= 2.0e9 ||
       g.GW >= 32768 || g.GH >= 32768) {
-    set_error("fast_geometry_init: problem too large for the 32-bit plan (cells %.0f, entries %.0f)", ncell, ecap);
+    set_error("fast_geometry_init: problem too large for the 32-bit plan (cells %.0f, entries %.0f, anchors %lld)", ncell,
+              ecap, (long long)M);
     return 1;
   }
   g.bucket_shift = shift;
