@@ -381,3 +381,39 @@ def test_entries_past_32_bit_offsets():
     gv = plan.backward(T(gS))
     close_rel(N(gv[n0:]), O.ats_pair_bwd(gS, p, h, tau, 3.0, n1), 1e-4)
     assert not gv[:n0].any()
+
+
+def _crowd(B=3, per=47_001, H=60, W=72, seed=4):
+    """Windows of events in two dense spots and a little noise, enough of them that the forward takes 16 anchors a wave."""
+    rng = np.random.default_rng(seed)
+    n = B * per
+    x = np.where(rng.random((n, 1)) < 0.5, [20.0, 25.0], [50.0, 30.0]) + 5 * rng.normal(size=(n, 2))
+    x = np.where(rng.random((n, 1)) < 0.1, rng.random((n, 2)) * [W, H], x).astype(F32)
+    t = np.sort(rng.random((B, per)).astype(F32), 1).ravel()
+    v = (rng.normal(size=(n, 2)) * 6).astype(F32)
+    return x, t, v, np.repeat(np.arange(B), per), B, H, W
+
+
+def test_crowd_of_many_anchors_matches_oracle():
+    x, t, v, b, B, H, W = _crowd()
+    xa = (x + np.random.default_rng(5).normal(size=x.shape)).astype(F32)
+    cnt = check_against_oracle(x, t, v, b, B, H, W, np.arange(len(t)), xa, 1.0, 0.05, 16)
+    assert cnt.mean() > 50
+
+
+def test_crowd_with_velocities_that_are_not_finite():
+    """Anchors taken 16 at a time from a common neighbourhood meet the same sources as in the passes of smaller anchor
+    sets, those of NaN, infinite and huge velocities among them (a NaN distance counts as a visit)."""
+    x, t, v, b, B, H, W = _crowd()
+    n, per = len(t), len(t) // B
+    v[per + 11], v[per + 30_000], v[2 * per + 7], v[2 * per + 8] = [np.nan, 0], [0, np.nan], [np.inf, 0], [1e31, -1e31]
+    print(f"crowd with wild velocities n={n}", flush=True)
+    run = lambda a: F.FastPairPlan(T(x), T(t), T(v), T(b), B, H, W, T(a), 1.0, 0.05, 3.0, 16)  # noqa: E731
+    parts = [run(a) for a in np.array_split(np.arange(n), 2)]      # below the count that takes 16 anchors a wave
+    cnt, want = (np.concatenate([N(f(p)) for p in parts]) for f in (lambda p: p.counts(), lambda p: p.forward()))
+    plan = run(np.arange(n))
+    assert np.isnan(want).any() and np.isfinite(want).mean() > 0.3
+    assert np.array_equal(N(plan.counts()), cnt)
+    got, fin = N(plan.forward()), np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fin)
+    assert_sums_close(got[fin], want[fin])

@@ -1267,8 +1267,9 @@ __device__ __forceinline__ float wave_ext(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
-// Finite and small enough that products of two such values stay finite.
-__device__ __forceinline__ bool bounded(float v) { return fabsf(v) < 1e30f; }
+// Finite and small enough that a product of two such values stays finite.
+constexpr float kBounded = 1e30f;
+__device__ __forceinline__ bool bounded(float v) { return fabsf(v) < kBounded; }
 
 // A wave takes kAnchorsPerWave consecutive anchors (lanes past them hold copies and idle through the group loop;
 // every lane takes candidates in the walks).  The wave's time follows the density around its anchors, and
@@ -1319,11 +1320,13 @@ __device__ __forceinline__ void fwd_common(const FPlan& p, const FGeo& G, int pl
   float acc = 0.f;
   int cnt = 0;
   group_walk(p.start, 0, plane, x0, x1, y0, y1, R, R2, G, load, [&](const Cand& c, int k) {
-    // the candidate's positions at the anchors' times; a NaN compares to "keep", as the pair tests would visit it
+    // the candidate's positions at the anchors' times.  One that is not bounded is kept: the pair tests decide (its
+    // distances may be NaN, which counts as a visit), and fmaxf would drop its NaN here.
     const float px0 = c.e.z * a0, px1 = c.e.z * a1, py0 = c.e.w * a0, py1 = c.e.w * a1;
     const float ex = fmaxf(fmaxf(x0 - (c.e.x + fmaxf(px0, px1)), (c.e.x + fminf(px0, px1)) - x1), 0.f);
     const float ey = fmaxf(fmaxf(y0 - (c.e.y + fmaxf(py0, py1)), (c.e.y + fminf(py0, py1)) - y1), 0.f);
-    const bool keep = (k >= 0) & !(ex * ex + ey * ey > cr2);
+    const bool wild = !(fabsf(c.e.x) + fabsf(c.e.y) + fabsf(c.e.z) + fabsf(c.e.w) < kBounded);
+    const bool keep = (k >= 0) & (wild | !(ex * ex + ey * ey > cr2));
     const uint64_t m = __ballot(keep);
     const int n = __popcll(m);
     __syncthreads();                               // one wave: the last chunk's reads are done
@@ -1399,7 +1402,7 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
   if (n == kAnchorsPerWave) {                    // anchors close together, in one plane: all of them at once
     const int cell = (ai.w >> 16) * G.GW + (ai.w & 0xffff);
     const int plane = uni(key - cell);
-    const bool plain = key - cell == plane && bounded(A.x) && bounded(A.y) && clampf(A.x, G.gx0, G.gx1) == A.x &&
+    const bool plain = key - cell == plane && bounded(A.x) && bounded(A.y) && bounded(A.w) && clampf(A.x, G.gx0, G.gx1) == A.x &&
                        clampf(A.y, G.gy0, G.gy1) == A.y;
     if (__ballot(!plain) == 0) {
       const float x0 = wave_ext<false>(A.x), x1 = wave_ext<true>(A.x);
