@@ -417,3 +417,26 @@ def test_crowd_with_velocities_that_are_not_finite():
     got, fin = N(plan.forward()), np.isfinite(want)
     assert np.array_equal(np.isfinite(got), fin)
     assert_sums_close(got[fin], want[fin])
+
+
+def test_backward_with_products_past_the_float_range():
+    """A pair that no test admits adds nothing, also where its velocity times its time offset is past the float range."""
+    rng = np.random.default_rng(6)
+    n, H, W = 400, 40, 48
+    x = (rng.random((n, 2)) * [W, H]).astype(F32)
+    t = np.sort(rng.random(n)).astype(F32)
+    v = (rng.normal(size=(n, 2)) * 4).astype(F32)
+    t[-1], t[-2] = 1e10, 0.97                      # an anchor far past the window, in the last slice with the others
+    v[-2], v[-5] = [9e29, 0], [1e25, -1e29]
+    print("products past the float range", flush=True)
+    gS = rng.normal(size=n).astype(F32)
+    run = lambda cls: N(cls(T(x), T(t), T(v), T(np.zeros(n, np.int64)), 1, H, W, None, 1.0, 0.2, 3.0, 16).backward(T(gS)))  # noqa: E731
+    got, want = run(_PlannedSums), run(F.FastPairPlan)   # the direct sums select every term
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    close_rel(got, want, 1e-4)
+    coef = np.zeros((n, 2), F32)                   # K = 1: the displacement grows linearly in time
+    coef[:, 0], coef[:, 1] = v[:, 1], v[:, 0]
+    from x_amd.motion import PixelTrajectories
+    tab = PixelTrajectories(torch.zeros(1, 2, 4, 5), 1, "polynomial", tile=1).slice_tables(16, DEV)
+    p = F.FastPairPlan(T(x), T(t), None, T(np.zeros(n, np.int64)), 1, H, W, None, 1.0, 0.2, 3.0, 16, T(x), traj=(T(coef), 1, tab))
+    assert all(bool(torch.isfinite(g).all()) for g in p.backward_traj(T(gS)))

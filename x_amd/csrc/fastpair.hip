@@ -1267,8 +1267,8 @@ __device__ __forceinline__ float wave_ext(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
-// Finite and small enough that a product of two such values stays finite.
-constexpr float kBounded = 1e30f;
+// Finite and small enough that a product of two such values stays finite (1e36 and its sums, below 3.4e38).
+constexpr float kBounded = 1e18f;
 __device__ __forceinline__ bool bounded(float v) { return fabsf(v) < kBounded; }
 
 // A wave takes kAnchorsPerWave consecutive anchors (lanes past them hold copies and idle through the group loop;
@@ -1523,8 +1523,8 @@ __device__ __forceinline__ EntSum<TRAJ> entry_sum(const FPlan& p, const FGeo& G,
   const int plane = pl * (G.GH * G.GW);
   const float cs = slice_centre(sl, G.delta);
   float g0 = 0.f, g1 = 0.f, g2 = 0.f, g3 = 0.f;
-  // one pair; `other` folds in the caller's own conditions.  FIN: every record and the entry are finite and below 1e30
-  // (checked), so a zero factor adds exactly nothing and one select does for all sums.
+  // one pair; `other` folds in the caller's own conditions.  FIN: every record and the entry are bounded (checked), so
+  // that v at, the offsets and A.w kern dt are finite and a zero factor adds exactly nothing and one select does for all sums.
   auto term = [&](const float4& A, bool other, auto fin) {
     constexpr bool FIN = decltype(fin)::value;
     const float at = A.z - cs;
