@@ -203,3 +203,17 @@ def test_tile_trajectories_match_torch(K, tile, kind, nt):
     # the basis to a few ulp of its recursions, K (nt) additions, positions up to 40 px
     assert (p0 - p1).abs().max() <= (K + 8) * 2.0 ** -23 * (coef.abs().max() * 4 + 40)
     assert (g0 - g1).abs().max() <= (nt + 8) * 2.0 ** -23 * (gout.abs().max() * nt ** 0.5 * 4)
+
+
+def test_tile_trajectories_and_table_take_batched_gradients():
+    """Several gradients at once through the backward (is_grads_batched: vmap over it), as the torch operations allow."""
+    from x_amd.motion import PixelTrajectories
+    from x_amd.objectives import MotionPriorCMaxLoss
+    coef = _smooth_coeffs(1, 8, 41, 54, 3, 9.0).to(DEV).requires_grad_(True)
+    obj = MotionPriorCMaxLoss(num_bins=3, num_knn=5)
+    m = PixelTrajectories(coef, 4, "bspline", tile=4)
+    for out in (m.tile_trajectories(torch.rand(5, device=DEV)), obj.lut_flow(m, 41, 54, torch.tensor(0.3, device=DEV))[0]):
+        g = torch.randn(3, *out.shape, device=DEV)
+        got, = torch.autograd.grad(out, coef, g, retain_graph=True, is_grads_batched=True)
+        want = torch.stack([torch.autograd.grad(out, coef, gi, retain_graph=True)[0] for gi in g])
+        assert (got - want).abs().max() <= 1e-5 * want.abs().max()     # fp32 sums of some hundred terms

@@ -1362,9 +1362,10 @@ TILE_TABLE_MAX = 4096
 
 def _plain_device(*ts) -> bool:
     """Whether a fused op that replaces a chain of torch operations may take these tensors: plain fp32 device tensors,
-    and no transform or mode at work that has to see the operations themselves (tracing, torch.func, forward-mode
-    derivatives, autocast's casts, dispatch modes)."""
-    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == F32 for t in ts)
+    and no transform or mode at work that has to see the operations themselves (tracing, torch.func, batched gradients,
+    forward-mode derivatives, autocast's casts, dispatch modes)."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == F32 and torch._C._has_storage(t)
+                for t in ts)
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
             and not torch.is_autocast_enabled("cuda") and torch._C._len_torch_dispatch_stack() == 0)
@@ -1372,7 +1373,8 @@ def _plain_device(*ts) -> bool:
 
 class _TileTrajectories(torch.autograd.Function):
     """PixelTrajectories.tile_trajectories (atl/motion/trajectories.py:88-97) in one kernel each way.  A backward that
-    is itself differentiated runs as the torch expression of the adjoint."""
+    is itself differentiated, or whose gradient comes batched (is_grads_batched) or otherwise transformed, runs as the
+    torch expression of the adjoint."""
 
     @staticmethod
     def forward(ctx, coef, times, K, kind, offset, tile):
@@ -1390,9 +1392,9 @@ class _TileTrajectories(torch.autograd.Function):
     def backward(ctx, g):
         times, = ctx.saved_tensors
         B, K, Hq, Wq = ctx.shape
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not _plain_device(g):
             from ..motion.trajectories import basis
-            gc = torch.einsum("tk,btnc->bckn", basis(times, K, ctx.kind), g).flip(1)
+            gc = torch.matmul(g.permute(0, 3, 2, 1), basis(times, K, ctx.kind)).transpose(2, 3).flip(1)   # (B, 2, K, n)
             return gc.reshape(B, 2 * K, Hq, Wq), None, None, None, None, None
         g = g.contiguous()
         gc = torch.empty(B, 2 * K, Hq, Wq, device=g.device, dtype=F32)
@@ -1435,7 +1437,8 @@ def lut_table_torch(tr: torch.Tensor, centres: torch.Tensor, k: int) -> torch.Te
 class _LutTable(torch.autograd.Function):
     """lut_table_torch over a lattice of centres in HIP kernels, without the indices: the forward keeps each query's
     k-th (distance, index) and the binned points, and the backward gathers each point's gradient from the queries that
-    took it.  A backward that is itself differentiated runs as torch operations."""
+    took it.  A backward that is itself differentiated, or whose gradient comes batched (is_grads_batched) or otherwise
+    transformed, runs as torch operations."""
 
     @staticmethod
     def forward(ctx, tr, x0, y0, step, nx, ny, k):
@@ -1457,7 +1460,7 @@ class _LutTable(torch.autograd.Function):
         x0, y0, step, nx, ny, k = ctx.lattice
         B, T, n, _ = tr.shape
         T -= 1
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not _plain_device(g):
             cy = torch.arange(ny, device=g.device, dtype=F32) * step + y0
             cx = torch.arange(nx, device=g.device, dtype=F32) * step + x0
             idx = knn_indices(torch.cartesian_prod(cy, cx).flip(-1), tr.detach()[:, 1:], k).view(B, T, -1, 1)
