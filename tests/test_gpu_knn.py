@@ -217,3 +217,27 @@ def test_tile_trajectories_and_table_take_batched_gradients():
         got, = torch.autograd.grad(out, coef, g, retain_graph=True, is_grads_batched=True)
         want = torch.stack([torch.autograd.grad(out, coef, gi, retain_graph=True)[0] for gi in g])
         assert (got - want).abs().max() <= 1e-5 * want.abs().max()     # fp32 sums of some hundred terms
+
+
+@pytest.mark.parametrize("where", ["subclass", "class", "instance"])
+def test_table_of_other_cell_centres(where, monkeypatch):
+    """Centres that a user puts in the place of the lattice are the ones looked up."""
+    from x_amd.motion import PixelTrajectories
+    from x_amd.objectives import MotionPriorCMaxLoss
+
+    def centres(self, H, W, device):
+        return torch.rand(-(-H // self.lut) * -(-W // self.lut), 2, device=device, generator=torch.Generator(device).manual_seed(2)) * 40
+
+    cls = type("Other", (MotionPriorCMaxLoss,), {"cell_centres": centres} if where == "subclass" else {})
+    if where == "class":
+        monkeypatch.setattr(MotionPriorCMaxLoss, "cell_centres", centres)
+    obj = cls(num_bins=3, num_knn=5)
+    if where == "instance":
+        obj.cell_centres = lambda H, W, device: centres(obj, H, W, device)
+    m = PixelTrajectories(_smooth_coeffs(1, 8, 41, 54, 3, 9.0).to(DEV), 4, "bspline", tile=4)
+    t_ref = torch.tensor(0.3, device=DEV)
+    mids = (torch.arange(3, device=DEV) + 0.5) / 3
+    tr = m.tile_trajectories(torch.cat([t_ref.reshape(1), mids]))
+    want = F.lut_table_torch(tr, centres(obj, 41, 54, DEV), 5)
+    got = obj.lut_flow(m, 41, 54, t_ref)[0]
+    assert (got.view_as(want) - want).abs().max() <= 1e-5 * want.abs().max()

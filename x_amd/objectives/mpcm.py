@@ -61,7 +61,7 @@ class MotionPriorCMaxLoss(Objective):
         B, nb = tr.shape[0], tr.shape[1] - 1
         half = self.lut / 2.0 - 0.5
         table = None
-        if type(self).cell_centres is MotionPriorCMaxLoss.cell_centres and self.lut > 0:
+        if getattr(self.cell_centres, "__func__", None) is _LATTICE and self.lut > 0:   # not replaced by the user
             table = lut_table(tr, half, half, float(self.lut), Wl, Hl, k)
         if table is None:
             table = lut_table_torch(tr, self.cell_centres(H, W, dev), k)
@@ -90,3 +90,6 @@ class MotionPriorCMaxLoss(Objective):
         else:
             smooth = focus.new_zeros(())
         return {"loss": focus + smooth, "focus": focus.detach(), "smooth": smooth.detach(), "sharpness": sharp.detach()}
+
+
+_LATTICE = MotionPriorCMaxLoss.cell_centres      # the centres that lut_table forms by itself
