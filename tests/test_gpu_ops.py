@@ -832,3 +832,33 @@ def test_standardise_nonzero_rows(shape):
     # the mean and the deviation are rounded to fp32 once each, then two operations
     assert (d.cpu().double() - want).abs().max() <= 8 * 2.0 ** -24 * max(float(want.abs().max()), 1.0)
     assert torch.equal(d.cpu() == 0, want.float() == 0) or shape[1] == 1
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 700, 16384])
+@pytest.mark.parametrize("kind", ["one", "four", "mixed", "spread", "border"])
+def test_few_events_on_shared_corners(kind, n):
+    """Splat and image gradient of few events, whose waves merge the events that share their corners."""
+    print(f"shared corners {kind} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    H, W = 30, 41
+    pos = (rng.random((n, 2)) * [W + 3, H + 3] - 2).astype(np.float32)
+    hot = np.array([[3.3, 4.4], [20.5, 7.25], [38.9, 28.5], [11.0, 22.0]], np.float32)
+    if kind in ("one", "four"):
+        pos = hot[rng.integers(0, 1 if kind == "one" else 4, n)]
+    elif kind == "mixed":
+        pos[rng.random(n) < 0.4] = hot[1]
+    elif kind == "border":
+        pos = np.array([[-0.5, 3.2], [W - 0.75, -0.25], [W - 1, H - 1], [5.0, H - 0.5]], np.float32)[rng.integers(0, 4, n)]
+    w = rng.normal(size=n).astype(np.float32)
+    w[rng.random(n) < 0.1] = 0
+    b = rng.integers(-1, 3, n)                     # two of the four values lie outside the batch
+    keep = (b >= 0) & (b < 2)
+    img = rng.normal(size=(2, H, W)).astype(np.float32)
+    got = N(F.get_ext().splat_bilinear_fwd(T(pos), T(w), T(b), 2, H, W))
+    mass = O.splat_bilinear_fwd(pos[keep], np.abs(w[keep]), b[keep], 2, H, W)
+    # fp32 sums in another order: their rounding against the sum of magnitudes
+    assert (np.abs(got - O.splat_bilinear_fwd(pos[keep], w[keep], b[keep], 2, H, W)) <= 2.0 ** -20 * mass + 1e-12).all()
+    gi, gp = F.get_ext().gather_bilinear_bwd(T(w), T(img), T(pos), T(b))
+    wi, wp = O.gather_bilinear_bwd(w[keep], img, pos[keep], b[keep])
+    assert (np.abs(N(gi) - wi) <= 2.0 ** -20 * mass + 1e-12).all()
+    assert np.abs(N(gp)[keep] - wp).max(initial=0) <= 1e-5 and not N(gp)[~keep].any()

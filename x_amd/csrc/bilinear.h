@@ -33,6 +33,36 @@ __device__ __forceinline__ void for_corners(float x, float y, int H, int W, F&& 
   }
 }
 
+// The same corners with one value each, in the order (y0, x0), (y0, x1), (y1, x0), (y1, x1), for kernels that add them
+// up with global atomics; add() merges the lanes of a wave that share their corners and is called by all its lanes.
+struct SplatCorners {
+  int x0, y0;
+  float v[4];
+
+  // value times the corner weights; false if no corner lies in the image
+  __device__ __forceinline__ bool set(float x, float y, float value, int H, int W) {
+    const float fx = floorf(x), fy = floorf(y);
+    if (!(fx >= -1.f && fx <= (float)(W - 1) && fy >= -1.f && fy <= (float)(H - 1))) return false;
+    x0 = (int)fx;
+    y0 = (int)fy;
+    const float ax = x - fx, ay = y - fy;
+    const float wx[2] = {1.f - ax, ax}, wy[2] = {1.f - ay, ay};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = value * (wx[k & 1] * wy[k >> 1]);
+    return true;
+  }
+  __device__ __forceinline__ void add(bool live, float* __restrict__ img, int64_t b, int H, int W) {
+    const int64_t key = (b * (H + 1) + y0) * (W + 1) + x0;
+    if (!merge_lanes(live, key, v)) return;
+    float* base = img + b * (int64_t)H * W;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int xx = x0 + (k & 1), yy = y0 + (k >> 1);
+      if (xx >= 0 && xx < W && yy >= 0 && yy < H && v[k] != 0.f) atomicAdd(base + yy * W + xx, v[k]);
+    }
+  }
+};
+
 // DenseLinearFlow.field + sample_grid (atl/motion/parametric.py:212-216, 235-251): grid coordinates
 // gx = x / sx * (Wg - 1) with sx = max(W - 1, 1) (when `scale` is set; raw grid coordinates otherwise),
 // border clamp, corners (y0, x0) .. (y1, x1) with x0 <= Wg - 2, fixed sum order c00 + c01 + c10 + c11.

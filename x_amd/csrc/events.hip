@@ -29,13 +29,16 @@ __global__ void __launch_bounds__(kBlock) k_splat_bilinear_fwd(const float2* __r
                                                                const int64_t* __restrict__ bidx, int64_t N, int64_t B,
                                                                int H, int W, float* __restrict__ img) {
   const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  const float wn = w[n];
-  const int64_t b = bidx[n];
-  if (wn == 0.f || !batch_ok(b, B)) return;
-  float* base = img + b * (int64_t)H * W;
-  const float2 p = pos[n];
-  for_corners(p.x, p.y, H, W, [&](int off, float c, float, float) { atomicAdd(base + off, wn * c); });
+  SplatCorners c{};
+  int64_t b = 0;
+  bool live = n < N;
+  if (live) {
+    const float wn = w[n];
+    const float2 p = pos[n];
+    b = bidx[n];
+    live = wn != 0.f && batch_ok(b, B) && c.set(p.x, p.y, wn, H, W);
+  }
+  c.add(live, img, b, H, W);
 }
 
 // csrc/atl_cpu.cpp:58-76
@@ -89,21 +92,26 @@ __global__ void __launch_bounds__(kBlock) k_gather_bilinear_bwd(const float* __r
                                                                 int64_t B, int H, int W, float* __restrict__ gimg,
                                                                 float2* __restrict__ gpos) {
   const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  const int64_t b = bidx[n];
-  const float g = gval[n];
-  float sx = 0.f, sy = 0.f;
-  if (batch_ok(b, B)) {
-    const int64_t plane = b * (int64_t)H * W;
-    const float2 p = pos[n];
-    for_corners(p.x, p.y, H, W, [&](int off, float c, float dcx, float dcy) {
-      const float v = img[plane + off];
-      sx += dcx * v;
-      sy += dcy * v;
-      if (g != 0.f) atomicAdd(gimg + plane + off, g * c);
-    });
+  SplatCorners c{};
+  int64_t b = 0;
+  bool live = false;
+  if (n < N) {
+    const float g = gval[n];
+    float sx = 0.f, sy = 0.f;
+    b = bidx[n];
+    if (batch_ok(b, B)) {
+      const int64_t plane = b * (int64_t)H * W;
+      const float2 p = pos[n];
+      for_corners(p.x, p.y, H, W, [&](int off, float, float dcx, float dcy) {
+        const float v = img[plane + off];
+        sx += dcx * v;
+        sy += dcy * v;
+      });
+      live = g != 0.f && c.set(p.x, p.y, g, H, W);
+    }
+    gpos[n] = make_float2(g * sx, g * sy);
   }
-  gpos[n] = make_float2(g * sx, g * sy);
+  c.add(live, gimg, b, H, W);
 }
 
 // Truncated Gaussian around (lround(x), lround(y)), csrc/atl_cpu.cpp:79-104.
