@@ -440,3 +440,27 @@ def test_backward_with_products_past_the_float_range():
     tab = PixelTrajectories(torch.zeros(1, 2, 4, 5), 1, "polynomial", tile=1).slice_tables(16, DEV)
     p = F.FastPairPlan(T(x), T(t), None, T(np.zeros(n, np.int64)), 1, H, W, None, 1.0, 0.2, 3.0, 16, T(x), traj=(T(coef), 1, tab))
     assert all(bool(torch.isfinite(g).all()) for g in p.backward_traj(T(gS)))
+
+
+@pytest.mark.parametrize("B,Hg,Wg", [(1, 1, 1), (1, 2, 2), (2, 1, 30), (2, 30, 1), (1, 32, 64), (1, 32, 65), (3, 40, 48)])
+@pytest.mark.parametrize("crowd", [False, True])
+def test_direct_flow_gradient_on_every_grid(B, Hg, Wg, crowd):
+    """The adjoint of the direct sums, in LDS up to 4096 floats of gradient and with global atomics above, sources on
+    the same cell merged by their wave: against the sources' own gradients put through the grid's adjoint."""
+    print(f"direct flow gradient B={B} {Hg}x{Wg} crowd={crowd}", flush=True)
+    rng = np.random.default_rng(Hg)
+    n, H, W = 2500, 40, 48
+    x = (rng.random((n, 2)) * [W + 30, H + 30] - 15).astype(F32)
+    if crowd:
+        x[rng.random(n) < 0.6] = [20.3, 17.6]
+    t, v = np.sort(rng.random(n)).astype(F32), (rng.normal(size=(n, 2)) * 4).astype(F32)
+    b = rng.integers(-1, B + 1, n)
+    gS = rng.normal(size=n).astype(F32)
+    p = F.FastPairPlan(T(x), T(t), T(v), T(b), B, H, W, None, 1.0, 0.2, 3.0, 16)
+    assert p.geo.direct
+    gv, got = N(p.backward(T(gS))), N(p.backward_flow(T(gS), B, Hg, Wg, H, W))
+    keep = (b >= 0) & (b < B)
+    _, idx, wts = O.dense_velocity(np.zeros((B, 2, Hg, Wg), F32), x[keep], b[keep], H, W)
+    want = O.sample_grid_bwd(gv[keep], idx, wts, got.shape)
+    mass = O.sample_grid_bwd(np.abs(gv[keep]), idx, wts, got.shape)
+    assert (np.abs(got - want) <= 2.0 ** -19 * mass + 1e-12).all()     # fp32 sums in another order

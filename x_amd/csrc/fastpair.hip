@@ -1993,7 +1993,9 @@ __global__ void __launch_bounds__(kAdjBlock) k_src_flow_adjoint(FPlan p, FGeo G,
 // backward take all sources (anchors) of the right slices, 64 at a time, compacted into LDS.  16 anchors (sources) share a
 // wave, each in four lanes, eight waves share them, every wave taking each eighth chunk; the waves' sums are added in
 // order.  The plan and its walks cost 12 launches and some 100 us of latency however few the events:
-// the anchored score of 3000 events runs 85 us of kernels instead of 130, and 10 launches less.
+// the anchored score of 3000 events runs 85 us of kernels instead of 130, and 10 launches less.  At the limits plan,
+// forward and flow backward on 40 x 48 px with a 2 x 2 grid run 52 us against 162 (5792 events, all anchors) and 70
+// against 181 (16384 events, 2048 anchors); the forward by itself is then the slower one, 45 against 21 to 29 us.
 constexpr int64_t kSmallPairs = 1 << 25, kSmallMax = 16384;
 constexpr int kSmallWaves = 8, kSmallBlock = kSmallWaves * kWave;
 constexpr int kSmallParts = 4, kSmallQ = kWave / kSmallParts;      // lanes per query, queries per workgroup
@@ -2173,23 +2175,38 @@ __global__ void __launch_bounds__(kSmallBlock) k_small_bwd(const Rec* __restrict
   if (threadIdx.x < kSmallQ && j < N) gv[j] = make_float2(sx, sy);
 }
 
-// The flow adjoint of few sources: the corners of each added with global atomics.
-__global__ void __launch_bounds__(kBlock) k_small_adjoint(const Rec* __restrict__ srec, int N, FlowGeo F,
-                                                          const float2* __restrict__ gvr, float* __restrict__ ggrid) {
-  const int j = blockIdx.x * kBlock + threadIdx.x;
-  if (j >= N) return;
-  const Rec r = srec[j];
-  const float2 g = gvr[j];
-  if (r.i.w < 0 || (g.x == 0.f && g.y == 0.f)) return;   // a zero row adds nothing
+// The flow adjoint of few sources: a wave merges its sources of the same grid cell, then their corners are added with
+// float atomics, in LDS where the whole gradient (nodes floats) fits kSmallGrid.  Atomics serialise on the few cache
+// lines of a coarse grid: pair and flow backward of 16384 sources and 2048 anchors on a 2 x 2 grid ran 1679 us without
+// the two and 22 us with them (planned: 74); on 9 x 14 nodes 90 and 27 (47), on 480 x 640 28 (44).
+constexpr int kSmallGrid = 4096, kSmallAdjBlock = 512;
+template <bool LDS>
+__global__ void __launch_bounds__(kSmallAdjBlock) k_small_adjoint(const Rec* __restrict__ srec, int N, FlowGeo F,
+                                                                  const float2* __restrict__ gvr, int64_t nodes,
+                                                                  float* __restrict__ ggrid) {
+  __shared__ float acc[LDS ? kSmallGrid : 1];
+  if (LDS) {
+    for (int i = threadIdx.x; i < (int)nodes; i += kSmallAdjBlock) acc[i] = 0.f;
+    __syncthreads();
+  }
+  const int j = blockIdx.x * kSmallAdjBlock + threadIdx.x;
+  const Rec r = srec[min(j, N - 1)];
+  const float2 g = gvr[min(j, N - 1)];
+  const bool live = j < N && r.i.w >= 0 && !(g.x == 0.f && g.y == 0.f);   // a zero row adds nothing
   const GridCorners c = grid_corners(r.f.x, r.f.y, F.Hg, F.Wg, F.sxw, F.syh, F.scale != 0);
-  const int64_t plane = (int64_t)F.Hg * F.Wg;
-  float* gb = ggrid + r.i.w * 2 * plane;
+  const int64_t plane = (int64_t)F.Hg * F.Wg, at = max(r.i.w, 0) * 2 * plane;
+  float v[8] = {g.x * c.w00, g.x * c.w01, g.x * c.w10, g.x * c.w11, g.y * c.w00, g.y * c.w01, g.y * c.w10, g.y * c.w11};
   const int o[4] = {c.o00, c.o01, c.o10, c.o11};
-  const float w[4] = {c.w00, c.w01, c.w10, c.w11};
+  if (merge_lanes(live, at + c.o00, v)) {
+    float* out = LDS ? acc + at : ggrid + at;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    atomicAdd(gb + o[k], g.x * w[k]);
-    atomicAdd(gb + plane + o[k], g.y * w[k]);
+    for (int k = 0; k < 8; ++k)
+      if (v[k] != 0.f) atomicAdd(out + (k >> 2) * plane + o[k & 3], v[k]);
+  }
+  if (LDS) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < (int)nodes; i += kSmallAdjBlock)
+      if (acc[i] != 0.f) atomicAdd(ggrid + i, acc[i]);
   }
 }
 
@@ -2584,8 +2601,9 @@ int atl_fast_flow_adjoint(const atl_fast_geometry* geo, void* ws, int64_t Hg, in
   if (is_small(geo)) {
     const int64_t ng = geo->B * 2 * Hg * Wg;
     hipLaunchKernelGGL(k_fill_zero, dim3(grid_for(ng)), dim3(kBlock), 0, stream, (int*)ggrid, ng);
-    hipLaunchKernelGGL(k_small_adjoint, dim3(grid_for(geo->N)), dim3(kBlock), 0, stream, p.srec, (int)geo->N, F,
-                       (const float2*)slots_of<float2>(ws, geo), ggrid);
+    auto adjoint = ng <= kSmallGrid ? k_small_adjoint<true> : k_small_adjoint<false>;
+    hipLaunchKernelGGL(adjoint, dim3(grid_for(geo->N, kSmallAdjBlock)), dim3(kSmallAdjBlock), 0, stream, p.srec,
+                       (int)geo->N, F, (const float2*)slots_of<float2>(ws, geo), ng, ggrid);
     return check_launch("fast_flow_adjoint");
   }
   const int64_t tiles = geo->B * ((G.GW + G.stile - 1) / G.stile) * ((G.GH + G.stile - 1) / G.stile);
