@@ -464,3 +464,20 @@ def test_direct_flow_gradient_on_every_grid(B, Hg, Wg, crowd):
     want = O.sample_grid_bwd(gv[keep], idx, wts, got.shape)
     mass = O.sample_grid_bwd(np.abs(gv[keep]), idx, wts, got.shape)
     assert (np.abs(got - want) <= 2.0 ** -19 * mass + 1e-12).all()     # fp32 sums in another order
+
+
+@pytest.mark.parametrize("B,S", [(5, 13), (63, 1), (65, 1), (33, 4), (300, 16), (4500, 1)])
+def test_backward_over_many_planes(B, S):
+    """Windows times slices around and past 64 and 64^2 planes, most of them empty, in the planned backward: the
+    gradients of the direct sums."""
+    print(f"many planes B={B} S={S}", flush=True)
+    rng = np.random.default_rng(B)
+    n, H, W = 3000, 20, 24
+    full = rng.choice(B, max(B // 3, 1), replace=False)
+    b = np.sort(np.concatenate([full[rng.integers(0, len(full), n - 2)], [0, B - 1]]))
+    x, t = (rng.random((n, 2)) * [W, H]).astype(F32), rng.random(n).astype(F32)
+    v = (rng.normal(size=(n, 2)) * 3).astype(F32)
+    gS = rng.normal(size=n).astype(F32)
+    plans = [cls(T(x), T(t), T(v), T(b), B, H, W, None, 1.5, 0.2, 3.0, S) for cls in (_PlannedSums, F.FastPairPlan)]
+    assert np.array_equal(*(N(p.counts()) for p in plans))
+    close_rel(*(N(p.backward(T(gS))) for p in plans), 1e-4)

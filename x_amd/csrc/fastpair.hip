@@ -1644,8 +1644,32 @@ __device__ __forceinline__ EntSum<TRAJ> entry_sum(const FPlan& p, const FGeo& G,
     return make_float2(g0, g1);
 }
 
+// The last plane from lo on that starts at or before position a, where plane lo does (empty planes start where the next
+// one does).  The wave looks at the next 64 planes, then at 64 evenly spaced ones of what is left: one read each at
+// up to 64 planes, three at 4096.  A scan of all of them made the backward of 256 windows of 400 events run 104 us
+// instead of 38, and of 1024 windows of 100 events 347 instead of 48.
+__device__ __forceinline__ int plane_at(const int* __restrict__ start, int a, int lo, int nplanes, int plane_cells) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int n = nplanes - lo;
+  auto upto = [&](int step) {                      // how many of the planes lo, lo + step, ... start at or before a
+    const bool in = lane < (n + step - 1) / step;
+    return __popcll(__ballot(in && start[(in ? lo + lane * step : lo) * plane_cells] <= a));
+  };
+  int c = upto(1);
+  if (c < kWave) return lo + c - 1;
+  lo += kWave - 1;
+  n -= kWave - 1;
+  while (n > 1) {
+    const int step = (n + kWave - 1) / kWave;
+    c = upto(step) - 1;
+    lo += c * step;
+    n = min(step, n - c * step);
+  }
+  return lo;
+}
+
 template <bool TRAJ>
-__global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(TRAJ ? 5 : 5))) k_entry_bwd(
+__global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5))) k_entry_bwd(
     FPlan p, FGeo G, int N, int ecap, EntSum<TRAJ>* __restrict__ slots) {
   __shared__ __align__(16) char lds[kRowTab * kPairBlock * sizeof(int2)];
   static_assert(sizeof(lds) >= (kWave + 4) * (sizeof(float4) + sizeof(int)), "the compact anchors share the row table");
@@ -1677,13 +1701,7 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
   EntSum<TRAJ> sum{};
   int pl = 0;
   for (int a = p0; a < p1;) {                        // the wave's entries plane by plane (mostly one plane)
-    // the last plane that starts at or before position a (empty planes start where the next one does)
-    for (int base = pl;; base += kWave) {
-      const int c = base + lane;
-      const int n = __popcll(__ballot(c < nplanes && p.start[min(c, nplanes - 1) * plane_cells] <= a));
-      pl = base + n - 1;
-      if (n < kWave) break;
-    }
+    pl = plane_at(p.start, a, pl, nplanes, plane_cells);
     const int e = min(p1, pl + 1 < nplanes ? uni(p.start[(pl + 1) * plane_cells]) : E);
     const bool active = p0 + lane >= a && p0 + lane < e;
     const int sl = pl % G.S;
