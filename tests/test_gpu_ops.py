@@ -862,3 +862,31 @@ def test_few_events_on_shared_corners(kind, n):
     wi, wp = O.gather_bilinear_bwd(w[keep], img, pos[keep], b[keep])
     assert (np.abs(N(gi) - wi) <= 2.0 ** -20 * mass + 1e-12).all()
     assert np.abs(N(gp)[keep] - wp).max(initial=0) <= 1e-5 and not N(gp)[~keep].any()
+
+
+@pytest.mark.parametrize("R,sigma", [(0, 0.4), (1, 0.6), (3, 1.0), (8, 2.5)])
+@pytest.mark.parametrize("kind", ["pixel", "pixels", "column", "row", "mixed", "corner"])
+def test_splat_gauss_of_crowded_centres(kind, R, sigma):
+    """Rounds whose centres fill few rows and columns of their tile: each pixel taken by several lanes."""
+    print(f"gauss crowd {kind} R={R}", flush=True)
+    rng = np.random.default_rng(R)
+    n, H, W = 20_000, 50, 70                       # crowded tiles: four rounds per workgroup
+    pos = rng.random((n, 2)) * [W, H]
+    if kind == "pixel":
+        pos[:] = [33.2, 18.9]
+    elif kind == "pixels":
+        pos = np.array([[20.3, 30.4], [31.6, 31.7], [60.5, 5.5]])[rng.integers(0, 3, n)]
+    elif kind == "column":
+        pos[:, 0] = 40 + rng.random(n)
+    elif kind == "row":
+        pos[:, 1] = 15.4 + rng.random(n)
+    elif kind == "mixed":
+        pos[rng.random(n) < 0.5] = [33.2, 18.9]
+    else:
+        pos = rng.random((n, 2)) * 1.5 - R
+    pos = pos.astype(np.float32)
+    w, b = rng.normal(size=n).astype(np.float32), rng.integers(0, 2, n)
+    got = N(F.get_ext().splat_gauss_fwd(T(pos), T(w), T(b), 2, H, W, sigma, R))
+    want, mass = (O.splat_gauss_fwd(pos, v, b, 2, H, W, sigma, R) for v in (w, np.abs(w)))
+    # exponentials to 2 ulp and fp32 sums in another order, against the sum of magnitudes
+    assert (np.abs(got - want) <= 2.0 ** -19 * mass + 1e-10).all()

@@ -689,28 +689,32 @@ __global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restric
 // Truncated-Gaussian splat in gather form (16 x 16 tiles): the scatter form's (2 R + 1)^2 LDS float atomics per
 // record took 47 us for 100k events of radius 3 on 320 x 240.  A round's records are put in the row-major order of
 // their centres (one LDS integer atomic each); the centres that reach a window pixel from one row then stand side by
-// side, and the pixel's thread adds up its 2 R + 1 runs, the same fp32 products, in registers: 23.5 us.
-constexpr int kGaussPix = 4;                      // window pixels per thread: (16 + 2 R)^2 <= 1024 for R <= 8
-static_assert((kBinT + 2 * kMaxGaussRadius) * (kBinT + 2 * kMaxGaussRadius) <= kGaussPix * kAccBlock, "window");
+// side, and the pixel's thread adds up its 2 R + 1 runs, the same fp32 products, in registers.  Only the pixels around
+// the round's occupied rows and columns are taken, and where these are few (events along an edge, hot pixels) each by
+// several lanes, which share its runs.  @GAUSS@
+constexpr int kGaussEdge = kBinT + 2 * kMaxGaussRadius;
 
 __global__ void __launch_bounds__(kAccBlock) k_gauss_accum(const int4* __restrict__ info,
                                                            const int* __restrict__ nchunk,
                                                            const float4* __restrict__ rec, TileGeo g,
                                                            float* __restrict__ out) {
   constexpr int T = kBinT;
+  static_assert(T == 16 && kWave == 4 * T, "a wave's ballot covers four rows of bins");
   __shared__ int bcnt[kBins];
   __shared__ int bstart[kBins + 1];
   __shared__ int wsum[kAccBlock / kWave + 1];
-  __shared__ float sx[kAccChunk], sy[kAccChunk], sw[kAccChunk];
+  __shared__ uint64_t occ[kAccBlock / kWave];     // occupied bins
+  __shared__ float4 srec[kAccChunk];              // (x, y, value)
+  __shared__ float acc[kGaussEdge * kGaussEdge];
   if ((int)blockIdx.x >= *nchunk) return;
   const int4 ci = info[blockIdx.x];
   const int key = ci.x, s0 = ci.y, s1 = ci.z;
-  const int tid = threadIdx.x, R = g.R, L = T + 2 * R;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), R = g.R, L = T + 2 * R;
   const int plane = g.TY * g.TX;
   const int b = key / plane, r = key - b * plane;
   const int ty = r / g.TX, tx = r - ty * g.TX;
   const int ox = tx * T - 2 * R, oy = ty * T - 2 * R;   // window column, row 0; centre columns start R later
-  float s[kGaussPix] = {};
+  for (int a = tid; a < L * L; a += kAccBlock) acc[a] = 0.f;
   for (int base = s0; base < s1; base += kAccChunk) {
     float4 q[kAccItems];
     int bin[kAccItems], rank[kAccItems];
@@ -732,44 +736,66 @@ __global__ void __launch_bounds__(kAccBlock) k_gauss_accum(const int4* __restric
     }
     __syncthreads();
     int total;
-    const int first = block_exclusive_scan<kAccBlock>(bcnt[tid], wsum, total);
+    const int mine = bcnt[tid];
+    const uint64_t some = __ballot(mine > 0);
+    if (lane == 0) occ[tid / kWave] = some;
+    const int first = block_exclusive_scan<kAccBlock>(mine, wsum, total);
     bstart[tid] = first;
     if (tid == 0) bstart[kBins] = total;
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kAccItems; ++u) {
       if (bin[u] < 0) continue;
-      const int p = bstart[bin[u]] + rank[u];
-      sx[p] = q[u].x;
-      sy[p] = q[u].y;
-      sw[p] = q[u].z * g.norm;
+      srec[bstart[bin[u]] + rank[u]] = make_float4(q[u].x, q[u].y, q[u].z * g.norm, 0.f);
+    }
+    unsigned cols = 0, rows = 0;                  // of the occupied bins
+#pragma unroll
+    for (int k = 0; k < T; ++k) {
+      const unsigned bits = (unsigned)(occ[k / 4] >> (16 * (k & 3))) & 0xffffu;
+      cols |= bits;
+      rows |= (bits ? 1u : 0u) << k;
     }
     __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kGaussPix; ++u) {
-      const int a = u * kAccBlock + tid;
-      if (a >= L * L) break;
-      const int ly = a / L, lx = a - ly * L;
-      const float fx = (float)(ox + lx), fy = (float)(oy + ly);
-      // centres within R: columns lx - 2 R .. lx and rows ly - 2 R .. ly of the tile's 16 x 16
-      const int c0 = max(lx - 2 * R, 0), c1 = min(lx, T - 1);
-      for (int row = max(ly - 2 * R, 0); row <= min(ly, T - 1); ++row) {
-        const int e = bstart[row * T + c1 + 1];
-        for (int p = bstart[row * T + c0]; p < e; ++p) {
-          const float dx = fx - sx[p], dy = fy - sy[p];
-          s[u] += sw[p] * expf(-(dx * dx + dy * dy) * g.inv2s2);
+    if (rows) {
+      const int c0 = __ffs(cols) - 1, c1 = 31 - __clz(cols), r0 = __ffs(rows) - 1, r1 = 31 - __clz(rows);
+      const int bw = c1 - c0 + 1 + 2 * R, np = bw * (r1 - r0 + 1 + 2 * R);   // the pixels within reach
+      int split = 1;                              // lanes per pixel
+      while (2 * split * np <= kAccBlock && split < kWave) split *= 2;
+      const int part = tid & (split - 1), step = kAccBlock / split;
+      for (int a = tid / split; a < np; a += step) {
+        const int ly = r0 + a / bw, lx = c0 + a % bw;
+        const float fx = (float)(ox + lx), fy = (float)(oy + ly);
+        // centres within R: columns lx - 2 R .. lx and rows ly - 2 R .. ly of the occupied ones
+        const int ca = max(lx - 2 * R, c0), cb = min(lx, c1), ra = max(ly - 2 * R, r0), rb = min(ly, r1);
+        // the wave's lanes step through the rows together (ly grows with the lane)
+        const int wa = __builtin_amdgcn_readfirstlane(ra), last = kWave - 1 - __clzll((long long)__ballot(true));
+        const int wb = __builtin_amdgcn_readlane(rb, last);
+        float s = 0.f;
+        auto add = [&](const float4& e) {
+          const float dx = fx - e.x, dy = fy - e.y;
+          s += e.z * expf(-(dx * dx + dy * dy) * g.inv2s2);
+        };
+        for (int row = wa; row <= wb; ++row) {
+          const bool in = row >= ra && row <= rb;
+          const int e = in ? bstart[row * T + cb + 1] : 0;
+          int p = in ? bstart[row * T + ca] + part : 0;
+          for (; p + 3 * split < e; p += 4 * split) {
+            const float4 e0 = srec[p], e1 = srec[p + split], e2 = srec[p + 2 * split], e3 = srec[p + 3 * split];
+            add(e0); add(e1); add(e2); add(e3);
+          }
+          for (; p < e; p += split) add(srec[p]);
         }
+        for (int d = 1; d < split; d <<= 1) s += __shfl_xor(s, d, kWave);
+        if (part == 0) acc[ly * L + lx] += s;
       }
     }
     __syncthreads();                              // the next round reuses the counts and the sorted records
   }
-#pragma unroll
-  for (int u = 0; u < kGaussPix; ++u) {
-    const int a = u * kAccBlock + tid;
-    if (a >= L * L) break;
+  for (int a = tid; a < L * L; a += kAccBlock) {
+    const float s = acc[a];
     const int py = oy + a / L, px = ox + a % L;
-    if (py < 0 || py >= g.H || px < 0 || px >= g.W || s[u] == 0.f) continue;
-    atomicAdd(out + ((int64_t)b * g.H + py) * g.W + px, s[u]);
+    if (py < 0 || py >= g.H || px < 0 || px >= g.W || s == 0.f) continue;
+    atomicAdd(out + ((int64_t)b * g.H + py) * g.W + px, s);
   }
 }
 
