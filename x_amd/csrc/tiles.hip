@@ -691,7 +691,10 @@ __global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restric
 // their centres (one LDS integer atomic each); the centres that reach a window pixel from one row then stand side by
 // side, and the pixel's thread adds up its 2 R + 1 runs, the same fp32 products, in registers.  Only the pixels around
 // the round's occupied rows and columns are taken, and where these are few (events along an edge, hot pixels) each by
-// several lanes, which share its runs.  @GAUSS@
+// several lanes, which share its runs. Whole calls of radius 3 on
+// 320 x 240, scatter form / this: 100k events spread 70 / 48 us, on one column 59 / 57, on one pixel 74 / 65, 30k on one
+// pixel 70 / 60 (1146 with one lane per pixel of the whole window, whose lanes met the occupied row at different steps);
+// 1M spread 317 / 116.
 constexpr int kGaussEdge = kBinT + 2 * kMaxGaussRadius;
 
 __global__ void __launch_bounds__(kAccBlock) k_gauss_accum(const int4* __restrict__ info,
