@@ -890,3 +890,27 @@ def test_splat_gauss_of_crowded_centres(kind, R, sigma):
     want, mass = (O.splat_gauss_fwd(pos, v, b, 2, H, W, sigma, R) for v in (w, np.abs(w)))
     # exponentials to 2 ulp and fp32 sums in another order, against the sum of magnitudes
     assert (np.abs(got - want) <= 2.0 ** -19 * mass + 1e-10).all()
+
+
+@pytest.mark.parametrize("C", [1, 5, 24])
+@pytest.mark.parametrize("kind", ["pixel", "pixels", "halves", "sevens"])
+def test_voxel_hot_pixels(kind, C):
+    """Records that share their base voxel are added up across a wave, where eight or more do, before the chains."""
+    print(f"voxel hot {kind} C={C}", flush=True)
+    rng = np.random.default_rng(C)
+    n, H, W = 20_000, 40, 50
+    pos = rng.random((n, 2)) * [W, H]
+    t = np.sort(rng.random(n))
+    if kind == "pixel":
+        pos[:], t[::2] = [17.25, 9.5], 0.5
+    elif kind == "pixels":
+        pos = np.array([[17.25, 9.5], [17.25, 10.5], [W - 0.5, -0.25], [-0.75, H - 0.5]])[rng.integers(0, 4, n)]
+    elif kind == "halves":
+        pos[rng.random(n) < 0.5] = [17.25, 9.5]
+    else:                                          # groups just below and at the merging count
+        pos = np.array([17.25, 9.5]) + np.repeat(rng.integers(0, 9, n // 7 + 1), 7)[:n, None]
+    pos, t = pos.astype(np.float32), t.astype(np.float32)
+    p, b = rng.normal(size=n).astype(np.float32), rng.integers(0, 2, n)
+    got = N(F.voxel_grid(T(pos), T(t), T(p), T(b), 2, C, H, W, normalize=None))
+    want, mass = (O.voxel_grid(pos, t, v, b, 2, C, H, W) for v in (p, np.abs(p)))
+    assert (np.abs(got - want) <= 2.0 ** -18 * mass.max()).all()      # the oracle adds in fp32 too

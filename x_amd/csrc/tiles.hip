@@ -595,10 +595,20 @@ __global__ void __launch_bounds__(kAccBlock) k_tile_accum_bins(const int4* __res
 // base voxel (time bin and base corner) with one LDS integer exchange each; the thread whose record opened a chain
 // adds up the chain's eight corner sums in registers (most chains hold one to three records: the time bins spread
 // the crowded pixels of an edge), and the sums are then added into the window in eight phases, one per corner.  In
-// one phase all base voxels write different voxels, so the additions are plain LDS reads and writes.  35 us on the same input.
+// one phase all base voxels write different voxels, so the additions are plain LDS reads and writes.  35 us on the same
+// input.  A hot pixel would make one long chain, so a wave first adds up the records that share a base voxel with its
+// first ones (kVoxMergeMin of them or more) across its lanes, and one lane puts the sums into the window.
+// Calls with all of 1M events, or of 30k, on one pixel: 74 and 35 us (339 and 247 as chains, 106 and 37 in the scatter
+// form); 1M events along edges as before.  Workgroups take 512 records, as in the scatter form, also on crowded tiles.
+constexpr int kVoxMergeRounds = 4, kVoxMergeMin = 8;
 constexpr int kVoxChainLds = 65536;               // bytes of LDS for the window, the chain heads and the records
 inline size_t vox_chain_lds(int C) {
   return (size_t)C * (kBinT + 1) * (kBinT + 1) * 4 + (size_t)(C + 1) * kBins * 4 + (size_t)kAccChunk * 20;
+}
+// Few events a tile do not pay for the chains' heads and phases: 83 a tile (100k on 640 x 480) 45.5 us a call against
+// 44.5 in the scatter form, 250 a tile 55.3 against 58.5.
+inline bool vox_chains(const TileGeo& g) {
+  return vox_chain_lds(g.C) <= kVoxChainLds && (int64_t)g.N >= (int64_t)128 * g.nkeys;
 }
 
 __global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restrict__ info,
@@ -622,6 +632,18 @@ __global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restric
   const int b = key / plane, r = key - b * plane;
   const int ty = r / g.TX, tx = r - ty * g.TX;
   const int ox = tx * T - 1, oy = ty * T - 1;
+  // the corner weights 1 - |corner - position| are a fraction or one minus it, from exact differences
+  auto corners = [](const float4& q, float (&c)[8]) {
+    const float wx[2] = {1.f - q.x, 1.f - (1.f - q.x)}, wy[2] = {1.f - q.y, 1.f - (1.f - q.y)},
+                wt[2] = {1.f - q.w, 1.f - (1.f - q.w)};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) c[k] = q.z * wt[k >> 2] * wy[(k >> 1) & 1] * wx[k & 1];
+  };
+  auto window_at = [&](int v, int k) {             // corner k of base voxel v; -1 outside the time bins
+    const int tt = v / (T * T) - 1 + (k >> 2);
+    const int ly = (v / T) % T + ((k >> 1) & 1), lx = v % T + (k & 1);
+    return (unsigned)tt < (unsigned)g.C ? (tt * L + ly) * L + lx : -1;
+  };
   __syncthreads();
   for (int base = s0; base < s1; base += kAccChunk) {
     int vox[kAccItems];                           // the chain this thread's record opened, -1: none
@@ -631,16 +653,41 @@ __global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restric
       const int i = u * kAccBlock + tid, k = base + i;
       vox[u] = -1;
       prev[u] = 0;
+      float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
       if (k < s1) {
         const float4 q = rec[k];
         int x0, y0;
         const int t1 = (int)floorf(q.w) + 1;      // base time bin + 1
         if (image_base(q.x, q.y, g.H, g.W, x0, y0) && (unsigned)t1 <= (unsigned)g.C) {   // as the binning tested
-          srec[i] = make_float4(q.x - (float)x0, q.y - (float)y0, q.z, q.w - (float)(t1 - 1));
+          f = make_float4(q.x - (float)x0, q.y - (float)y0, q.z, q.w - (float)(t1 - 1));
           vox[u] = (t1 * T + (y0 - oy)) * T + (x0 - ox);
-          prev[u] = atomicExch(head + vox[u], i);
-          snext[i] = prev[u];
         }
+      }
+      // neighbours that share a voxel, twice: worth a look (a tenth of the records on one: 14% of the waves; a fifth: 74%)
+      const bool pair = vox[u] >= 0 && __shfl_xor(vox[u], 1, kWave) == vox[u];
+      uint64_t todo = __popcll(__ballot(pair)) >= 4 ? __ballot(vox[u] >= 0) : 0;
+      for (int m = 0; m < kVoxMergeRounds && todo; ++m) {
+        const int v = __builtin_amdgcn_readlane(vox[u], __ffsll((unsigned long long)todo) - 1);
+        const uint64_t same = __ballot(vox[u] == v);
+        todo &= ~same;
+        if (__popcll(same) < kVoxMergeMin) continue;
+        float c[8];
+        corners(f, c);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) c[j] = wave_sum(vox[u] == v ? c[j] : 0.f);
+        // other waves may hold the voxel too: atomics, ahead of the barrier before the plain additions below
+        if ((tid & (kWave - 1)) == 0)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const int at = window_at(v, j);
+            if (at >= 0) atomicAdd(acc + at, c[j]);
+          }
+        if (vox[u] == v) vox[u] = -1;
+      }
+      if (vox[u] >= 0) {
+        srec[i] = f;
+        prev[u] = atomicExch(head + vox[u], i);
+        snext[i] = prev[u];
       }
     }
     __syncthreads();
@@ -654,13 +701,11 @@ __global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restric
         vox[u] = -1;
         continue;
       }
-      // the corner weights 1 - |corner - position| are a fraction or one minus it, from exact differences
       for (int i = head[vox[u]]; i >= 0; i = snext[i]) {
-        const float4 q = srec[i];
-        const float wx[2] = {1.f - q.x, 1.f - (1.f - q.x)}, wy[2] = {1.f - q.y, 1.f - (1.f - q.y)},
-                    wt[2] = {1.f - q.w, 1.f - (1.f - q.w)};
+        float c[8];
+        corners(srec[i], c);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) s[u][k] += q.z * wt[k >> 2] * wy[(k >> 1) & 1] * wx[k & 1];
+        for (int k = 0; k < 8; ++k) s[u][k] += c[k];
       }
       head[vox[u]] = -1;
     }
@@ -669,9 +714,8 @@ __global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restric
 #pragma unroll
       for (int u = 0; u < kAccItems; ++u) {
         if (vox[u] < 0) continue;
-        const int tt = vox[u] / (T * T) - 1 + (k >> 2);
-        const int ly = (vox[u] / T) % T + ((k >> 1) & 1), lx = vox[u] % T + (k & 1);
-        if ((unsigned)tt < (unsigned)g.C) acc[(tt * L + ly) * L + lx] += s[u][k];
+        const int at = window_at(vox[u], k);
+        if (at >= 0) acc[at] += s[u][k];
       }
       __syncthreads();
     }
@@ -1623,14 +1667,14 @@ template <int MODE, int C>
 bool tile_gather(const TileGeo& g) {
   constexpr bool kGatherForm = MODE == kImage || MODE == kImageG || MODE == kGridVal || MODE == kGauss ||
                                MODE == kVoxel || (MODE == kGrid && C >= 1 && C <= 4);
-  return kGatherForm && g.T == kBinT && (MODE != kVoxel || vox_chain_lds(g.C) <= kVoxChainLds) && !tile_scatter_form();
+  return kGatherForm && g.T == kBinT && (MODE != kVoxel || vox_chains(g)) && !tile_scatter_form();
 }
 
 template <int MODE, int C>
 ChunkList tile_chunk_list(const TileGeo& g, const TileLayout& L, void* ws) {
   char* w = (char*)ws;
   return ChunkList{(int4*)(w + L.info), (int*)(w + L.nchunk), kAccChunk,
-                   tile_gather<MODE, C>(g) ? kBinChunk : kAccChunk};
+                   MODE != kVoxel && tile_gather<MODE, C>(g) ? kBinChunk : kAccChunk};
 }
 
 // Histogram, scan and scatter of the records; with cl, the scatter launch's extra workgroup writes that chunk
