@@ -598,9 +598,9 @@ __global__ void __launch_bounds__(kAccBlock) k_tile_accum_bins(const int4* __res
 // one phase all base voxels write different voxels, so the additions are plain LDS reads and writes.  35 us on the same
 // input.  A hot pixel would make one long chain, so a wave first adds up the records that share a base voxel with its
 // first ones (kVoxMergeMin of them or more) across its lanes, and one lane puts the sums into the window.
-// Calls with all of 1M events, or of 30k, on one pixel: 74 and 35 us (339 and 247 as chains, 106 and 37 in the scatter
+// Calls with all of 1M events, or of 30k, on one pixel: 74 and 36 us (339 and 247 as chains, 106 and 37 in the scatter
 // form); 1M events along edges as before.  Workgroups take 512 records, as in the scatter form, also on crowded tiles.
-constexpr int kVoxMergeRounds = 4, kVoxMergeMin = 8;
+constexpr int kVoxMergeRounds = 4, kVoxMergeMin = 16;
 constexpr int kVoxChainLds = 65536;               // bytes of LDS for the window, the chain heads and the records
 inline size_t vox_chain_lds(int C) {
   return (size_t)C * (kBinT + 1) * (kBinT + 1) * 4 + (size_t)(C + 1) * kBins * 4 + (size_t)kAccChunk * 20;
@@ -663,9 +663,10 @@ __global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restric
           vox[u] = (t1 * T + (y0 - oy)) * T + (x0 - ox);
         }
       }
-      // neighbours that share a voxel, twice: worth a look (a tenth of the records on one: 14% of the waves; a fifth: 74%)
-      const bool pair = vox[u] >= 0 && __shfl_xor(vox[u], 1, kWave) == vox[u];
-      uint64_t todo = __popcll(__ballot(pair)) >= 4 ? __ballot(vox[u] >= 0) : 0;
+      // enough neighbours that share a voxel (quad_perm [1, 0, 3, 2]): worth a look, from about a third of the records on
+      // one voxel
+      const bool pair = vox[u] >= 0 && __builtin_amdgcn_update_dpp(0, vox[u], 0xB1, 0xF, 0xF, false) == vox[u];
+      uint64_t todo = __popcll(__ballot(pair)) >= kVoxMergeMin / 2 ? __ballot(vox[u] >= 0) : 0;
       for (int m = 0; m < kVoxMergeRounds && todo; ++m) {
         const int v = __builtin_amdgcn_readlane(vox[u], __ffsll((unsigned long long)todo) - 1);
         const uint64_t same = __ballot(vox[u] == v);
