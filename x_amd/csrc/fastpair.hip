@@ -1286,12 +1286,13 @@ static_assert(kPairBlock == kWave && kWave % kAnchorsPerWave == 0, "one wave per
 // time are put into LDS, and an anchor's lanes evaluate every kFwdParts-th of them, the 16 lanes of a part reading one
 // address.  The passes of up to eight wave-uniform
 // anchors evaluate all candidates of their box's cells, 3.5 per contributing pair in a crowd; here it is half of that:
-// 4M events in blobs 46 -> 31 ms.  All 64 lanes with an anchor each took 100 ms: a wave then lasts four times as long
-// and the densest end last.  On the edges of 1M events neither wins; kCommonFwd = 4, 8 and 14 run 1085, 1082 and 1074
-// us a step, with h = 2 406, 405 and 413.
+// 4M events in blobs 46 -> 35 ms.  All 64 lanes with an anchor each took 100 ms: a wave then lasts four times as long
+// and the densest end last.  kCommonFwd bounds the anchors' box in units of (cut h)^2: 3, 5 and 8 run the blobs, the
+// edges of 1M events and uniform events alike, but 200k anchors of 1M events on edges with h = 2 take 172, 172 and 194
+// us (168 in the passes).
 // [x0, x1] x [y0, y1]: the box of the anchors.
 constexpr int kFwdParts = kWave / kAnchorsPerWave;
-constexpr float kCommonFwd = 8.f;
+constexpr float kCommonFwd = 4.f;
 constexpr int kFwdSlots = kWave + 4 * kFwdParts;   // candidates of a chunk, padded to four of every part
 template <bool COUNT>
 __device__ __forceinline__ void fwd_common(const FPlan& p, const FGeo& G, int plane, float R, float R2, float vmax,
@@ -1399,7 +1400,10 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
   const int4 ai = AR.i;
   const int key = ai.z;
   const int es = p.eself[ai.x];                  // the anchor event's own entry in this slice, -1 if none
-  if (n == kAnchorsPerWave) {                    // anchors close together, in one plane: all of them at once
+  // anchors close together, in one plane: all of them at once.  The first and the last one tell most others apart (the
+  // whole test in every wave cost 1M uniform events 242 instead of 232 us)
+  auto near = [&](float bw, float bh) { return bw * bh + 2.f * G.cuth * (bw + bh) <= kCommonFwd * G.cuth * G.cuth; };
+  if (n == kAnchorsPerWave && near(fabsf(rdlanef(A.x, n - 1) - rdlanef(A.x, 0)), fabsf(rdlanef(A.y, n - 1) - rdlanef(A.y, 0)))) {
     const int cell = (ai.w >> 16) * G.GW + (ai.w & 0xffff);
     const int plane = uni(key - cell);
     const bool plain = key - cell == plane && bounded(A.x) && bounded(A.y) && bounded(A.w) && clampf(A.x, G.gx0, G.gx1) == A.x &&
@@ -1407,8 +1411,7 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
     if (__ballot(!plain) == 0) {
       const float x0 = wave_ext<false>(A.x), x1 = wave_ext<true>(A.x);
       const float y0 = wave_ext<false>(A.y), y1 = wave_ext<true>(A.y);
-      const float bw = x1 - x0, bh = y1 - y0;
-      if (bw * bh + 2.f * G.cuth * (bw + bh) <= kCommonFwd * G.cuth * G.cuth) {
+      if (near(x1 - x0, y1 - y0)) {
         const float vg = planes ? fminf(vmax, ordered_to_float(vpl[plane / (G.GH * G.GW)])) : vmax;
         float mine;
         int mine_n;
