@@ -481,3 +481,41 @@ def test_backward_over_many_planes(B, S):
     plans = [cls(T(x), T(t), T(v), T(b), B, H, W, None, 1.5, 0.2, 3.0, S) for cls in (_PlannedSums, F.FastPairPlan)]
     assert np.array_equal(*(N(p.counts()) for p in plans))
     close_rel(*(N(p.backward(T(gS))) for p in plans), 1e-4)
+
+
+@pytest.mark.parametrize("m,S,wild", [(2000, 1, False), (900, 16, False), (700, 16, True), (None, 5, False)])
+def test_backward_source_by_source(m, S, wild):
+    """Sparse anchors of many sources take the backward source by source: unsorted and repeated anchors, one and several
+    slices, a velocity past the bounds of the plain sums; against the oracle."""
+    rng = np.random.default_rng(S + 2)
+    n, B, H, W = 140_001, 3, 200, 260
+    x = (rng.random((n, 2)) * [W + 20, H + 20] - 10).astype(F32)
+    if m is None:                                  # all of them anchors, on a sensor that leaves few pairs
+        H, W = 900, 1200
+        x = (rng.random((n, 2)) * [W, H]).astype(F32)
+    t = rng.random(n).astype(F32)
+    v = (rng.normal(size=(n, 2)) * 3).astype(F32)
+    if wild:
+        v[7] = [5e18, 0]
+    b = np.sort(rng.integers(0, B, n))
+    anchors = np.arange(n) if m is None else np.concatenate([rng.integers(0, n, m), [7, 7, n - 1, 0]])
+    check_against_oracle(x, t, v, b, B, H, W, anchors, None, 1.0, 0.1, S)
+
+
+@pytest.mark.parametrize("n", [131_073, 500_001, 790_000])
+def test_plans_of_every_block_size(n):
+    """Event counts of each block size of the plan's passes, none a multiple of a block, half of them anchors: the linear
+    sums and the flow gradient against the oracle."""
+    rng = np.random.default_rng(n)
+    B, H, W, Hg, Wg = 2, 300, 400, 9, 14
+    x = (rng.random((n, 2)) * [W, H]).astype(F32)
+    t = rng.random(n).astype(F32)
+    b = np.sort(rng.integers(0, B, n))
+    grid = (rng.normal(size=(B, 2, Hg, Wg)) * 4).astype(F32)
+    v, idx, wts = O.dense_velocity(grid, x, b, H, W)
+    anchors = np.sort(rng.choice(n, n // 2, replace=False))
+    check_against_oracle(x, t, v, b, B, H, W, anchors, None, 1.0, 0.05, 16)
+    p = F.FastPairPlan(T(x), T(t), T(v), T(b), B, H, W, T(anchors), 1.0, 0.05, 3.0, 16)
+    gS = rng.normal(size=len(anchors)).astype(F32)
+    want = O.sample_grid_bwd(N(p.backward(T(gS))), idx, wts, grid.shape)
+    close_rel(N(p.backward_flow(T(gS), B, Hg, Wg, H, W)), want, 1e-4)

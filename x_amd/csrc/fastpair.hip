@@ -1,7 +1,7 @@
 // Fused anchored pair sums on gfx950: the reference's (source, slice) entries and the anchors binned into
 // one fixed, clamped fine-cell grid per slice, then a gather-form forward (the anchors of one cell share a
-// wave, whose lanes take the candidate entries of their neighbourhood) and an entry-centric backward (one
-// lane per entry, over the anchors around it), both over disc-pruned rows of fine cells.
+// wave, whose lanes take the candidate entries of their neighbourhood) and a backward with one lane per entry over
+// the anchors around it (sparse anchors: two lanes per source), both over disc-pruned rows of fine cells.
 //
 // What is kept identical to the reference (csrc/atl_cpu.cpp:176-253, atl/ops/functional.py:150-177):
 //   * the slice range of every source and its slice-centre position y = x + v (c_s - t), op for op in fp32;
@@ -95,7 +95,8 @@ struct FParams {
   int atmax;                   // max |t_a - c_s| over anchors
   int nonfinite;               // non-zero if a backward record (anchor position, time or gS) is not finite
   int planes;                  // non-zero if the per-plane maxima below were written (trajectory plans)
-  int pad[4];
+  int bysource;                // non-zero if the linear backward goes source by source (k_fast_gather_gs)
+  int pad[3];
 };                             // followed by B * S ints (ordered): each plane's max ||v|| when `planes`
 
 __device__ __forceinline__ int* plane_vmax(const FParams* P) { return (int*)(P + 1) ; }
@@ -1476,10 +1477,43 @@ __device__ __forceinline__ int2 src_tile_range(const FPlan& p, const FGeo& G, in
 // anchor's at = t - c_s is recomputed with the same fp32 operation); bes[q]: the event's own entry in the slice, which
 // the leave-one-out test skips.  Threads q < N clear gv[q] and, with gcoef, the rows of C coefficients of events without
 // a source record: the backward writes every source's total, and only what it does not write has to be cleared.
+//
+// Workgroup 0 chooses the way of the linear backward that follows from the pairs per entry, estimated over an anchor for
+// each thread as the entries in the 3 x 3 cells around it (`scale`: the area of the disc over that of the cells): below
+// `sparse` it goes source by source.  0: always entry by entry.
+__device__ __forceinline__ void choose_backward(const FPlan& p, const FGeo& G, float scale, float sparse) {
+  __shared__ float part[kBlock / kWave];
+  const int E = p.start[G.ncell_pad], Mv = p.start[2 * G.ncell_pad] - E;
+  float s = 0.f;
+  if (sparse > 0.f && Mv > 0) {
+    const int4 ai = p.arec[(int)((int64_t)threadIdx.x * Mv / kBlock)].i;
+    const int cy = ai.w >> 16, cx = ai.w & 0xffff, plane = ai.z - (cy * G.GW + cx);
+    int n[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {                    // all six loads in flight: this workgroup is the last to end
+      const int r = cy - 1 + k, row = plane + min(max(r, 0), G.GH - 1) * G.GW;
+      const int c = p.start[row + min(cx + 1, G.GW - 1) + 1] - p.start[row + max(cx - 1, 0)];
+      n[k] = r >= 0 && r < G.GH ? c : 0;
+    }
+    s = (float)n[0] + (float)n[1] + (float)n[2];
+  }
+  s = wave_sum(s);
+  if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = s;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  s = 0.f;
+  for (int w = 0; w < kBlock / kWave; ++w) s += part[w];
+  p.P->bysource = s * scale / (float)kBlock * ((float)Mv / (float)max(E, 1)) < sparse;
+}
+
 __global__ void __launch_bounds__(kBlock) k_fast_gather_gs(FPlan p, FGeo G, int M, const float* __restrict__ gS,
                                                            int N, float2* __restrict__ gv,
-                                                           float* __restrict__ gcoef, int C) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+                                                           float* __restrict__ gcoef, int C, float scale, float sparse) {
+  if (blockIdx.x == 0) {
+    choose_backward(p, G, scale, sparse);
+    return;
+  }
+  const int q = (blockIdx.x - 1) * blockDim.x + threadIdx.x;
   if (gv && q < N) gv[q] = make_float2(0.f, 0.f);
   if (gcoef && q < N && (M == 0 || p.spos[q] < 0))
     for (int c = 0; c < C; ++c) gcoef[(int64_t)q * C + c] = 0.f;
@@ -1671,11 +1705,102 @@ __device__ __forceinline__ int plane_at(const int* __restrict__ start, int a, in
   return lo;
 }
 
+// The linear backward source by source, for sparse anchors (kSparse): a lane walks the anchors of every second slice of
+// its source, whose entries it forms again, and a source's two lanes add up to the slot of its first slice.  It reads 32
+// bytes a source where the entries are 24 bytes each and write 8: 1M events on edges with 20k anchors run 119 us instead
+// of 166, uniform ones with all of them as anchors 233 instead of 279.  Looking at the pairs and at the choice costs the
+// entries' way 7 us (1M events on edges, all anchors: 358 -> 365).
+constexpr int kSrcPerWave = kWave / 2;
+template <bool LOO>
+__device__ __forceinline__ float2 source_sum(const FPlan& p, const FGeo& G, float R, float R2, const Rec& S, int half,
+                                             int2* tab) {
+  const int* astart = p.start + G.ncell_pad;
+  const int* aid = (const int*)p.arec + 4;           // event id of record k: aid[8 * k]
+  const int E = uni(p.start[G.ncell_pad]), plane_cells = G.GH * G.GW, bj = S.i.z / (G.S * plane_cells);
+  const float tj = __int_as_float(S.i.x);
+  int lo, hi;
+  slice_range(tj, G, lo, hi);
+  float gx = 0.f, gy = 0.f;
+  for (int s = lo + half; s <= hi; s += 2) {
+    float yx, yy;
+    entry_key(make_float2(S.f.x, S.f.y), make_float2(S.f.z, S.f.w), tj, bj, s, G, yx, yy);
+    const float cs = slice_centre(s, G.delta);
+    walk_flat(astart, E, (bj * G.S + s) * plane_cells, clampf(yx, G.gx0, G.gx1), clampf(yy, G.gy0, G.gy1), R, R2, G, tab,
+              [&](int k, int e, auto step) {
+      constexpr int U = decltype(step)::value;
+      float4 A[U];
+      int id[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        A[u] = ld((const float4*)p.brec + u, (uint32_t)k);
+        if (LOO) id[u] = aid[8 * (int64_t)(k + u)];
+      }
+      const int rem = e - k;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float at = A[u].z - cs, dt = A[u].z - tj;
+        const float rx = A[u].x - (yx + S.f.z * at), ry = A[u].y - (yy + S.f.w * at);
+        const float d2 = rx * rx + ry * ry;
+        const bool ok = (LOO ? id[u] != S.i.y : true) & !(fabsf(dt) > G.tau) & !(d2 > G.r2max) & (u < rem);
+        float f = A[u].w * __builtin_amdgcn_exp2f(d2 * G.kexp) * dt;      // A.w = gS / h^2
+        if (LOO) {                                   // a record may hold anything, NaN included
+          gx = ok ? fmaf(f, rx, gx) : gx;
+          gy = ok ? fmaf(f, ry, gy) : gy;
+        } else {                                     // all bounded: a zero factor adds exactly nothing
+          f = ok ? f : 0.f;
+          asm volatile("" : "+v"(f));                // keep one select
+          gx = fmaf(f, rx, gx);
+          gy = fmaf(f, ry, gy);
+        }
+      }
+    });
+  }
+  return make_float2(gx + __shfl_xor(gx, kSrcPerWave, kWave), gy + __shfl_xor(gy, kSrcPerWave, kWave));
+}
+
+// The choice as a scalar load (a kernel before wrote it): every wave of either way waits for it.
+__device__ __forceinline__ bool by_source(const FPlan& p) {
+  return *(const __attribute__((address_space(4))) int*)(uintptr_t)&p.P->bysource != 0;
+}
+
+__device__ __forceinline__ void source_wave(const FPlan& p, const FGeo& G, int lb, float2* __restrict__ slots,
+                                            float2* __restrict__ gv, char* lds) {
+  const int lane = threadIdx.x & (kWave - 1), half = lane / kSrcPerWave, q0 = lb * kSrcPerWave;
+  const int Nv = uni(p.start[3 * G.ncell_pad]) - uni(p.start[2 * G.ncell_pad]);
+  if (q0 >= Nv) return;
+  const int q = min(q0 + lane % kSrcPerWave, Nv - 1);   // copies past the last source, so that all lanes stay together
+  const Rec S = p.srec[q];
+  float R, R2;
+  search_radius(p.P, G, R, R2);
+  const float rj = G.cuth * 1.000001f + sqrtf(S.f.z * S.f.z + S.f.w * S.f.w) * ordered_to_float(p.P->atmax) * 1.000001f + 0.01f;
+  if (rj < R) {                                      // false for NaN / inf velocities: keep the whole-slice walk
+    R = rj;
+    R2 = rj * rj;
+  }
+  const bool finite = bounded(S.f.x) && bounded(S.f.y) && bounded(S.f.z) && bounded(S.f.w) && bounded(__int_as_float(S.i.x));
+  // the own pair has dt = 0: its term is exactly zero when every number is finite
+  const bool loo = uni(p.P->nonfinite) != 0 || __ballot(!finite) != 0;
+  int2* tab = (int2*)lds + threadIdx.x;
+  const float2 g = loo ? source_sum<true>(p, G, R, R2, S, half, tab) : source_sum<false>(p, G, R, R2, S, half, tab);
+  if (half == 0 && q0 + lane < Nv) {                  // by event, or for the flow adjoint by source record
+    if (gv)
+      gv[S.i.y] = g;
+    else
+      slots[q] = g;
+  }
+}
+
 template <bool TRAJ>
 __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5))) k_entry_bwd(
-    FPlan p, FGeo G, int N, int ecap, EntSum<TRAJ>* __restrict__ slots) {
+    FPlan p, FGeo G, int N, int ecap, EntSum<TRAJ>* __restrict__ slots, float2* __restrict__ gv) {
   __shared__ __align__(16) char lds[kRowTab * kPairBlock * sizeof(int2)];
   static_assert(sizeof(lds) >= (kWave + 4) * (sizeof(float4) + sizeof(int)), "the compact anchors share the row table");
+  if constexpr (!TRAJ)
+    if (by_source(p)) {
+      const int sb = xcd_block((N + kSrcPerWave - 1) / kSrcPerWave);
+      if (sb >= 0) source_wave(p, G, sb, slots, gv, lds);
+      return;
+    }
   const int lb = xcd_block((ecap + kWave - 1) / kWave);
   if (lb < 0) return;
   const int lane = threadIdx.x & (kWave - 1);
@@ -1718,10 +1843,12 @@ __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu
   }
 }
 
-// A source's gradient from its entries' slots, in slice order; q its record, t its time.
-__device__ __forceinline__ float2 slot_sum(const FGeo& G, const float2* __restrict__ slots, int N, int q, float t) {
+// A source's gradient from its entries' slots, in slice order, or from its first one; q its record, t its time.
+__device__ __forceinline__ float2 slot_sum(const FPlan& p, const FGeo& G, const float2* __restrict__ slots, int N, int q,
+                                           float t) {
   int lo, hi;
   slice_range(t, G, lo, hi);
+  if (by_source(p)) hi = lo;
   float gx = 0.f, gy = 0.f;
 #pragma unroll 4
   for (int k = 0; k <= hi - lo; ++k) {
@@ -1735,9 +1862,9 @@ __device__ __forceinline__ float2 slot_sum(const FGeo& G, const float2* __restri
 __global__ void __launch_bounds__(kBlock) k_slot_sum(FPlan p, FGeo G, int N, const float2* __restrict__ slots,
                                                      float2* __restrict__ gv) {
   const int q = blockIdx.x * kBlock + threadIdx.x;
-  if (q >= p.start[3 * G.ncell_pad] - p.start[2 * G.ncell_pad]) return;
+  if (by_source(p) || q >= p.start[3 * G.ncell_pad] - p.start[2 * G.ncell_pad]) return;
   const int4 si = p.srec[q].i;
-  gv[si.y] = slot_sum(G, slots, N, q, __int_as_float(si.x));
+  gv[si.y] = slot_sum(p, G, slots, N, q, __int_as_float(si.x));
 }
 
 // The trajectory model's: y_s = p + sum_k cf_k g_k(c_s) and v_s = sum_k cf_k g_k'(c_s) chain the slots (Gy_s, Gv_s)
@@ -1915,7 +2042,7 @@ __global__ void __launch_bounds__(kAdjBlock) k_src_flow_adjoint(FPlan p, FGeo G,
     Rec R{};
     if (live[u]) R = p.srec[q];
     const float4 f = R.f;
-    g[u] = live[u] ? slot_sum(G, slots, N, q, __int_as_float(R.i.x)) : make_float2(0.f, 0.f);
+    g[u] = live[u] ? slot_sum(p, G, slots, N, q, __int_as_float(R.i.x)) : make_float2(0.f, 0.f);
     c[u] = grid_corners(f.x, f.y, F.Hg, F.Wg, F.sxw, F.syh, F.scale != 0);
     live[u] = live[u] && !(g[u].x == 0.f && g[u].y == 0.f);   // a zero row adds nothing
     if (live[u]) {
@@ -2314,11 +2441,30 @@ void launch_small_bwd(const FPlan& p, const FGeo& G, const atl_fast_geometry* ge
                      p.srec, (int)geo->N, p.arec, (int)geo->M, G, gS, gv);
 }
 
+// The pairs per entry below which the linear backward goes source by source, 24 / radius px from 1M sources on and fewer
+// below, where the entries' own traffic, which it saves, stays in the caches.  Times source by source / entry by entry in
+// us, 16 slices on 640 x 480: 1M events, h = 1, 1.6 pairs 170 / 223, 4.8 226 / 280, 6.7 216 / 231, 20 410 / 360; h = 2, 1.1
+// pairs 146 / 171, 5.3 207 / 203, 17 339 / 286; h = 1/2, 2.6 pairs 166 / 219, 7.8 266 / 296; 200k events, h = 1, 0.4 pairs
+// 38 / 43, 1.3 45 / 50, 4 68 / 62; 50k events alike or entry by entry the faster one throughout.
+constexpr int64_t kSparseMin = 131072;
+float sparse_pairs(int64_t N, double radius) {
+  return N > kSparseMin ? (float)(24.0 / radius * std::min(1e-6 * (double)N, 1.0)) : 0.f;
+}
+
+// Backward records and, with `linear`, the choice between the two ways.
+void launch_gather_gs(const FPlan& p, const FGeo& G, const atl_fast_geometry* geo, const float* gS, float2* gv,
+                      float* gcoef, int C, bool linear, hipStream_t stream) {
+  const double r = geo->cut * geo->h, scale = M_PI * r * r / (9.0 * (double)geo->cell * (double)geo->cell);
+  hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N)) + 1), dim3(kBlock), 0, stream, p, G,
+                     (int)geo->M, gS, (int)geo->N, gv, gcoef, C, (float)scale, linear ? sparse_pairs(geo->N, r) : 0.f);
+}
+
 template <bool TRAJ>
-void launch_entry_bwd(const FPlan& p, const FGeo& G, const atl_fast_geometry* geo, void* ws, hipStream_t stream) {
-  const int64_t nblocks = (geo->ecap + kWave - 1) / kWave;
+void launch_entry_bwd(const FPlan& p, const FGeo& G, const atl_fast_geometry* geo, void* ws, float2* gv, hipStream_t stream) {
+  const int64_t by_source = TRAJ ? 0 : (geo->N + kSrcPerWave - 1) / kSrcPerWave;   // the device chooses
+  const int64_t nblocks = std::max((geo->ecap + kWave - 1) / kWave, by_source);
   hipLaunchKernelGGL(k_entry_bwd<TRAJ>, dim3(xcd_grid(nblocks)), dim3(kPairBlock), 0, stream, p, G, (int)geo->N,
-                     (int)geo->ecap, slots_of<EntSum<TRAJ>>(ws, geo));
+                     (int)geo->ecap, slots_of<EntSum<TRAJ>>(ws, geo), gv);
 }
 
 }  // namespace
@@ -2572,11 +2718,9 @@ int atl_fast_pair_bwd(const atl_fast_geometry* geo, void* ws, const float* gS, f
     launch_small_bwd(p, G, geo, gS, (float2*)gv, stream);
     return check_launch("fast_pair_bwd");
   }
-  hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
-                     (int)geo->M, gS, (int)geo->N, (float2*)gv, (float*)nullptr, 0);
-  if (geo->M > 0)
-  {
-    launch_entry_bwd<false>(p, G, geo, ws, stream);
+  launch_gather_gs(p, G, geo, gS, (float2*)gv, nullptr, 0, true, stream);
+  if (geo->M > 0) {
+    launch_entry_bwd<false>(p, G, geo, ws, (float2*)gv, stream);
     hipLaunchKernelGGL(k_slot_sum, dim3(grid_for(geo->N)), dim3(kBlock), 0, stream, p, G, (int)geo->N,
                        (const float2*)slots_of<float2>(ws, geo), (float2*)gv);
   }
@@ -2595,9 +2739,8 @@ int atl_fast_pair_bwd_src(const atl_fast_geometry* geo, void* ws, const float* g
     launch_small_bwd(p, G, geo, gS, slots_of<float2>(ws, geo), stream);
     return check_launch("fast_pair_bwd_src");
   }
-  hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
-                     (int)geo->M, gS, (int)geo->N, (float2*)nullptr, (float*)nullptr, 0);
-  launch_entry_bwd<false>(p, G, geo, ws, stream);
+  launch_gather_gs(p, G, geo, gS, nullptr, nullptr, 0, true, stream);
+  launch_entry_bwd<false>(p, G, geo, ws, nullptr, stream);
   return check_launch("fast_pair_bwd_src");
 }
 
@@ -2660,10 +2803,9 @@ int atl_fast_pair_bwd_traj(const atl_fast_geometry* geo, void* ws, const float* 
   if (geo->N == 0) return 0;
   const FPlan p = make_plan(ws, geo);
   // the record pass clears gp and the rows of gcoef that no source writes: they keep zero gradients
-  hipLaunchKernelGGL(k_fast_gather_gs, dim3(grid_for(std::max(geo->M, geo->N))), dim3(kBlock), 0, stream, p, G,
-                     (int)geo->M, gS, (int)geo->N, (float2*)gp, gcoef, (int)(2 * K));
+  launch_gather_gs(p, G, geo, gS, (float2*)gp, gcoef, (int)(2 * K), false, stream);
   if (geo->M > 0) {
-    launch_entry_bwd<true>(p, G, geo, ws, stream);
+    launch_entry_bwd<true>(p, G, geo, ws, nullptr, stream);
     const float4* slots = slots_of<float4>(ws, geo);
     switch (K) {
 #define ATL_K(k) case k: hipLaunchKernelGGL(k_slot_traj<k>, dim3(grid_for(geo->N)), dim3(kBlock), 0, stream, p, G, (int)geo->N, slots, tab, (float2*)gp, gcoef); break;
