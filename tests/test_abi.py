@@ -79,3 +79,6 @@ def test_pair_geometry_refuses_what_32_bit_offsets_cannot_reach(lib):
         rc = L.atl_fast_geometry_init(16, m, 1, 40, 48, 1, 1.0, 0.2, 3.0, ctypes.byref(g))
         assert (rc == 0) == ok, m
         assert ok or b"too large" in L.atl_last_error()
+    # far more anchors than events on a sensor with many buckets: the blocks' rows of counts stay within bounds
+    g = _ext.FastGeometry()
+    assert L.atl_fast_geometry_init(1000, 260_000_000, 13, 480, 640, 16, 1.0, 0.2, 3.0, ctypes.byref(g)) == 0

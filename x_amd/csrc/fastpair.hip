@@ -54,7 +54,10 @@ constexpr int kSrcPerBlock = 4096;                 // pass-1 sources per block, 
 // 25 us whatever the count, as its threads take their sources one after another (100k sources of 17 slices: 28 blocks
 // of 4096 ran 24 + 14 us and the entry passes 48 us, 108 blocks of 1024 run 11 + 6 us and the entry passes 21 us).  Anchors: twice as many per
 // block; entry passes: half as many.
-__host__ inline int src_per_block(int64_t N) { return N > 786432 ? kSrcPerBlock : N > 393216 ? kSrcPerBlock / 2 : kSrcPerBlock / 4; }
+__host__ inline int src_per_block(int64_t N, int64_t M) {
+  const int64_t n = std::max(N, M / 2);           // far more anchors than events (repeated ones) count too: the blocks' bucket rows
+  return n > 786432 ? kSrcPerBlock : n > 393216 ? kSrcPerBlock / 2 : kSrcPerBlock / 4;
+}
 constexpr int kUnroll = 8;                         // record arrays padded by at least a walk step
 constexpr int kStep = 4;                           // candidates per walk step
 constexpr int kSliceBatch = 4;                     // pass 1: slices of one source keyed and placed together
@@ -2378,7 +2381,7 @@ bool make_geo(const atl_fast_geometry* geo, FGeo& G) {
   G.icf = 1.f / G.cf;
   G.GW = (int)geo->GW; G.GH = (int)geo->GH; G.S = (int)geo->S; G.B = geo->B;
   G.ncell = (int)geo->ncell; G.ncell_pad = (int)geo->ncell_pad; G.MS = (int)geo->max_span;
-  G.spb = src_per_block(geo->N);
+  G.spb = src_per_block(geo->N, geo->M);
   G.nblk_e = (int)((geo->N + G.spb - 1) / G.spb);
   G.nblk_a = (int)((geo->M + 2 * G.spb - 1) / (2 * G.spb));
   G.apw = anchors_per_wave(geo->M);
@@ -2516,7 +2519,7 @@ int atl_fast_geometry_init(int64_t N, int64_t M, int64_t B, int64_t H, int64_t W
     nbuckets = 3 * ncell_pad / keys;
     if (nbuckets <= kMaxBuckets) break;
   }
-  const int spb = src_per_block(N);
+  const int spb = src_per_block(N, M);
   const double nblk = std::ceil((double)N / spb) + std::ceil((double)M / (2 * spb));
   // GW, GH < 32768: anchor records pack (cy, cx) into 16-bit halves
   if (3 * ncell_pad + 1 >= 2.0e9 || ecap + M + N >= 2.0e9 || M > kMaxAnchors || nbuckets > kMaxBuckets || nbuckets * nblk + 1 >= 2.0e9 ||
