@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(kBlock) k_knn_query(const float2* __restrict__
 //
 // The adjoint gathers: a point takes the gradient of every query whose k-th (distance, index) it does not exceed, the
 // same fp32 distance giving the same decision.  Queries stand in blocks of 4 x 4 with the largest k-th distance of
-// each block, so that a point tests about ten blocks (61 us; 88 us with a gradient loaded per taken query; torch's
+// each block, so that a point tests about ten blocks (47 to 61 us; 75 to 88 us with a gradient loaded per taken query; torch's
 // scatter of 9.2M rows through atomics took 180 us, and the gather and mean forward another 130).
 constexpr int kQB = 4;                           // queries per block side
 constexpr int kQStep = 8;                        // candidates a query reads at once (2: 238, 4: 216, 8: 211 us)
@@ -372,8 +372,9 @@ __global__ void __launch_bounds__(kBlock) k_lut_query(float x0, float y0, float 
       r += 1 + r / 2;
     }
     // narrow (lo, hi] until at most three points of it are taken; the first cuts lie where the bound above usually
-    // leaves the distance, so that one round is enough for most waves
-    for (int it = 0; it < 8; ++it) {
+    // leaves the distance, so that one round is enough for most waves.  A cut that leaves all of the points in is the
+    // last: they may share their distance (all points in one place: 1053 -> 775 ms, as every pass reads them all; the indices path 585)
+    for (int it = 0, held = -1; it < 8; ++it) {
       const float w = hi - lo;
       if (it == 0 && hi < INFINITY) {
         th[0] = 0.55f * hi; th[1] = 0.68f * hi; th[2] = 0.76f * hi; th[3] = 0.82f * hi; th[4] = 0.88f * hi;
@@ -404,7 +405,8 @@ __global__ void __launch_bounds__(kBlock) k_lut_query(float x0, float y0, float 
         if (th[i] < hi && c[i] >= k) { nhi = th[i]; nch = c[i]; }
       const bool same = nlo == lo && nhi == hi;
       lo = nlo; hi = nhi; clo = ncl; chi = nch;
-      if (chi < k || k - clo < kPick || same) break;
+      if (chi < k || k - clo < kPick || same || chi - clo == held) break;
+      held = chi - clo;
     }
     // the points under lo, and the k - clo first of those in [lo, hi) by (distance, index), kPick at a time
     float sx = 0.f, sy = 0.f;
