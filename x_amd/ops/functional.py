@@ -203,7 +203,8 @@ def _interleaved(fld: torch.Tensor) -> torch.Tensor:
 
 
 # Flow look-ups of at most this many positions read the planar field: 2.6 us against 2.4 + 2.8 us and a launch more for the
-# interleaved copy at 3000 positions of a 48 x 40 grid.
+# interleaved copy at 3000 positions of a 48 x 40 grid.  Whole calls on 480 x 640, 40 x 48 and 2 x 2 nodes alike: 13 us
+# against 26 at 3000 to 16384 positions; at 30000 the interleaved copy has 20.
 IL_MIN_EVENTS = 16384
 
 
@@ -1362,10 +1363,9 @@ TILE_TABLE_MAX = 4096
 
 def _plain_device(*ts) -> bool:
     """Whether a fused op that replaces a chain of torch operations may take these tensors: plain fp32 device tensors,
-    and no transform or mode at work that has to see the operations themselves (tracing, torch.func, batched gradients,
-    forward-mode derivatives, autocast's casts, dispatch modes)."""
-    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == F32 and torch._C._has_storage(t)
-                for t in ts)
+    and no transform or mode at work that has to see the operations themselves (tracing, torch.func, forward-mode
+    derivatives, autocast's casts, dispatch modes)."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == F32 for t in ts)
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
             and not torch.is_autocast_enabled("cuda") and torch._C._len_torch_dispatch_stack() == 0)
@@ -1373,8 +1373,8 @@ def _plain_device(*ts) -> bool:
 
 class _TileTrajectories(torch.autograd.Function):
     """PixelTrajectories.tile_trajectories (atl/motion/trajectories.py:88-97) in one kernel each way.  A backward that
-    is itself differentiated, or whose gradient comes batched (is_grads_batched) or otherwise transformed, runs as the
-    torch expression of the adjoint."""
+    is itself differentiated, or whose gradient comes batched (is_grads_batched: no storage of its own), runs as
+    the torch expression of the adjoint."""
 
     @staticmethod
     def forward(ctx, coef, times, K, kind, offset, tile):
@@ -1392,7 +1392,7 @@ class _TileTrajectories(torch.autograd.Function):
     def backward(ctx, g):
         times, = ctx.saved_tensors
         B, K, Hq, Wq = ctx.shape
-        if torch.is_grad_enabled() or not _plain_device(g):
+        if torch.is_grad_enabled() or not torch._C._has_storage(g):
             from ..motion.trajectories import basis
             gc = torch.matmul(g.permute(0, 3, 2, 1), basis(times, K, ctx.kind)).transpose(2, 3).flip(1)   # (B, 2, K, n)
             return gc.reshape(B, 2 * K, Hq, Wq), None, None, None, None, None
@@ -1437,8 +1437,8 @@ def lut_table_torch(tr: torch.Tensor, centres: torch.Tensor, k: int) -> torch.Te
 class _LutTable(torch.autograd.Function):
     """lut_table_torch over a lattice of centres in HIP kernels, without the indices: the forward keeps each query's
     k-th (distance, index) and the binned points, and the backward gathers each point's gradient from the queries that
-    took it.  A backward that is itself differentiated, or whose gradient comes batched (is_grads_batched) or otherwise
-    transformed, runs as torch operations."""
+    took it.  A backward that is itself differentiated, or whose gradient comes batched (is_grads_batched: no
+    storage of its own), runs as torch operations."""
 
     @staticmethod
     def forward(ctx, tr, x0, y0, step, nx, ny, k):
@@ -1460,7 +1460,7 @@ class _LutTable(torch.autograd.Function):
         x0, y0, step, nx, ny, k = ctx.lattice
         B, T, n, _ = tr.shape
         T -= 1
-        if torch.is_grad_enabled() or not _plain_device(g):
+        if torch.is_grad_enabled() or not torch._C._has_storage(g):
             cy = torch.arange(ny, device=g.device, dtype=F32) * step + y0
             cx = torch.arange(nx, device=g.device, dtype=F32) * step + x0
             idx = knn_indices(torch.cartesian_prod(cy, cx).flip(-1), tr.detach()[:, 1:], k).view(B, T, -1, 1)
