@@ -42,20 +42,35 @@ def _case(seed=0, n=6000, B=2, H=40, W=48, h=1.0):
     return win, xs, v, xa
 
 
+class _PlannedSums(F.FastPairPlan):
+    """The fused path with its plan, also where few events would be summed directly."""
+
+    def _geometry(self, *sizes):
+        super()._geometry(*sizes)
+        self.geo.direct = 0.0
+
+
 def check_against_oracle(xs, t, v, b, B, H, W, anchors, xa, h, tau, S, seed=0, index_free=False):
-    """Counts, sums and gradients of the fused path vs the oracle on the reference plan.  ``index_free``: the
-    anchors are every event in order and the fused plan gets no index array (the benchmarked form)."""
+    """Counts, sums and gradients of the fused path vs the oracle on the reference plan, with its plan and, where few
+    events are summed directly, that way too.  ``index_free``: the anchors are every event in order and the fused plan
+    gets no index array (the benchmarked form)."""
     print(f"fast pair case N={len(t)} M={len(anchors)} B={B} HxW={H}x{W} h={h} tau={tau} S={S}", flush=True)
     p = O.build_pair_plan(xs, t, v, b, B, H, W, anchors, h, tau, 3.0, S, anchor_xy=xa)
     want, wcnt = O.ats_pair_fwd(p, h, tau, 3.0, with_counts=True)
     if index_free:
         assert np.array_equal(anchors, np.arange(len(t)))
-    plan = F.FastPairPlan(T(xs), T(t), T(v), T(b), B, H, W, None if index_free else T(anchors), h, tau, 3.0, S,
-                          None if xa is None else T(xa))
-    assert np.array_equal(N(plan.counts()), wcnt)
-    assert_sums_close(N(plan.forward()), want)
     gS = np.random.default_rng(seed + 3).standard_normal(len(anchors)).astype(F32)
-    close_rel(N(plan.backward(T(gS))), O.ats_pair_bwd(gS, p, h, tau, 3.0, len(t)), 1e-4)
+    want_g = O.ats_pair_bwd(gS, p, h, tau, 3.0, len(t))
+    direct = False
+    for cls in (F.FastPairPlan, _PlannedSums):
+        plan = cls(T(xs), T(t), T(v), T(b), B, H, W, None if index_free else T(anchors), h, tau, 3.0, S,
+                   None if xa is None else T(xa))
+        if cls is _PlannedSums and not direct:
+            break                                  # the plan was taken already
+        direct = plan.geo.direct != 0
+        assert np.array_equal(N(plan.counts()), wcnt)
+        assert_sums_close(N(plan.forward()), want)
+        close_rel(N(plan.backward(T(gS))), want_g, 1e-4)
     return wcnt
 
 
@@ -249,13 +264,17 @@ def test_fast_blob_contention_matches_reference_layout():
     close_rel(N(plan.backward(gS)), N(e.ats_pair_bwd(gS, *args, win.n)), 1e-4)
 
 
+@pytest.mark.parametrize("planned", [False, True])
 @pytest.mark.parametrize("B,H,W,Hg,Wg,h", [(2, 40, 48, 40, 48, 1.0), (2, 37, 53, 9, 14, 0.5), (1, 30, 36, 30, 1, 2.0),
                                             (3, 24, 20, 2, 2, 1.0)])
-def test_pair_sums_flow_matches_oracle(B, H, W, Hg, Wg, h):
+def test_pair_sums_flow_matches_oracle(B, H, W, Hg, Wg, h, planned, monkeypatch):
     """ats_pair_sums_flow (the flow sampled inside, its gradient accumulated over the plan's source records) against
     the oracle: sums within 1e-5, and the flow-grid gradient (pair backward, then sample_grid's adjoint) within
     1e-4, on full-resolution, coarse and degenerate grids, with sources far outside the sensor (clamped into the
-    border nodes and the plan's box, so that their records fall outside the tile's window)."""
+    border nodes and the plan's box, so that their records fall outside the tile's window).  ``planned``: with the plan,
+    also where the events are few enough for the direct sums."""
+    if planned:
+        monkeypatch.setattr(F, "FastPairPlan", _PlannedSums)
     print(f"pair sums flow B={B} {H}x{W} grid {Hg}x{Wg} h={h}", flush=True)
     rng = np.random.default_rng(B * 100 + Hg)
     n = 2500 * B
@@ -302,14 +321,6 @@ def test_pair_sums_flow_full_size_matches_composed():
     # the same pairs; the within-cell record order follows the plan's LDS atomics, so sums differ in the last bits
     assert_sums_close(res[0][0], res[1][0])
     close_rel(res[0][1], res[1][1], 1e-4)
-
-
-class _PlannedSums(F.FastPairPlan):
-    """The fused path with its plan, also where few events would be summed directly."""
-
-    def _geometry(self, *sizes):
-        super()._geometry(*sizes)
-        self.geo.direct = 0.0
 
 
 @pytest.mark.parametrize("n,m,B,S,h,tau", [(1, None, 1, 16, 1.0, 0.2), (15, 7, 2, 1, 2.0, 0.4), (64, None, 1, 3, 1.0, 1.0),
@@ -519,3 +530,24 @@ def test_plans_of_every_block_size(n):
     gS = rng.normal(size=len(anchors)).astype(F32)
     want = O.sample_grid_bwd(N(p.backward(T(gS))), idx, wts, grid.shape)
     close_rel(N(p.backward_flow(T(gS), B, Hg, Wg, H, W)), want, 1e-4)
+
+
+@pytest.mark.parametrize("n", [196_609, 530_001])
+def test_reference_layout_of_every_block_size(n):
+    """The reference-layout entries where pass A of its plan and of its anchors takes two and four items per thread:
+    counts, sums and gradients of the fused path."""
+    print(f"reference layout n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    B, H, W = 2, 240, 320
+    x, t = T((rng.random((n, 2)) * [W, H]).astype(F32)), T(rng.random(n).astype(F32))
+    v, b = T((rng.normal(size=(n, 2)) * 4).astype(F32)), T(np.sort(rng.integers(0, B, n)))
+    a = torch.arange(n, device=DEV)
+    q = F.build_pair_plan(x, t, v, b, B, H, W, a, 1.0, 0.05, 3.0, 16)
+    p = F.FastPairPlan(x, t, v, b, B, H, W, None, 1.0, 0.05, 3.0, 16)
+    assert np.array_equal(N(F.pair_counts(q, 1.0, 0.05, 3.0)), N(p.counts()))
+    tv = v.clone().requires_grad_(True)
+    S = F._ATSPair.apply(tv, q, 1.0, 0.05, 3.0)
+    assert_sums_close(N(S), N(p.forward()))
+    gS = torch.randn(n, device=DEV, generator=torch.Generator(device=DEV).manual_seed(2))
+    S.backward(gS)
+    close_rel(N(tv.grad), N(p.backward(gS)), 1e-4)

@@ -405,12 +405,14 @@ def test_plan_bit_exact(tau, S, h):
 
 
 @pytest.mark.parametrize("n,B,H,W,tau,S", [(20000, 2, 40, 48, 0.2, 16), (30000, 4, 480, 640, 0.05, 96),
-                                            (7, 1, 40, 48, 0.3, 8)])
+                                            (7, 1, 40, 48, 0.3, 8), (196_609, 2, 240, 320, 0.1, 16),
+                                            (530_001, 3, 240, 320, 0.05, 8), (790_001, 2, 240, 320, 0.05, 8)])
 def test_sorted_plan_equals_the_atomic_plan(n, B, H, W, tau, S):
     """atl_plan_sort (bucketed counting sort, one call) against atl_plan_count + atl_scan_counts + atl_plan_fill
     (per-entry atomics) on the same geometry: cell_start bit for bit, the same (cell, source) entries with the same
     slice positions, velocities and times; events of an absent batch and positions leaving the grid are dropped by
-    both.  The second case has about 9M cells (buckets of 1024 keys), the third seven events."""
+    both.  The second case has about 9M cells (buckets of 1024 keys), the third seven events; the last three take two,
+    four and eight events per thread of pass A, the first three one."""
     print(f"sorted plan n={n} B={B} {H}x{W} tau={tau} S={S}", flush=True)
     rng = np.random.default_rng(n + S)
     x = np.stack([rng.uniform(-30, W + 30, n), rng.uniform(-30, H + 30, n)], 1).astype(F32)
