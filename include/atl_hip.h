@@ -390,7 +390,8 @@ int atl_fast_pair_bwd(const atl_fast_geometry* geo, void* ws, const float* gS, f
  * 235-251): the gradient goes to the flow grid (B,2,Hg,Wg), written to ggrid (no fill needed), as
  * atl_fast_pair_bwd followed by sample_grid's adjoint at x would give it (float sums in another order), with no
  * per-event gradient array.  img_h, img_w: the pixel -> grid scaling of atl_sample_grid_fwd (0, 0: x are grid
- * coordinates).  The plan's temporary sort records (dead after the plan) hold the per-source gradients. */
+ * coordinates).  The plan's temporary sort records (dead after the plan) hold the
+ * gradient sums of the entries or sources. */
 int atl_fast_pair_bwd_flow(const atl_fast_geometry* geo, void* ws, const float* gS, int64_t Hg, int64_t Wg,
                            int64_t img_h, int64_t img_w, float* ggrid, hipStream_t stream);
 /* atl_fast_pair_bwd_flow in its two steps: the pair backward (the source gradients, kept in ws), then the

@@ -265,10 +265,8 @@ __global__ void __launch_bounds__(kBlock) k_fill_zero(int* __restrict__ p, int64
   if (i < n) p[i] = 0;
 }
 
-
-
-// Pass 1.  Blocks [0, nblk_a) cover kAncPerBlock anchors each, blocks [nblk_a, nblk_a + nblk_e) kSrcPerBlock
-// sources each (their entries and one source record keyed by the cell of the own-slice entry).
+// Pass 1.  Blocks [0, nblk_a) cover 2 G.spb anchors each, blocks [nblk_a, nblk_a + nblk_e) G.spb sources each (their
+// entries and one source record keyed by the cell of the own-slice entry).
 // SCATTER = false: per-block bucket histogram into cnt[block * nbuckets + bucket] (block-major: written and read
 // back coalesced), its non-zero counts added into the bucket totals tot[bucket], and the reductions behind the
 // search radius: vmax over the sources' velocities and max |at| over the anchors (block maxima, one atomic max
@@ -1372,12 +1370,9 @@ __device__ __forceinline__ void fwd_common(const FPlan& p, const FGeo& G, int pl
 // sums one candidate per chunk, the 64 lane partials are added in a tree (the reference's CPU path sums
 // sequentially in fp64; both stay well inside 1e-5 of the exact sum).
 
-// Register budgets (amdgpu_waves_per_eu: the compiler keeps the kernel within the registers of that many waves
-// per SIMD): the forward fits 8 waves without spills (53 VGPRs, 69 unconstrained), the backward 6 (80 VGPRs, three
-// spills outside its walk loop; 88 unconstrained), the trajectory backward 4 at K = 10 (128 VGPRs, 135
-// unconstrained).  Same code, more waves to hide the candidate loads: C3 forward 0.329 -> 0.322 ms, backward
-// 0.446 -> 0.435 ms, C4 trajectory backward 1.89 -> 1.67 ms (alternating runs on one box).  Tighter budgets spill
-// inside the walks (backward at 7 waves: 13 spills; trajectory backward at 5: 42).
+// Register budgets (amdgpu_waves_per_eu: the compiler keeps the kernel within the registers of that many waves per
+// SIMD): the forward fits 8 waves without vector spills (54 VGPRs), the backward 5 (89 VGPRs, trajectories 91).  More
+// waves hide the candidate loads: the forward of 1M events ran 0.329 ms unconstrained and 0.322 at 8 waves.
 template <bool COUNT>
 __global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(8))) k_fast_fwd(FPlan p, FGeo G, int M, float* __restrict__ out,
                                                      int* __restrict__ count) {
@@ -2542,7 +2537,7 @@ int atl_fast_geometry_init(int64_t N, int64_t M, int64_t B, int64_t H, int64_t W
   g.off_start = off;   off += align256((3 * g.ncell_pad + 1) * 4);
   // the sort's records sit at their bucket positions in all three key spaces (the linear model's anchor and
   // source records after the entries' counted places), so the region holds ecap + M + N records; after the plan
-  // it also serves the flow adjoint's scratch (per-source gradients, chunk list, tile counts) and the backward's slots
+  // it also serves the flow adjoint's scratch (chunk list, chunk count, tile counts) and the backward's slots
   g.off_trec = off;    off += align256(std::max((g.ecap + M + N) * (int64_t)sizeof(Rec),
                                                 align256(adj_scratch_bytes(B, N, g.GW, g.GH, g.cell)) +
                                                     g.ecap * (int64_t)sizeof(float4)));

@@ -1576,9 +1576,6 @@ TileLayout tile_layout(const TileGeo& g) {
 
 __global__ void k_tile_zero1(int* p) { p[0] = 0; }
 
-// ATL_TILE_SCATTER=1 in the environment selects the scatter form of the accumulation for every mode (read at
-// every call, so that a test can compare both forms in one process).  A backward that reuses its forward's chunk
-// list may therefore run the other form on it: the scatter form takes chunks of any length, in rounds.
 // Standardisation of a row's non-zero entries (x - mean) / sd in place (sd of n - 1; 1 where it is not positive, as
 // for a single entry): chunk sums of count, x and x^2 in fp64, then every workgroup adds up its row's chunk sums in a
 // fixed order and rewrites its own chunk.  Two launches that read the row twice and write it once; the twenty torch
@@ -1656,6 +1653,9 @@ __global__ void __launch_bounds__(kBlock) k_nz_apply(float* __restrict__ x, int6
   }
 }
 
+// ATL_TILE_SCATTER=1 in the environment selects the scatter form of the accumulation for every mode (read at
+// every call, so that a test can compare both forms in one process).  A backward that reuses its forward's chunk
+// list may therefore run the other form on it: the scatter form takes chunks of any length, in rounds.
 bool tile_scatter_form() {
   const char* e = std::getenv("ATL_TILE_SCATTER");
   return e && e[0] == '1';
