@@ -159,7 +159,7 @@ def summarize(dirs, out, title, command, copy_mb, cal_dirs=(), pairs=0.0):
                 traffic[k] = (fetch + write) * 1024.0
         lines.append("")
     if pairs > 0:
-        rows = [(k, agg[k]) for k in sorted(agg) if k.startswith("k_fast_") and "SQ_INSTS_VALU" in agg[k]]
+        rows = [(k, agg[k]) for k in sorted(agg) if k.startswith(("k_fast_fwd", "k_entry_bwd")) and "SQ_INSTS_VALU" in agg[k]]
         if rows:
             lines += [f"VALU lane-slots per contributing pair (SQ_INSTS_VALU x 64 / K, K = {pairs:.4g} pairs per "
                       f"launch):", ""]
