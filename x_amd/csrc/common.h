@@ -47,6 +47,23 @@ __device__ __forceinline__ int wave_min_i(int v) {
   return v;
 }
 
+// A lane's value through a DPP row operation (gfx9: quad_perm, row mirrors, row_shr, row_bcast), no LDS permute.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dppf(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, false));
+}
+
+// Sum over the 64 lanes, returned wave-uniform.
+__device__ __forceinline__ float wave_sum_f(float v) {
+  v += dppf<0xB1, 0xF>(v);                       // quad_perm [1, 0, 3, 2]
+  v += dppf<0x4E, 0xF>(v);                       // quad_perm [2, 3, 0, 1]
+  v += dppf<0x141, 0xF>(v);                      // row_half_mirror
+  v += dppf<0x140, 0xF>(v);                      // row_mirror: every lane holds its row's sum
+  v += dppf<0x142, 0xA>(v);                      // row_bcast:15 into rows 1, 3
+  v += dppf<0x143, 0xC>(v);                      // row_bcast:31 into rows 2, 3: lane 63 holds the total
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
 // Lanes of a wave that are about to add to the same addresses (the same key) let one of them add their sums: global
 // atomics on one cache line serialise (18 ns an event of four corners where all events meet in one pixel).  Up to
 // kMergeRounds keys, each that of the first lane still open, are merged where at least kMergeMin lanes hold it; a key
@@ -66,7 +83,7 @@ __device__ __forceinline__ bool merge_lanes(bool live, int64_t key, float (&v)[N
     if (__popcll(same) < kMergeMin) continue;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const float s = wave_sum(in ? v[k] : 0.f);
+      const float s = wave_sum_f(in ? v[k] : 0.f);
       v[k] = in ? s : v[k];
     }
     adds = adds && (!in || lane == lead);

@@ -937,21 +937,6 @@ template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp(int v) {
   return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
 }
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dppf(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, false));
-}
-
-// Sum over the 64 lanes, returned wave-uniform.
-__device__ __forceinline__ float wave_sum_f(float v) {
-  v += dppf<0xB1, 0xF>(v);                       // quad_perm [1, 0, 3, 2]
-  v += dppf<0x4E, 0xF>(v);                       // quad_perm [2, 3, 0, 1]
-  v += dppf<0x141, 0xF>(v);                      // row_half_mirror
-  v += dppf<0x140, 0xF>(v);                      // row_mirror: every lane holds its row's sum
-  v += dppf<0x142, 0xA>(v);                      // row_bcast:15 into rows 1, 3
-  v += dppf<0x143, 0xC>(v);                      // row_bcast:31 into rows 2, 3: lane 63 holds the total
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
 
 __device__ __forceinline__ int wave_sum_i(int v) {
   v += dpp<0xB1, 0xF>(v);

@@ -675,7 +675,7 @@ __global__ void __launch_bounds__(kAccBlock) k_voxel_accum(const int4* __restric
         float c[8];
         corners(f, c);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) c[j] = wave_sum(vox[u] == v ? c[j] : 0.f);
+        for (int j = 0; j < 8; ++j) c[j] = wave_sum_f(vox[u] == v ? c[j] : 0.f);
         // other waves may hold the voxel too: atomics, ahead of the barrier before the plain additions below
         if ((tid & (kWave - 1)) == 0)
 #pragma unroll
