@@ -696,29 +696,32 @@ def mpcm_lut_main(a, dev):
     for _ in range(a.warmup):
         step()
     torch.cuda.synchronize()
-    rec = _ext.time_kernels(["atl_knn_indices"], every=1)
+    rec = _ext.time_kernels(["atl_lut_table_fwd", "atl_lut_table_bwd"], every=1)
     t0 = time.perf_counter()
     for _ in range(a.steps):
         step()
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
-    kms = float(np.mean([e0.elapsed_time(e1) for e0, e1, _ in rec["atl_knn_indices"]]))
+    ms = {k: float(np.mean([e0.elapsed_time(e1) for e0, e1, _ in rec[k]])) for k in rec}
+    kms = ms["atl_lut_table_fwd"]
     _ext.time_kernels(())
     P, Q, n, k = 15, 120 * 160, 120 * 160, 32
-    # algorithmic bytes of the KNN entry point: the points (8 B each) and queries (8 B) read, the indices written
-    nbytes = P * n * 8 + Q * 8 + P * Q * k * 8
+    # algorithmic bytes of the table's entry point: the positions at the bins and at the reference time read, the table
+    # written (8 B each)
+    nbytes = (P + 1) * n * 8 + P * Q * 8
     line = {
         "metric": "look-up-table queries/s for MotionPriorCMax's KNN table fwd+bwd (15 bins x 19200 cells, k=32, "
-                  "19200 trajectories); % HBM roofline of the KNN pass",
+                  "19200 trajectories); % HBM roofline of the table's forward",
         "value": P * Q * a.steps / dt, "unit": "queries/s", "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
         "ms_per_step": 1e3 * dt / a.steps, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f32", "data": "synthetic",
         "config": {"workload": "MotionPriorCMaxLoss.lut_flow, 640x480, lut 4, PixelTrajectories(K=10, bspline, tile 4), "
                                "15 bins, 32 neighbours, backward to the (1, 20, 480, 640) coefficients",
                    "parallelism": "single GPU"},
-        "roofline": {"bound": "hbm", "kernel": "atl_knn_indices", "achieved": nbytes / (kms * 1e-3) / 1e9,
+        "roofline": {"bound": "hbm", "kernel": "atl_lut_table_fwd", "achieved": nbytes / (kms * 1e-3) / 1e9,
                      "peak": 8000.0, "unit": "GB/s", "frac": nbytes / (kms * 1e-3) / 8e12, "traffic": None,
                      "kernel_ms": kms, "algorithmic_bytes": nbytes},
+        "kernel_ms": ms,
     }
     if not a.no_cpu:
         O = _oracle()
@@ -791,8 +794,10 @@ def main():
         step()
     torch.cuda.synchronize()
     # the pair kernels first (the roofline's candidates); the objective's dense flow takes the flow path, whose
-    # backward is the pair backward (atl_fast_pair_bwd_src) and then the flow-grid adjoint
+    # backward is the pair backward (atl_fast_pair_bwd_src) and then the flow-grid adjoint, the blobs' Sim2 motion the
+    # backward to the velocities
     kernels = (["atl_ats_pair_fwd_ws", "atl_ats_pair_bwd_ws_binned"] if reflayout else
+               ["atl_fast_pair_fwd", "atl_fast_pair_bwd"] if blobs else
                ["atl_fast_pair_fwd", "atl_fast_pair_bwd_src", "atl_fast_flow_adjoint"]) + (
         ["atl_splat_bilinear_fwd_ws", "atl_splat_bilinear_bwd"] if blobs else [])
     rec = _ext.time_kernels(kernels, every=4)      # every bracket delays the next launch: sample the steps
