@@ -1,7 +1,7 @@
 // ORACLE — test infrastructure only.
 //
-// A CPU (OpenMP) restatement of the reference's event-transport loops, used as the checker for the HIP
-// library and as the timed CPU baseline.  Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline
+// A CPU (OpenMP) restatement of the reference's event-transport loops, used to check the HIP
+// library's results and as the timed CPU baseline.  Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline
 // leg may load this library; the product path (x_amd) never does.
 //
 // Each function follows csrc/atl_cpu.cpp of the reference (file:line cited per function): same loop order,
